@@ -19,25 +19,37 @@
 
 #include "device_common.hpp"
 #include "internal.hpp"
+#include "traverse.hpp"
 
 namespace asc {
+
+// An iteration's count of vertices that moved, as the device publishes it to
+// mapped host memory; seq is written last.
+struct PrRefPub {
+    unsigned long long moved;
+    unsigned long long seq;
+};
 
 struct PrState {
     uint64_t V = 0;
     float* rank[2] = {nullptr, nullptr};
     float* contrib[2] = {nullptr, nullptr};
-    double* acc = nullptr;        // [0, MAXIT): residual; [MAXIT, 2*MAXIT+1): dangling
-    uint32_t* heavy = nullptr;    // vertices with in-degree >= heavy threshold
-    uint32_t n_heavy = 0;
-    int heavy_thr = 0;
-    int acc_iters = 0;
+    double* acc = nullptr;        // ring of kAccSlots slots of kAccSlot sums (PrArgs::acc_in / acc_out)
+    double* resid = nullptr;      // residual of each iteration
+    int resid_iters = 0;
     // reference mode
     double* val64 = nullptr;
-    double* sum64 = nullptr;
-    double* contrib64 = nullptr;
+    double* contrib64[2] = {nullptr, nullptr};   // read by / written for the next iteration
     uint8_t* active = nullptr;
-    uint32_t* count = nullptr;
-    HostBuf<uint32_t> h_count;
+    uint32_t* count = nullptr;    // kPrLines counters, one per 128-byte line
+    HostBuf<PrRefPub> h_refpub;   // ring written by the device through d_refpub (mapped)
+    PrRefPub* d_refpub = nullptr;
+    unsigned long long ref_seq = 0;
+    // row blocks and heavy rows of the resident vertices (RowPlan)
+    void* rows_blocks = nullptr;
+    uint32_t* rows_heavy = nullptr;
+    uint32_t rows_n = 0, rows_cap = 0, rows_front = 0, rows_back = 0;
+    bool rows_built = false;
     // on-demand in-edges: vertex-range chunks [v0, v1) whose in-edges
     // [off[v0], off[v1]) fit one part buffer, copied from the pinned tail
     struct Chunk {
@@ -80,7 +92,8 @@ void pr_free(PrState* p) {
         if (x) (void)hipFree(x);
     };
     f(p->rank[0]); f(p->rank[1]); f(p->contrib[0]); f(p->contrib[1]);
-    f(p->acc); f(p->heavy); f(p->val64); f(p->sum64); f(p->contrib64); f(p->active); f(p->count);
+    f(p->acc); f(p->resid); f(p->val64); f(p->contrib64[0]); f(p->contrib64[1]); f(p->active);
+    f(p->count); f(p->rows_heavy); f(p->rows_blocks);
     f(p->part[0]); f(p->part[1]);
     f(p->pb_src); f(p->pb_pos); f(p->pb_dl); f(p->pb_vals); f(p->pb_bin_start); f(p->pb_cnt);
     f(p->tl_edges); f(p->tl_off); f(p->tl_heavy);
@@ -141,10 +154,270 @@ static int pr_stream_chunks(asc_graph* g, PrState* p, F&& pull) {
     return ASC_OK;
 }
 
+// ---- row sums ---------------------------------------------------------------
+// Resident rows (in-lists) are summed in row blocks: at most 256 consecutive
+// vertices whose lists start within one window of kRowsWindow edges and hold
+// fewer than kRowsHeavy edges each (a longer row ends a block), so a block is
+// one contiguous stretch of at most kRowsTile edges whatever the degrees (cut
+// once per graph, below).  A workgroup reads the stretch's ids, gathers their
+// contributions into LDS, and each vertex's lane adds its own part in CSR
+// order.  Longer rows are left to a wave or a workgroup each.
+constexpr int kRowsPer = 8;
+constexpr int kRowsTile = kBlock * kRowsPer;
+constexpr uint32_t kRowsWindow = 1536;
+constexpr uint32_t kRowsHeavy = 512;
+static_assert(kRowsWindow + kRowsHeavy <= kRowsTile, "a row block is one tile");
+constexpr uint32_t kRowsLong = 4096;    // rows summed by a whole workgroup, started before all others
+constexpr int kSeqPer = 4;              // a heavy row's pass of the reference mode
+constexpr int kSeqTile = kBlock * kSeqPer;
+static_assert(2 * kSeqTile <= kRowsTile, "two passes share the row tile's LDS");
+constexpr int kPrLines = 16;            // counters spread over this many 128-byte lines
+constexpr int kPrLineWords = 32;
+
+// s + x[0] + x[1] + ... in that order, B values read ahead of their adds.
+template <uint32_t B, class T>
+__device__ __forceinline__ double add_in_order(double s, const T* x, uint32_t n) {
+    uint32_t k = 0;
+    for (; k + B <= n; k += B) {
+        T y[B];
+#pragma unroll
+        for (uint32_t j = 0; j < B; j++) y[j] = x[k + j];
+#pragma unroll
+        for (uint32_t j = 0; j < B; j++) s += (double)y[j];
+    }
+    for (; k < n; k++) s += (double)x[k];
+    return s;
+}
+
+// The same for a long stretch: 16 values are read while the 16 before them
+// are added (two register sets, so nothing is copied, and a scheduling fence
+// so that the reads are not moved behind the adds), and the chain waits for
+// its adds alone.
+__device__ __forceinline__ double add_chain(double s, const double* x, uint32_t n) {
+    constexpr uint32_t B = 16;
+    uint32_t k = 0;
+    if (n >= 3 * B) {
+        double y[B], z[B];
+#pragma unroll
+        for (uint32_t j = 0; j < B; j++) y[j] = x[j];
+        for (; k + 3 * B <= n; k += 2 * B) {
+#pragma unroll
+            for (uint32_t j = 0; j < B; j++) z[j] = x[k + B + j];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (uint32_t j = 0; j < B; j++) s += y[j];
+#pragma unroll
+            for (uint32_t j = 0; j < B; j++) y[j] = x[k + 2 * B + j];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (uint32_t j = 0; j < B; j++) s += z[j];
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < B; j++) s += y[j];
+        k += B;
+    }
+    return add_in_order<8>(s, x + k, n - k);
+}
+
+// Sums the rows of at most 256 vertices [base, end) of any length (streamed
+// chunks, whose rows have no plan): their concatenated edges a tile at a time,
+// the owner of an edge found by a binary search of the degree prefix in LDS.
+// take(v): whether v is summed; fin(v, sum) is called for those.
+template <class OffT, class T, class Take, class Fin>
+__device__ __forceinline__ void pull_rows(const OffT* off, const uint32_t* src, const T* contrib, uint64_t base,
+                                          uint64_t end, T* s_val, Take take, Fin fin) {
+    using PT = unsigned long long;
+    __shared__ PT s_pref[kBlock];
+    __shared__ OffT s_beg[kBlock];
+    __shared__ PT s_tmp[kWavesPerBlock];
+    const uint32_t tid = threadIdx.x;
+    const uint64_t v = base + tid;
+    const bool mine = v < end && take(v);
+    OffT b = 0;
+    PT deg = 0;
+    if (mine) {
+        b = off[v];
+        deg = (PT)(off[v + 1] - b);
+    }
+    PT total;
+    const PT pre = block_scan_excl(deg, s_tmp, total);
+    s_pref[tid] = pre;
+    s_beg[tid] = b;
+    __syncthreads();
+    double s = 0;
+    for (PT t0 = 0; t0 < total; t0 += kRowsTile) {
+        uint32_t u[kRowsPer];
+        T c[kRowsPer];
+#pragma unroll
+        for (int j = 0; j < kRowsPer; j++) {
+            const PT e = min((PT)(t0 + j * kBlock + tid), (PT)(total - 1));
+            uint32_t k = 0;
+#pragma unroll
+            for (uint32_t step = kBlock / 2; step > 0; step >>= 1)
+                if (s_pref[k + step] <= e) k += step;
+            u[j] = src[s_beg[k] + (OffT)(e - s_pref[k])];
+        }
+#pragma unroll
+        for (int j = 0; j < kRowsPer; j++) c[j] = contrib[u[j]];
+        if (t0) __syncthreads();   // the previous tile's adds are done
+#pragma unroll
+        for (int j = 0; j < kRowsPer; j++) s_val[j * kBlock + tid] = c[j];
+        __syncthreads();
+        const PT t1 = total - t0 > kRowsTile ? (PT)(t0 + kRowsTile) : total;
+        const PT lo = max(pre, t0), hi = min((PT)(pre + deg), t1);
+        if (lo < hi) s = add_in_order<8>(s, s_val + (uint32_t)(lo - t0), (uint32_t)(hi - lo));
+    }
+    if (mine) fin(v, s);
+    __syncthreads();
+}
+
+// Row blocks of the vertices [0, n), written in any order.
+struct RowBlock {
+    unsigned long long e;           // first edge
+    uint32_t v, n, edges;           // vertices [v, v + n), their edges
+    uint32_t pad;
+};
+
+template <class OffT>
+__global__ __launch_bounds__(kBlock) void k_row_blocks(const OffT* off, uint64_t n, RowBlock* blocks, uint32_t* cnt) {
+    __shared__ uint64_t s_break[kWavesPerBlock];
+    const uint32_t lane = lane_id(), w = wave_id();
+    for (uint64_t base = (uint64_t)blockIdx.x * kBlock; base < n; base += (uint64_t)gridDim.x * kBlock) {
+        const uint64_t v = base + threadIdx.x;
+        uint64_t b = 0, d = 0;
+        bool heavy = false, starts = false;
+        if (v < n) {
+            b = (uint64_t)off[v];
+            d = (uint64_t)off[v + 1] - b;
+            heavy = d >= kRowsHeavy;
+            // a new block at every multiple of 256, in every window and after a heavy row
+            starts = !heavy && (threadIdx.x == 0 || (uint64_t)off[v - 1] / kRowsWindow != b / kRowsWindow ||
+                                b - (uint64_t)off[v - 1] >= kRowsHeavy);
+        }
+        const uint64_t brk = wave_ballot(starts || heavy || v >= n);
+        if (lane == 0) s_break[w] = brk;
+        __syncthreads();
+        const uint64_t m = wave_ballot(starts);
+        uint32_t at = 0;
+        if (lane == 0 && m) at = atomicAdd(cnt, (uint32_t)__popcll(m));
+        at = __shfl(at, 0, kWave);
+        if (starts) {
+            // the next break after this lane ends the block
+            uint32_t end = kBlock;
+            uint64_t rest = lane == kWave - 1 ? 0 : brk & (~0ull << (lane + 1));
+            for (uint32_t i = w; i < (uint32_t)kWavesPerBlock; i++) {
+                if (i > w) rest = s_break[i];
+                if (rest) {
+                    end = i * kWave + (uint32_t)__builtin_ctzll(rest);
+                    break;
+                }
+            }
+            const uint32_t cntv = end - threadIdx.x;
+            blocks[at + lanes_below(m)] =
+                RowBlock{b, (uint32_t)v, cntv, (uint32_t)((uint64_t)off[v + cntv] - b), 0u};
+        }
+        __syncthreads();
+    }
+}
+
+// Sums the rows of a row block.  s_val: kRowsTile values of LDS.  pre(v) reads
+// what fin(v, sum, pre(v)) needs of a vertex, ahead of the gathers.
+template <class OffT, class T, class Pre, class Fin>
+__device__ __forceinline__ void pull_block(const OffT* off, const uint32_t* src, const T* contrib, const RowBlock& rb,
+                                           T* s_val, Pre pre, Fin fin) {
+    const uint32_t tid = threadIdx.x;
+    const uint32_t* ids = src + rb.e;
+    uint32_t u[kRowsPer];
+#pragma unroll
+    for (int j = 0; j < kRowsPer; j++) u[j] = rb.edges ? ids[min(j * (uint32_t)kBlock + tid, rb.edges - 1)] : 0u;
+    const bool mine = tid < rb.n;
+    const uint32_t v = rb.v + (mine ? tid : 0);
+    const uint32_t lo = (uint32_t)((uint64_t)off[v] - rb.e), hi = (uint32_t)((uint64_t)off[v + 1] - rb.e);
+    const auto own = pre(v);
+    T c[kRowsPer];
+#pragma unroll
+    for (int j = 0; j < kRowsPer; j++) c[j] = contrib[u[j]];
+#pragma unroll
+    for (int j = 0; j < kRowsPer; j++) s_val[j * kBlock + tid] = c[j];
+    __syncthreads();
+    if (mine) fin(v, add_in_order<8>(0.0, s_val + lo, hi - lo), own);
+    __syncthreads();   // s_val is free again
+}
+
+// Rows of kRowsHeavy edges and more among the vertices [0, n): those of
+// kRowsLong edges from the front of `list`, the others from its back.
+template <class OffT>
+__global__ __launch_bounds__(kBlock) void k_rows_heavy_list(const OffT* off, uint64_t n, uint32_t* list, uint32_t cap,
+                                                            uint32_t* cnt) {
+    for (uint64_t base = (uint64_t)blockIdx.x * kBlock; base < n; base += (uint64_t)gridDim.x * kBlock) {
+        const uint64_t v = base + threadIdx.x;
+        const uint64_t d = v < n ? (uint64_t)(off[v + 1] - off[v]) : 0;
+        const bool front = d >= kRowsLong, back = d >= kRowsHeavy && !front;
+        const uint64_t mf = wave_ballot(front), mb = wave_ballot(back);
+        uint32_t at = 0;
+        if (lane_id() == 0 && mf) at = atomicAdd(cnt, (uint32_t)__popcll(mf));
+        at = __shfl(at, 0, kWave);
+        if (front) list[at + lanes_below(mf)] = (uint32_t)v;
+        if (lane_id() == 0 && mb) at = atomicAdd(cnt + 1, (uint32_t)__popcll(mb));
+        at = __shfl(at, 0, kWave);
+        if (back) list[cap - 1 - (at + lanes_below(mb))] = (uint32_t)v;
+    }
+}
+
+// The row plan of a graph's resident vertices.
+struct RowPlan {
+    const RowBlock* blocks;
+    const uint32_t* heavy;        // rows >= kRowsLong from the front, >= kRowsHeavy from the back
+    uint32_t n_blocks, cap, n_front, n_back;
+    __device__ __forceinline__ uint32_t front(uint32_t i) const { return heavy[i]; }
+    __device__ __forceinline__ uint32_t back(uint32_t i) const { return heavy[cap - 1 - i]; }
+};
+
 // ---- normalised mode --------------------------------------------------------
 
-__global__ void k_pr_init(float* rank, float* contrib, const uint32_t* outdeg, uint64_t V, double* dang0) {
-    __shared__ double s_red[kWavesPerBlock];
+// The residual and dangling sums of an iteration: every workgroup adds its
+// share to one of kPrLines cache lines of a slot (same-address atomics of a
+// whole grid take ~9 ns each, 18 us for 2048 workgroups), and the readers add
+// the lines up.  Slot it & 3 holds the dangling mass of the ranks iteration
+// `it` reads and the residual of iteration it - 1; iteration `it` clears slot
+// (it + 2) & 3.
+constexpr int kAccLine = 16;                            // doubles per 128-byte line
+constexpr int kAccDang = kPrLines * kAccLine;           // the dangling lines follow the residual lines
+constexpr int kAccSlot = 2 * kAccDang;
+constexpr int kAccSlots = 4;
+
+// Sum of a slot's lines (the residual's at `p`, the dangling mass's at
+// p + kAccDang), in every lane of the calling wave.
+__device__ __forceinline__ double acc_lines(const double* p) {
+    const uint32_t l = lane_id();
+    return wave_sum(l < (uint32_t)kPrLines ? p[l * kAccLine] : 0.0);
+}
+
+// Workgroup sums of res and dang, added to this workgroup's lines of `acc`.
+template <int THREADS>
+__device__ __forceinline__ void acc_add(double res, double dang, double* acc) {
+    __shared__ double s_r[THREADS / kWave], s_d[THREADS / kWave];
+    res = wave_sum(res);
+    dang = wave_sum(dang);
+    if (lane_id() == 0) {
+        s_r[wave_id()] = res;
+        s_d[wave_id()] = dang;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double r = 0, d = 0;
+        for (int i = 0; i < THREADS / kWave; i++) {
+            r += s_r[i];
+            d += s_d[i];
+        }
+        double* line = acc + (blockIdx.x % kPrLines) * kAccLine;
+        if (r != 0) atomicAdd(line, r);
+        if (d != 0) atomicAdd(line + kAccDang, d);
+    }
+}
+
+__global__ __launch_bounds__(kBlock) void k_pr_init(float* rank, float* contrib, const uint32_t* outdeg, uint64_t V,
+                                                    double* acc) {
     const float r0 = (float)(1.0 / (double)V);
     double dang = 0;
     for (uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v < V; v += (uint64_t)gridDim.x * blockDim.x) {
@@ -153,14 +426,13 @@ __global__ void k_pr_init(float* rank, float* contrib, const uint32_t* outdeg, u
         contrib[v] = d ? r0 / (float)d : 0.0f;
         if (!d) dang += (double)r0;
     }
-    dang = wave_sum(dang);
-    if (lane_id() == 0) s_red[wave_id()] = dang;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double t = 0;
-        for (int i = 0; i < kWavesPerBlock; i++) t += s_red[i];
-        if (t != 0) atomicAdd(dang0, t);
-    }
+    acc_add<kBlock>(0.0, dang, acc);
+}
+
+// The last iteration's residual (one wave).
+__global__ void k_pr_last_residual(const double* slot, double* resid) {
+    const double r = acc_lines(slot);
+    if (threadIdx.x == 0) *resid = r;
 }
 
 struct PrArgs {
@@ -174,50 +446,149 @@ struct PrArgs {
     const float* contrib_in;
     float* rank_out;
     float* contrib_out;
-    const double* dang_in;        // dangling mass of rank_in
-    double* dang_out;             // dangling mass of rank_out
-    double* residual;
+    const double* acc_in;         // slot with the dangling mass of rank_in
+    double* acc_out;              // slot of this iteration's residual and rank_out's dangling mass
+    double* acc_clear;            // slot to clear (the iteration's first launch; else null)
+    double* resid_prev;           // where that launch stores the previous iteration's residual (or null)
     uint64_t V;
     float damping;
     double damping64;
     uint32_t heavy_thr;
 };
 
+// What a vertex's new rank is finished with.
+struct PrOwn {
+    uint32_t outdeg;
+    float rank;
+};
+
+__device__ __forceinline__ PrOwn pr_own(const PrArgs& a, uint64_t v) { return PrOwn{a.outdeg[v], a.rank_in[v]}; }
+
+__device__ __forceinline__ void pr_finish_vertex(const PrArgs& a, uint64_t v, double s, const PrOwn& own, double base,
+                                                 double& res, double& dang) {
+    const float nr = (float)(base + a.damping64 * s);
+    res += fabs((double)nr - (double)own.rank);
+    a.rank_out[v] = nr;
+    a.contrib_out[v] = own.outdeg ? nr / (float)own.outdeg : 0.0f;
+    if (!own.outdeg) dang += (double)nr;
+}
+
 __device__ __forceinline__ void pr_finish_vertex(const PrArgs& a, uint64_t v, double s, double base, double& res,
                                                  double& dang) {
-    const float nr = (float)(base + a.damping64 * s);
-    const uint32_t d = a.outdeg[v];
-    res += fabs((double)nr - (double)a.rank_in[v]);
-    a.rank_out[v] = nr;
-    a.contrib_out[v] = d ? nr / (float)d : 0.0f;
-    if (!d) dang += (double)nr;
+    pr_finish_vertex(a, v, s, pr_own(a, v), base, res, dang);
 }
 
-__device__ __forceinline__ void pr_block_reduce2(double res, double dang, double* out_res, double* out_dang) {
-    __shared__ double s_r[kWavesPerBlock], s_d[kWavesPerBlock];
-    res = wave_sum(res);
-    dang = wave_sum(dang);
-    if (lane_id() == 0) {
-        s_r[wave_id()] = res;
-        s_d[wave_id()] = dang;
+// Rank of a vertex whose in-sum is zero, in every lane; called by the whole
+// workgroup.  Workgroup 0 of an iteration's first launch also stores the
+// previous residual and clears the slot of the iteration after the next.
+__device__ __forceinline__ double pr_base(const PrArgs& a) {
+    __shared__ double s_base;
+    if (threadIdx.x < kWave) {
+        const double dang = acc_lines(a.acc_in + kAccDang);
+        if (threadIdx.x == 0) s_base = (1.0 - a.damping64) / (double)a.V + a.damping64 * dang / (double)a.V;
+        if (blockIdx.x == 0 && a.resid_prev) {
+            const double r = acc_lines(a.acc_in);
+            if (threadIdx.x == 0) *a.resid_prev = r;
+        }
+        if (blockIdx.x == 0 && a.acc_clear)
+            for (int i = threadIdx.x; i < kAccSlot; i += kWave) a.acc_clear[i] = 0;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        double r = 0, d = 0;
-        for (int i = 0; i < kWavesPerBlock; i++) {
-            r += s_r[i];
-            d += s_d[i];
-        }
-        if (r != 0) atomicAdd(out_res, r);
-        if (d != 0) atomicAdd(out_dang, d);
-    }
+    return s_base;
 }
 
-// G lanes per vertex; vertices with in-degree >= heavy_thr are skipped here.
+// Sum of one long row by the whole workgroup (the result in thread 0): 8
+// gathers in flight per lane.  s_sum: one double per wave.
+template <class OffT>
+__device__ __forceinline__ double pull_long_row(const uint32_t* src, const float* contrib, OffT b, OffT e,
+                                                double* s_sum) {
+    constexpr int U = 8;
+    double s = 0;
+    for (OffT k = b + threadIdx.x; k < e; k += (OffT)U * kBlock) {
+        uint32_t u[U];
+        float c[U];
+#pragma unroll
+        for (int j = 0; j < U; j++) u[j] = src[min((OffT)(k + j * kBlock), (OffT)(e - 1))];
+#pragma unroll
+        for (int j = 0; j < U; j++) c[j] = contrib[u[j]];
+#pragma unroll
+        for (int j = 0; j < U; j++)
+            if (k + (OffT)(j * kBlock) < e) s += (double)c[j];
+    }
+    s = wave_sum(s);
+    if (lane_id() == 0) s_sum[wave_id()] = s;
+    __syncthreads();
+    double t = 0;
+    if (threadIdx.x == 0)
+        for (int j = 0; j < kWavesPerBlock; j++) t += s_sum[j];
+    __syncthreads();
+    return t;
+}
+
+// The same by one wave (the result in every lane).
+template <class OffT>
+__device__ __forceinline__ double pull_wave_row(const uint32_t* src, const float* contrib, OffT b, OffT e) {
+    constexpr int U = 8;
+    double s = 0;
+    for (OffT k = b + lane_id(); k < e; k += (OffT)U * kWave) {
+        uint32_t u[U];
+        float c[U];
+#pragma unroll
+        for (int j = 0; j < U; j++) u[j] = src[min((OffT)(k + j * kWave), (OffT)(e - 1))];
+#pragma unroll
+        for (int j = 0; j < U; j++) c[j] = contrib[u[j]];
+#pragma unroll
+        for (int j = 0; j < U; j++)
+            if (k + (OffT)(j * kWave) < e) s += (double)c[j];
+    }
+    return wave_sum(s);
+}
+
+// The pull of an iteration: over the resident rows (HEAVY: the first `hb`
+// workgroups take the rows above kRowsHeavy, longest first, the others the
+// row blocks), or over the vertices [v_begin, v_end) of a streamed chunk.
+template <class OffT, bool HEAVY>
+__global__ __launch_bounds__(kBlock) void k_pr_rows(PrArgs a, RowPlan rows, uint32_t hb) {
+    __shared__ float s_val[kRowsTile];
+    __shared__ double s_sum[kWavesPerBlock];
+    const OffT* off = (const OffT*)a.off;
+    const uint32_t* src = a.src - a.e_base;
+    const double base = pr_base(a);
+    double res = 0, dang = 0;
+    if (HEAVY && blockIdx.x < hb) {
+        for (uint32_t i = blockIdx.x; i < rows.n_front; i += hb) {
+            const uint32_t v = rows.front(i);
+            const double s = pull_long_row<OffT>(src, a.contrib_in, off[v], off[v + 1], s_sum);
+            if (threadIdx.x == 0) pr_finish_vertex(a, v, s, base, res, dang);
+        }
+        for (uint32_t i = blockIdx.x * kWavesPerBlock + wave_id(); i < rows.n_back; i += hb * kWavesPerBlock) {
+            const uint32_t v = rows.back(i);
+            const double s = pull_wave_row<OffT>(src, a.contrib_in, off[v], off[v + 1]);
+            if (lane_id() == 0) pr_finish_vertex(a, v, s, base, res, dang);
+        }
+    } else {
+        const uint32_t bid = blockIdx.x - (HEAVY ? hb : 0), nblk = gridDim.x - (HEAVY ? hb : 0);
+        if (HEAVY) {
+            auto pre = [&](uint64_t v) { return pr_own(a, v); };
+            auto fin = [&](uint64_t v, double s, const PrOwn& own) { pr_finish_vertex(a, v, s, own, base, res, dang); };
+            for (uint32_t i = bid; i < rows.n_blocks; i += nblk)
+                pull_block(off, src, a.contrib_in, rows.blocks[i], s_val, pre, fin);
+        } else {
+            auto take = [](uint64_t) { return true; };
+            auto fin = [&](uint64_t v, double s) { pr_finish_vertex(a, v, s, base, res, dang); };
+            for (uint64_t v = a.v_begin + (uint64_t)bid * kBlock; v < a.v_end; v += (uint64_t)nblk * kBlock)
+                pull_rows(off, src, a.contrib_in, v, a.v_end, s_val, take, fin);
+        }
+    }
+    acc_add<kBlock>(res, dang, a.acc_out);
+}
+
+// G lanes per vertex (asc_config.pr_group or a tuned graph); vertices with
+// in-degree >= heavy_thr are skipped here.
 template <int G, class OffT>
 __global__ __launch_bounds__(kBlock) void k_pr_pull(PrArgs a) {
     const OffT* off = (const OffT*)a.off;
-    const double base = (1.0 - a.damping64) / (double)a.V + a.damping64 * (*a.dang_in) / (double)a.V;
+    const double base = pr_base(a);
     const uint32_t sub = threadIdx.x % G;
     const uint64_t groups_per_grid = (uint64_t)gridDim.x * (blockDim.x / G);
     const uint32_t* src = a.src - a.e_base;
@@ -247,34 +618,21 @@ __global__ __launch_bounds__(kBlock) void k_pr_pull(PrArgs a) {
         for (int d = G / 2; d > 0; d >>= 1) s += __shfl_xor(s, d, G);
         if (sub == 0 && !heavy) pr_finish_vertex(a, v, s, base, res, dang);
     }
-    pr_block_reduce2(res, dang, a.residual, a.dang_out);
+    acc_add<kBlock>(res, dang, a.acc_out);
 }
 
 template <class OffT>
 __global__ __launch_bounds__(kBlock) void k_pr_pull_heavy(PrArgs a, const uint32_t* heavy, uint32_t n_heavy) {
     __shared__ double s_sum[kWavesPerBlock];
     const OffT* off = (const OffT*)a.off;
-    const double base = (1.0 - a.damping64) / (double)a.V + a.damping64 * (*a.dang_in) / (double)a.V;
+    const double base = pr_base(a);
     double res = 0, dang = 0;
     for (uint32_t i = blockIdx.x; i < n_heavy; i += gridDim.x) {
         const uint32_t v = heavy[i];
-        const OffT b = off[v], e = off[v + 1];
-        double s = 0;
-        for (OffT k = b + threadIdx.x; k < e; k += blockDim.x) s += (double)a.contrib_in[a.src[k]];
-        s = wave_sum(s);
-        if (lane_id() == 0) s_sum[wave_id()] = s;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            double t = 0;
-            for (int j = 0; j < kWavesPerBlock; j++) t += s_sum[j];
-            pr_finish_vertex(a, v, t, base, res, dang);
-        }
-        __syncthreads();
+        const double s = pull_long_row<OffT>(a.src, a.contrib_in, off[v], off[v + 1], s_sum);
+        if (threadIdx.x == 0) pr_finish_vertex(a, v, s, base, res, dang);
     }
-    if (threadIdx.x == 0) {
-        if (res != 0) atomicAdd(a.residual, res);
-        if (dang != 0) atomicAdd(a.dang_out, dang);
-    }
+    acc_add<kBlock>(res, dang, a.acc_out);
 }
 
 // ---- propagation-blocked normalised mode -----------------------------------
@@ -384,7 +742,6 @@ template <class OffT>
 __global__ __launch_bounds__(kPbBlock) void k_pb_gather(PrArgs a, const unsigned long long* reg_base,
                                                         const uint32_t* cnt, const uint16_t* dl, const float* vals) {
     __shared__ float acc[kPbBin];
-    __shared__ double s_r[kPbBlock / kWave], s_d[kPbBlock / kWave];
     const OffT* off = (const OffT*)a.off;
     const uint32_t b = blockIdx.x;
     for (uint32_t i = threadIdx.x; i < kPbBin; i += kPbBlock) acc[i] = 0.0f;
@@ -395,29 +752,14 @@ __global__ __launch_bounds__(kPbBlock) void k_pb_gather(PrArgs a, const unsigned
         for (uint32_t k = lane_id(); k < n; k += kWave) atomicAdd(&acc[dl[k0 + k]], vals[k0 + k]);
     }
     __syncthreads();
-    const double base = (1.0 - a.damping64) / (double)a.V + a.damping64 * (*a.dang_in) / (double)a.V;
+    const double base = pr_base(a);
     double res = 0, dang = 0;
     for (uint32_t i = threadIdx.x; i < kPbBin; i += kPbBlock) {
         const uint64_t v = (uint64_t)b * kPbBin + i;
         if (v >= a.V || (uint64_t)(off[v + 1] - off[v]) >= a.heavy_thr) continue;
         pr_finish_vertex(a, v, (double)acc[i], base, res, dang);
     }
-    res = wave_sum(res);
-    dang = wave_sum(dang);
-    if (lane_id() == 0) {
-        s_r[threadIdx.x / kWave] = res;
-        s_d[threadIdx.x / kWave] = dang;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double r = 0, d = 0;
-        for (int i = 0; i < kPbBlock / kWave; i++) {
-            r += s_r[i];
-            d += s_d[i];
-        }
-        if (r != 0) atomicAdd(a.residual, r);
-        if (d != 0) atomicAdd(a.dang_out, d);
-    }
+    acc_add<kPbBlock>(res, dang, a.acc_out);
 }
 
 // ---- source-segmented normalised mode --------------------------------------
@@ -508,11 +850,10 @@ __global__ __launch_bounds__(kTlBlock) void k_pr_tiled(PrArgs a, const uint32_t*
                                                        const unsigned long long* __restrict__ toff, TileShape ts,
                                                        const uint32_t* heavy_bits) {
     __shared__ float acc[1u << DB];
-    __shared__ double s_r[kTlBlock / kWave], s_d[kTlBlock / kWave];
     const uint32_t G = gridDim.x;
     const uint32_t nb = blockIdx.x < ts.nd ? (ts.nd - blockIdx.x + G - 1) / G : 0;   // blocks of this workgroup
     const uint32_t dsz = 1u << ts.db, smask = (1u << ts.sb) - 1;
-    const double base = (1.0 - a.damping64) / (double)a.V + a.damping64 * (*a.dang_in) / (double)a.V;
+    const double base = pr_base(a);
     double res = 0, dang = 0;
     for (uint32_t r = 0; r < nb; r++) {
         const uint64_t d = blockIdx.x + (uint64_t)r * G;
@@ -571,75 +912,194 @@ __global__ __launch_bounds__(kTlBlock) void k_pr_tiled(PrArgs a, const uint32_t*
         }
         __syncthreads();
     }
-    res = wave_sum(res);
-    dang = wave_sum(dang);
-    if (lane_id() == 0) {
-        s_r[threadIdx.x / kWave] = res;
-        s_d[threadIdx.x / kWave] = dang;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double rr = 0, dd = 0;
-        for (int i = 0; i < kTlBlock / kWave; i++) {
-            rr += s_r[i];
-            dd += s_d[i];
-        }
-        if (rr != 0) atomicAdd(a.residual, rr);
-        if (dd != 0) atomicAdd(a.dang_out, dd);
-    }
+    acc_add<kTlBlock>(res, dang, a.acc_out);
 }
 
 // ---- reference mode --------------------------------------------------------
 
-__global__ void k_prref_init(double* val, uint8_t* active, uint64_t V) {
+__global__ void k_prref_init(double* val, double* contrib, uint8_t* active, const uint32_t* outdeg, uint64_t V) {
     for (uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v < V; v += (uint64_t)gridDim.x * blockDim.x) {
-        val[v] = 1.0 / (double)V;  // GraphMeta.cuh:418
+        const double r0 = 1.0 / (double)V;  // GraphMeta.cuh:418
+        val[v] = r0;
+        contrib[v] = outdeg[v] ? r0 / (double)outdeg[v] : 0.0;
         active[v] = 1;
     }
 }
 
-__global__ void k_prref_contrib(const double* val, const uint32_t* outdeg, double* contrib, uint64_t V) {
-    for (uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v < V; v += (uint64_t)gridDim.x * blockDim.x)
-        contrib[v] = outdeg[v] ? val[v] / (double)outdeg[v] : 0.0;
-}
+struct PrRefArgs {
+    const void* off;              // OffT[V+1]
+    const uint32_t* src;          // in-edges: edge k at src[k - e_base]
+    unsigned long long e_base;
+    unsigned long long v_begin, v_end;
+    const double* contrib_in;
+    double* contrib_out;
+    double* val;
+    uint8_t* active;
+    const uint32_t* outdeg;
+    uint32_t* count;              // vertices moved (kPrLines counters)
+    double base, damping, threshold;
+    RowPlan rows;                 // resident rows
+};
 
-// prSumKernel_static / _dynamic (gpu_kernels.cuh:554-594): sequential FP64
-// sum in CSR order for each active vertex.
-template <class OffT>
-__global__ void k_prref_sum(const OffT* off, const uint32_t* src, unsigned long long e_base, const double* contrib,
-                            const uint8_t* active, double* sum, uint64_t v_begin, uint64_t v_end) {
-    src -= e_base;
-    for (uint64_t v = v_begin + blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v < v_end;
-         v += (uint64_t)gridDim.x * blockDim.x) {
-        if (!active[v]) continue;
-        double s = 0;
-        for (OffT k = off[v]; k < off[v + 1]; k++) s += contrib[src[k]];
-        sum[v] = s;
-    }
-}
-
-// prKernel_Opt (gpu_kernels.cuh:533-552).
-__global__ void k_prref_update(double* val, double* sum, uint8_t* active, uint64_t V, double base, double damping,
-                               double threshold, uint32_t* count) {
+// prKernel_Opt (gpu_kernels.cuh:533-552) for active vertex v with in-sum s; a
+// vertex that stops keeps its value.  Its contribution is written for the
+// next iteration either way, so both buffers hold it from then on.
+__device__ __forceinline__ uint32_t prref_finish(const PrRefArgs& a, uint64_t v, double s) {
 #pragma clang fp contract(off)
-    uint32_t c = 0;
-    for (uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v < V; v += (uint64_t)gridDim.x * blockDim.x) {
-        if (!active[v]) continue;
-        const double t = base + damping * sum[v];
-        const double diff = t > val[v] ? (t - val[v]) : (val[v] - t);
-        if (diff > threshold) {
-            val[v] = t;
-            c++;
-        } else {
-            active[v] = 0;
-        }
-        sum[v] = 0;
+    const double t = a.base + a.damping * s;
+    const double old = a.val[v];
+    const double diff = t > old ? (t - old) : (old - t);
+    const uint32_t d = a.outdeg[v];
+    if (diff > a.threshold) {
+        a.val[v] = t;
+        a.contrib_out[v] = d ? t / (double)d : 0.0;
+        return 1;
     }
-    c = wave_sum(c);
-    if (lane_id() == 0 && c) atomicAdd(count, c);
+    a.active[v] = 0;
+    a.contrib_out[v] = a.contrib_in[v];
+    return 0;
+}
+
+// One iteration over [v_begin, v_end): prSumKernel_static / _dynamic
+// (gpu_kernels.cuh:554-594) and prKernel_Opt.  The result must equal a
+// sequential FP64 sum in CSR order, so a row is one chain of adds and the
+// longest row bounds an iteration; everything else is kept off that chain.
+// The first `hb` workgroups take the heavy rows, the longest first: 2048
+// contributions a pass are gathered by all lanes, then added by one lane out
+// of LDS while the next pass's gathers are in flight.  The other workgroups
+// run pull_block.  R-MAT scale 20 (31 M in-edges, longest row 64.8 k): 24.4 ms
+// an iteration with one thread per row loading and adding edge by edge, 0.43
+// ms this way, all of it the longest row's chain (6.6 ns an add).
+template <class OffT, bool HEAVY>
+__global__ __launch_bounds__(kBlock) void k_prref_rows(PrRefArgs a, uint32_t hb) {
+    __shared__ double s_val[kRowsTile];
+    __shared__ uint32_t s_cnt[kWavesPerBlock];
+    const OffT* off = (const OffT*)a.off;
+    const uint32_t* src = a.src - a.e_base;
+    const uint32_t tid = threadIdx.x;
+    uint32_t moved = 0;
+    if (HEAVY && blockIdx.x < hb) {
+        for (uint32_t i = blockIdx.x; i < a.rows.n_front + a.rows.n_back; i += hb) {
+            const uint32_t v = i < a.rows.n_front ? a.rows.front(i) : a.rows.back(i - a.rows.n_front);
+            if (!a.active[v]) continue;   // the same for the whole workgroup: only its own lane 0 clears it, below
+            const OffT b = off[v], e = off[v + 1];
+            // pass t: the ids of pass t + 2 are loaded and the contributions
+            // of pass t + 1 gathered (by the ids loaded a pass ago) while
+            // pass t is added, so that no wave waits for either
+            uint32_t u[kSeqPer];
+            double c[kSeqPer];
+            auto load_ids = [&](OffT t0) {
+#pragma unroll
+                for (int j = 0; j < kSeqPer; j++) u[j] = src[min((OffT)(t0 + j * kBlock + tid), (OffT)(e - 1))];
+            };
+            auto gather = [&] {
+#pragma unroll
+                for (int j = 0; j < kSeqPer; j++) c[j] = a.contrib_in[u[j]];
+            };
+            load_ids(b);
+            gather();
+            load_ids(b + kSeqTile);
+            double s = 0;
+            uint32_t half = 0;   // passes alternate between two halves of s_val: one barrier each
+            __syncthreads();     // the previous row's adds are done
+            for (OffT t0 = b; t0 < e; t0 += kSeqTile, half ^= 1) {
+                double* buf = s_val + half * kSeqTile;
+#pragma unroll
+                for (int j = 0; j < kSeqPer; j++) buf[j * kBlock + tid] = c[j];
+                __syncthreads();
+                if (e - t0 > kSeqTile) {
+                    gather();
+                    load_ids(t0 + 2 * kSeqTile);
+                }
+                if (tid == 0) s = add_chain(s, buf, (uint32_t)min((OffT)kSeqTile, (OffT)(e - t0)));
+            }
+            if (tid == 0) moved += prref_finish(a, v, s);
+        }
+    } else {
+        const uint32_t bid = blockIdx.x - (HEAVY ? hb : 0), nblk = gridDim.x - (HEAVY ? hb : 0);
+        if (HEAVY) {
+            auto pre = [&](uint64_t v) { return a.active[v] != 0; };
+            auto fin = [&](uint64_t v, double s, bool act) {
+                if (act) moved += prref_finish(a, v, s);
+            };
+            for (uint32_t i = bid; i < a.rows.n_blocks; i += nblk) {
+                const RowBlock rb = a.rows.blocks[i];
+                if (__syncthreads_or(tid < rb.n && a.active[rb.v + tid]))   // else every row has stopped
+                    pull_block(off, src, a.contrib_in, rb, s_val, pre, fin);
+            }
+        } else {
+            auto take = [&](uint64_t v) { return a.active[v] != 0; };
+            auto fin = [&](uint64_t v, double s) { moved += prref_finish(a, v, s); };
+            for (uint64_t v = a.v_begin + (uint64_t)bid * kBlock; v < a.v_end; v += (uint64_t)nblk * kBlock)
+                pull_rows(off, src, a.contrib_in, v, a.v_end, s_val, take, fin);
+        }
+    }
+    moved = wave_sum(moved);
+    if (lane_id() == 0) s_cnt[wave_id()] = moved;
+    __syncthreads();
+    if (tid == 0) {
+        uint32_t t = 0;
+        for (int i = 0; i < kWavesPerBlock; i++) t += s_cnt[i];
+        if (t) atomicAdd(a.count + (blockIdx.x % kPrLines) * kPrLineWords, t);
+    }
+}
+
+// Sums and clears an iteration's counters and publishes the sum (one wave).
+__global__ void k_prref_publish(uint32_t* count, PrRefPub* host, unsigned long long seq) {
+    uint32_t n = 0;
+    if (threadIdx.x < kPrLines) {
+        n = count[threadIdx.x * kPrLineWords];
+        count[threadIdx.x * kPrLineWords] = 0;
+    }
+    n = wave_sum(n);
+    if (threadIdx.x == 0) {
+        host->moved = n;
+        __threadfence_system();
+        host->seq = seq;
+    }
 }
 
 // ---- host -------------------------------------------------------------------
+
+constexpr int kRefRing = 4;   // published iterations of the reference mode
+
+// Cuts the resident vertices into row blocks and lists their heavy rows, once
+// per graph.
+template <class OffT>
+static int pr_rows_build(asc_graph* g, PrState* p) {
+    if (p->rows_built) return ASC_OK;
+    const uint64_t n = g->static_vertices;
+    const uint64_t cap = std::min<uint64_t>(n, g->static_edges / kRowsHeavy) + 1;
+    const uint64_t bcap = std::min<uint64_t>(n, (n + kBlock - 1) / kBlock + g->static_edges / kRowsWindow + cap) + 1;
+    hipStream_t s = g->ctx->s_main;
+    DevTmp<uint32_t> d_cnt;
+    uint32_t cnt[3] = {0, 0, 0};
+    if (!p->rows_heavy) ASC_HIP(hipMalloc(&p->rows_heavy, 4 * cap));
+    if (!p->rows_blocks) ASC_HIP(hipMalloc(&p->rows_blocks, sizeof(RowBlock) * bcap));
+    ASC_HIP(hipMalloc(&d_cnt.p, sizeof(cnt)));
+    ASC_HIP(hipMemsetAsync(d_cnt.p, 0, sizeof(cnt), s));
+    if (n) {
+        const int grid = (int)std::min<uint64_t>((n + kBlock - 1) / kBlock, (uint64_t)g->ctx->num_cus * 8);
+        hipLaunchKernelGGL((k_rows_heavy_list<OffT>), dim3(grid), dim3(kBlock), 0, s, (const OffT*)g->d_off, n,
+                           p->rows_heavy, (uint32_t)cap, d_cnt.p);
+        hipLaunchKernelGGL((k_row_blocks<OffT>), dim3(grid), dim3(kBlock), 0, s, (const OffT*)g->d_off, n,
+                           (RowBlock*)p->rows_blocks, d_cnt.p + 2);
+        ASC_HIP(hipGetLastError());
+    }
+    ASC_HIP(hipMemcpyAsync(cnt, d_cnt.p, sizeof(cnt), hipMemcpyDeviceToHost, s));
+    ASC_HIP(hipStreamSynchronize(s));
+    p->rows_cap = (uint32_t)cap;
+    p->rows_front = cnt[0];
+    p->rows_back = cnt[1];
+    p->rows_n = cnt[2];
+    p->rows_built = true;
+    return ASC_OK;
+}
+
+static RowPlan row_plan(const PrState* p) {
+    return RowPlan{(const RowBlock*)p->rows_blocks, p->rows_heavy, p->rows_n, p->rows_cap, p->rows_front,
+                   p->rows_back};
+}
 
 static int pr_ensure(asc_graph* g, int iters, bool ref) {
     PrState* p = g->pr;
@@ -657,46 +1117,52 @@ static int pr_ensure(asc_graph* g, int iters, bool ref) {
             ASC_HIP(hipMalloc(&p->contrib[i], 4 * V));
         }
     }
-    if (!ref && p->acc_iters < iters) {
-        if (p->acc) (void)hipFree(p->acc);
-        ASC_HIP(hipMalloc(&p->acc, sizeof(double) * (2 * (size_t)iters + 1)));
-        p->acc_iters = iters;
-    }
-    const int thr = 4096;  // in-degree from which a workgroup sums one vertex
-    if (!ref && p->heavy_thr != thr) {
-        // resident vertices only: their in-edges are on the device
-        std::vector<uint32_t> hv;
-        for (uint64_t v = 0; v < g->static_vertices; v++)
-            if (g->h.off[v + 1] - g->h.off[v] >= (uint64_t)thr) hv.push_back((uint32_t)v);
-        p->n_heavy = (uint32_t)hv.size();
-        p->heavy_thr = thr;
-        if (!hv.empty()) {
-            ASC_HIP(hipMalloc(&p->heavy, 4 * hv.size()));
-            ASC_HIP(hipMemcpy(p->heavy, hv.data(), 4 * hv.size(), hipMemcpyHostToDevice));
-        }
+    if (!ref && !p->acc) ASC_HIP(hipMalloc(&p->acc, sizeof(double) * kAccSlots * kAccSlot));
+    if (!ref && p->resid_iters < iters) {
+        if (p->resid) (void)hipFree(p->resid);
+        p->resid = nullptr;
+        p->resid_iters = 0;
+        ASC_HIP(hipMalloc(&p->resid, sizeof(double) * (size_t)iters));
+        p->resid_iters = iters;
     }
     if (ref && !p->val64) {
-        ASC_HIP(hipMalloc(&p->val64, 8 * V));
-        ASC_HIP(hipMalloc(&p->sum64, 8 * V));
-        ASC_HIP(hipMalloc(&p->contrib64, 8 * V));
+        ASC_HIP(hipMalloc(&p->contrib64[0], 8 * V));
+        ASC_HIP(hipMalloc(&p->contrib64[1], 8 * V));
         ASC_HIP(hipMalloc(&p->active, V));
-        ASC_HIP(hipMalloc(&p->count, 4));
-        ASC_TRY(p->h_count.alloc(1, true));
+        ASC_HIP(hipMalloc(&p->count, 4 * kPrLines * kPrLineWords));
+        ASC_TRY(p->h_refpub.alloc(kRefRing, true));
+        ASC_HIP(hipHostGetDevicePointer((void**)&p->d_refpub, p->h_refpub.p, 0));
+        for (int i = 0; i < kRefRing; i++) p->h_refpub[i].seq = 0;
+        ASC_HIP(hipMalloc(&p->val64, 8 * V));   // last: set once all of the above are
     }
     return pr_plan_chunks(g, p);
 }
 
-static int pr_group_for(const asc_graph* g) {
-    if (g->pr_group > 0) return g->pr_group;
-    const double avg = g->h.V ? (double)g->h.E / (double)g->h.V : 0;
-    if (avg >= 48) return 32;
-    if (avg >= 12) return 16;
-    if (avg >= 6) return 8;
-    return 4;
-}
-
+// One pull over [a.v_begin, a.v_end): the row kernel (with its heavy rows when
+// a.skip_heavy), or k_pr_pull with the G lanes per vertex asked for.
+// Measured on R-MAT scale 18 (7.6 M in-edges): the row kernel 40 us an
+// iteration; 16 lanes a vertex, heavy rows from 4096 edges on, 283 us (a group
+// walks up to 4095 edges, and the heavy kernel held one gather in flight).
+// What is left is mostly the 128-byte L2 line that every 4-byte gather brings
+// into L1: 64 bytes a clock per CU make 7.6 M of them 25 us.
 template <class OffT>
-static int launch_pull(int G, int grid, hipStream_t s, const PrArgs& a) {
+static int launch_pull(int G, int num_cus, hipStream_t s, const PrArgs& a, const PrState* p) {
+    const uint64_t n = a.v_end - a.v_begin;
+    const uint32_t cap = (uint32_t)num_cus * 8;
+    if (G == 0) {
+        if (a.skip_heavy) {
+            const uint32_t hb = std::min<uint32_t>(p->rows_front + (p->rows_back + kWavesPerBlock - 1) / kWavesPerBlock,
+                                                   cap / 2);
+            hipLaunchKernelGGL((k_pr_rows<OffT, true>), dim3(hb + std::min(p->rows_n, cap)), dim3(kBlock), 0, s, a,
+                               row_plan(p), hb);
+        } else {
+            const uint32_t rb = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((n + kBlock - 1) / kBlock, cap));
+            hipLaunchKernelGGL((k_pr_rows<OffT, false>), dim3(rb), dim3(kBlock), 0, s, a, RowPlan{}, 0u);
+        }
+        ASC_HIP(hipGetLastError());
+        return ASC_OK;
+    }
+    const uint32_t grid = (uint32_t)std::min<uint64_t>(cap, (n * G + kBlock - 1) / kBlock + 1);
     switch (G) {
         case 4: hipLaunchKernelGGL((k_pr_pull<4, OffT>), dim3(grid), dim3(kBlock), 0, s, a); break;
         case 8: hipLaunchKernelGGL((k_pr_pull<8, OffT>), dim3(grid), dim3(kBlock), 0, s, a); break;
@@ -757,7 +1223,7 @@ static int pr_blocked_build(asc_graph* g, PrState* p) {
     hipLaunchKernelGGL((k_pb_src<unsigned long long>), dim3(grid), dim3(kBlock), 0, s, d_out_off.p, V, p->pb_src);
     ASC_HIP(hipGetLastError());
     // slot layout: counts per (bin, range), exclusive scan in bin-major order
-    const uint32_t thr = (uint32_t)p->heavy_thr;
+    const uint32_t thr = kRowsLong;
     ASC_HIP(hipMalloc(&d_cnt.p, 4 * (size_t)kPbRanges * nb));
     hipLaunchKernelGGL((k_pb_count<OffT>), dim3(std::min<uint32_t>(kPbRanges, grid)), dim3(kBlock), 0, s, out_dst, E,
                        in_off, thr, (uint32_t)nb, d_cnt.p);
@@ -817,7 +1283,7 @@ static int pr_tiled_build(asc_graph* g, PrState* p, uint32_t sb, uint32_t db) {
     hipStream_t s = g->ctx->s_main;
     const OffT* off = (const OffT*)g->d_off;
     const uint32_t* src = (const uint32_t*)g->d_edges;
-    const uint32_t thr = (uint32_t)p->heavy_thr;
+    const uint32_t thr = kRowsLong;
     const TileShape ts{sb, db, (uint32_t)ns, (uint32_t)nd};
     DevTmp<uint32_t> d_cnt;
     ASC_HIP(hipMalloc(&d_cnt.p, 4 * nd * ns));
@@ -860,13 +1326,14 @@ static int pr_normalised(asc_graph* g, const asc_pr_opts* o, float* rank_out, do
     const uint64_t V = g->h.V;
     hipStream_t s = ctx->s_main;
     const int grid = ctx->num_cus * 8;
-    ASC_HIP(hipMemsetAsync(p->acc, 0, sizeof(double) * (2 * (size_t)iters + 1), s));
-    double* resid = p->acc;
-    double* dang = p->acc + iters;
-    hipLaunchKernelGGL(k_pr_init, dim3(grid), dim3(kBlock), 0, s, p->rank[0], p->contrib[0], g->d_outdeg, V, dang);
+    ASC_TRY(pr_rows_build<OffT>(g, p));
+    auto slot = [&](int it) { return p->acc + (size_t)(it % kAccSlots) * kAccSlot; };
+    ASC_HIP(hipMemsetAsync(p->acc, 0, sizeof(double) * kAccSlots * kAccSlot, s));
+    hipLaunchKernelGGL(k_pr_init, dim3(std::max<uint64_t>(1, std::min<uint64_t>((V + kBlock - 1) / kBlock, (uint64_t)grid))), dim3(kBlock), 0,
+                       s, p->rank[0], p->contrib[0], g->d_outdeg, V, slot(0));
     ASC_HIP(hipGetLastError());
     ASC_HIP(hipStreamSynchronize(s));
-    const int G = pr_group_for(g);
+    const int G = g->pr_group > 0 ? g->pr_group : 0;
     if (o->method == ASC_PR_BLOCKED) ASC_TRY(pr_blocked_build<OffT>(g, p));
     const bool blocked = o->method == ASC_PR_BLOCKED && p->pb_state == 1;
     if (o->method == ASC_PR_BLOCKED && !blocked) {
@@ -908,13 +1375,19 @@ static int pr_normalised(asc_graph* g, const asc_pr_opts* o, float* rank_out, do
         a.contrib_in = p->contrib[it & 1];
         a.rank_out = p->rank[(it + 1) & 1];
         a.contrib_out = p->contrib[(it + 1) & 1];
-        a.dang_in = dang + it;
-        a.dang_out = dang + it + 1;
-        a.residual = resid + it;
+        a.acc_in = slot(it);
+        a.acc_out = slot(it + 1);
+        // only the iteration's first launch: `led` takes these off for the others
+        a.acc_clear = slot(it + 2);
+        a.resid_prev = it ? p->resid + it - 1 : nullptr;
+        auto led = [&] {
+            a.acc_clear = nullptr;
+            a.resid_prev = nullptr;
+        };
         a.V = V;
         a.damping = (float)o->damping;
         a.damping64 = o->damping;
-        a.heavy_thr = (uint32_t)p->heavy_thr;
+        a.heavy_thr = kRowsLong;
         // resident vertices from the device edges, heavy in-lists by workgroups
         a.e_base = 0;
         a.v_begin = 0;
@@ -926,7 +1399,7 @@ static int pr_normalised(asc_graph* g, const asc_pr_opts* o, float* rank_out, do
             // destinations (64 KB of LDS each), one with 2^15 (128 KB)
             const bool big = p->tl_db > 14;
             const uint32_t tgrid = (uint32_t)std::min<uint64_t>((uint64_t)ctx->num_cus * (big ? 1 : 2), p->tl_nd);
-            const uint32_t* hb = p->n_heavy ? (const uint32_t*)p->tl_heavy : nullptr;
+            const uint32_t* hb = p->rows_front ? (const uint32_t*)p->tl_heavy : nullptr;
             if (big)
                 hipLaunchKernelGGL(k_pr_tiled<15>, dim3(tgrid), dim3(kTlBlock), 0, s, a,
                                    (const uint32_t*)p->tl_edges, (const unsigned long long*)p->tl_off, ts, hb);
@@ -934,18 +1407,22 @@ static int pr_normalised(asc_graph* g, const asc_pr_opts* o, float* rank_out, do
                 hipLaunchKernelGGL(k_pr_tiled<14>, dim3(tgrid), dim3(kTlBlock), 0, s, a,
                                    (const uint32_t*)p->tl_edges, (const unsigned long long*)p->tl_off, ts, hb);
             ASC_HIP(hipGetLastError());
+            led();
         } else if (blocked) {
             hipLaunchKernelGGL(k_pb_scatter, dim3(grid), dim3(kBlock), 0, s, p->pb_src, p->pb_pos, p->pb_edges,
                                a.contrib_in, p->pb_vals);
             hipLaunchKernelGGL((k_pb_gather<OffT>), dim3(p->pb_nbins), dim3(kPbBlock), 0, s, a, p->pb_bin_start,
                                p->pb_cnt, p->pb_dl, p->pb_vals);
             ASC_HIP(hipGetLastError());
+            led();
         } else if (a.v_end > 0) {
-            ASC_TRY(launch_pull<OffT>(G, grid, s, a));
+            ASC_TRY(launch_pull<OffT>(G, ctx->num_cus, s, a, p));
+            led();
         }
-        if (p->n_heavy) {
-            hipLaunchKernelGGL((k_pr_pull_heavy<OffT>), dim3(std::min<uint32_t>(p->n_heavy, grid)), dim3(kBlock), 0,
-                               s, a, p->heavy, p->n_heavy);
+        // rows of kRowsLong edges and more (the row kernel takes them itself)
+        if (p->rows_front && (tiled || blocked || G)) {
+            hipLaunchKernelGGL((k_pr_pull_heavy<OffT>), dim3(std::min<uint32_t>(p->rows_front, grid)), dim3(kBlock), 0,
+                               s, a, p->rows_heavy, p->rows_front);
             ASC_HIP(hipGetLastError());
         }
         // on-demand vertices from streamed chunks
@@ -956,17 +1433,20 @@ static int pr_normalised(asc_graph* g, const asc_pr_opts* o, float* rank_out, do
             c.v_begin = v0;
             c.v_end = v1;
             c.skip_heavy = 0;
-            const int cgrid = (int)std::min<uint64_t>(grid, (v1 - v0 + 63) / 64 + 1);
-            return launch_pull<OffT>(G, cgrid, s, c);
+            led();
+            return launch_pull<OffT>(G, ctx->num_cus, s, c, p);
         }));
     }
+    hipLaunchKernelGGL(k_pr_last_residual, dim3(1), dim3(kWave), 0, s, (const double*)slot(iters),
+                       p->resid + iters - 1);
+    ASC_HIP(hipGetLastError());
     ASC_HIP(hipEventRecord(e1.e, s));
     ASC_HIP(hipStreamSynchronize(s));
     const double t1 = now_ms();
     float kms = 0;
     (void)hipEventElapsedTime(&kms, e0.e, e1.e);
     std::vector<double> hres(iters);
-    ASC_HIP(hipMemcpy(hres.data(), resid, sizeof(double) * iters, hipMemcpyDeviceToHost));
+    ASC_HIP(hipMemcpy(hres.data(), p->resid, sizeof(double) * iters, hipMemcpyDeviceToHost));
     if (residual_out) std::memcpy(residual_out, hres.data(), sizeof(double) * iters);
     if (rank_out) ASC_HIP(hipMemcpy(rank_out, p->rank[iters & 1], 4 * V, hipMemcpyDeviceToHost));
     if (st) {
@@ -1006,38 +1486,69 @@ static int pr_reference(asc_graph* g, const asc_pr_opts* o, double* rank_out, as
     const double damping = o->damping;
     const double base = damping == 0.85 ? 0.15 : 1.0 - damping;
     const int maxit = o->max_iterations > 0 ? o->max_iterations : 10000;
-    hipLaunchKernelGGL(k_prref_init, dim3(grid), dim3(256), 0, s, p->val64, p->active, V);
+    ASC_TRY(pr_rows_build<OffT>(g, p));
+    ASC_HIP(hipMemsetAsync(p->count, 0, 4 * kPrLines * kPrLineWords, s));
+    hipLaunchKernelGGL(k_prref_init, dim3(grid), dim3(256), 0, s, p->val64, p->contrib64[0], p->active, g->d_outdeg,
+                       V);
     ASC_HIP(hipGetLastError());
     ASC_HIP(hipStreamSynchronize(s));
     const double t0 = now_ms();
-    uint64_t node_sum = V;
-    uint32_t active = (uint32_t)V;
-    int it = 0;
-    while (active && it < maxit) {
-        it++;
-        hipLaunchKernelGGL(k_prref_contrib, dim3(grid), dim3(256), 0, s, p->val64, g->d_outdeg, p->contrib64, V);
-        if (g->static_vertices)
-            hipLaunchKernelGGL((k_prref_sum<OffT>), dim3(grid), dim3(256), 0, s, (const OffT*)g->d_off,
-                               (const uint32_t*)g->d_edges, 0ull, p->contrib64, p->active, p->sum64, 0ull,
-                               (unsigned long long)g->static_vertices);
+    // Queues iteration `it` (from 1) and the publish of its count.
+    const unsigned long long seq0 = p->ref_seq;
+    auto iterate = [&](int it) -> int {
+        p->ref_seq = seq0 + (unsigned long long)it;
+        PrRefArgs a{};
+        a.off = g->d_off;
+        a.contrib_in = p->contrib64[(it + 1) & 1];
+        a.contrib_out = p->contrib64[it & 1];
+        a.val = p->val64;
+        a.active = p->active;
+        a.outdeg = g->d_outdeg;
+        a.count = p->count;
+        a.base = base;
+        a.damping = damping;
+        a.threshold = o->threshold;
+        if (g->static_vertices) {
+            a.src = (const uint32_t*)g->d_edges;
+            a.v_end = g->static_vertices;
+            a.rows = row_plan(p);
+            const uint32_t hb = std::min<uint32_t>(p->rows_front + p->rows_back, (uint32_t)grid / 2);
+            const uint32_t rb = std::min<uint32_t>(p->rows_n, (uint32_t)grid);
+            hipLaunchKernelGGL((k_prref_rows<OffT, true>), dim3(hb + rb), dim3(kBlock), 0, s, a, hb);
+            ASC_HIP(hipGetLastError());
+        }
         ASC_TRY(pr_stream_chunks(g, p, [&](const uint32_t* src, uint64_t e0, uint64_t v0, uint64_t v1) {
-            const int cgrid = (int)std::min<uint64_t>(grid, (v1 - v0 + 255) / 256);
-            hipLaunchKernelGGL((k_prref_sum<OffT>), dim3(cgrid), dim3(256), 0, s, (const OffT*)g->d_off, src,
-                               (unsigned long long)e0, p->contrib64, p->active, p->sum64, (unsigned long long)v0,
-                               (unsigned long long)v1);
+            PrRefArgs c = a;
+            c.src = src;
+            c.e_base = e0;
+            c.v_begin = v0;
+            c.v_end = v1;
+            const int cgrid = (int)std::max<uint64_t>(1, std::min<uint64_t>(grid, (v1 - v0 + 255) / 256));
+            hipLaunchKernelGGL((k_prref_rows<OffT, false>), dim3(cgrid), dim3(kBlock), 0, s, c, 0u);
             ASC_HIP(hipGetLastError());
             return ASC_OK;
         }));
-        ASC_HIP(hipMemsetAsync(p->count, 0, 4, s));
-        hipLaunchKernelGGL(k_prref_update, dim3(grid), dim3(256), 0, s, p->val64, p->sum64, p->active, V, base,
-                           damping, o->threshold, p->count);
+        hipLaunchKernelGGL(k_prref_publish, dim3(1), dim3(kWave), 0, s, p->count, p->d_refpub + it % kRefRing,
+                           p->ref_seq);
         ASC_HIP(hipGetLastError());
-        ASC_HIP(hipMemcpyAsync(p->h_count.p, p->count, 4, hipMemcpyDeviceToHost, s));
-        ASC_HIP(hipStreamSynchronize(s));
-        active = p->h_count[0];
+        return ASC_OK;
+    };
+    uint64_t node_sum = V;
+    uint64_t active = V;
+    // A resident graph's next iteration is queued before the count of the
+    // current one arrives: after the last one it finds no active vertex and
+    // changes nothing.  A streamed one would copy its tail for that.
+    const int ahead = p->chunks.empty() ? 1 : 0;
+    int it = 0, queued = 0;
+    while (active && it < maxit) {
+        it++;
+        for (; queued < std::min(it + ahead, maxit);) ASC_TRY(iterate(++queued));
+        ASC_TRY(wait_host_seq(&p->h_refpub.p[it % kRefRing].seq, seq0 + (unsigned long long)it, s));
+        active = (uint64_t)((const volatile PrRefPub*)p->h_refpub.p)[it % kRefRing].moved;
         node_sum += active;
     }
     const double t1 = now_ms();
+    ASC_HIP(hipStreamSynchronize(s));   // a queued iteration past the last
     if (rank_out) ASC_HIP(hipMemcpy(rank_out, p->val64, 8 * V, hipMemcpyDeviceToHost));
     if (st) {
         std::memset(st, 0, sizeof(*st));

@@ -134,7 +134,8 @@ typedef struct {
     int heavy_threshold;         /* degree at/above which a frontier vertex is
                                     expanded grid-cooperatively; 0 = tuned    */
     int pr_group;                /* lanes per vertex in the PageRank pull
-                                    (4,8,16,32,64); 0 = tuned                 */
+                                    (4,8,16,32,64); 0 = blocks of rows, or
+                                    the tuned value                           */
     int sssp_delta;              /* SSSP bucket width (near-far); 0 = tuned,
                                     <0 = plain frontier Bellman-Ford          */
     int verbose;                 /* print per-phase timings like the reference */
