@@ -583,19 +583,33 @@ static int run_bfs_do(asc_graph* g, uint32_t src, uint32_t* out, asc_stats* st) 
             if (!e0) return ASC_ERR_DEVICE;
             ASC_HIP(hipEventRecord(e0, s));
         }
-        if (!bottom_up && level > 0 && mf > m_unexplored / kAlpha) {
-            // queue -> bitmap
-            hipLaunchKernelGGL(k_do_fill, dim3(fill_grid), dim3(kBlock), 0, s, t->bm[cur], words, 0u);
-            hipLaunchKernelGGL(k_queue_to_bitmap, dim3(std::max<uint64_t>(1, std::min<uint64_t>((nf + 255) / 256, grid))),
-                               dim3(kBlock), 0, s, t->q[level & 1], t->slots + (level & 3), t->bm[cur]);
-            bottom_up = true;
-        } else if (bottom_up && nf < V / kBeta && nf < prev_nf) {
+        if (bottom_up && nf < V / kBeta && nf < prev_nf) {
             // bitmap -> queue, slot ring restarted at this level
             hipLaunchKernelGGL(k_do_fill, dim3(1), dim3(kBlock), 0, s, (uint32_t*)t->slots, sizeof(Slot) * 4 / 4, 0u);
             hipLaunchKernelGGL(k_bitmap_to_queue, dim3(std::max<uint64_t>(1, std::min<uint64_t>((words + kBlock - 1) / kBlock, grid))),
                                dim3(kBlock), 0, s, t->bm[cur], (uint32_t)V,
                                t->q[level & 1], &t->slots[level & 3].n_res);
             bottom_up = false;
+        }
+        if (!bottom_up && nf <= kNarrowCap && mf <= kNarrowEdges) {
+            // small top-down levels run back to back in one workgroup
+            NarrowState io;
+            io.level = level;
+            ASC_TRY((narrow_run<ALG_BFS, OffT, EdgeT>(g, a, (uint32_t)nf, 0, 0, io)));
+            const uint64_t reached = io.expanded + io.edges - mf;   // edges of the vertices claimed
+            m_unexplored = m_unexplored > reached ? m_unexplored - reached : 0;
+            level = io.level;
+            prev_nf = nf;
+            nf = io.n;
+            mf = io.edges;
+            continue;
+        }
+        if (!bottom_up && level > 0 && mf > m_unexplored / kAlpha) {
+            // queue -> bitmap
+            hipLaunchKernelGGL(k_do_fill, dim3(fill_grid), dim3(kBlock), 0, s, t->bm[cur], words, 0u);
+            hipLaunchKernelGGL(k_queue_to_bitmap, dim3(std::max<uint64_t>(1, std::min<uint64_t>((nf + 255) / 256, grid))),
+                               dim3(kBlock), 0, s, t->q[level & 1], t->slots + (level & 3), t->bm[cur]);
+            bottom_up = true;
         }
         if (bottom_up) {
             ASC_TRY(timed_launch(t, prof, KERN_BU, s, [&] {

@@ -18,6 +18,12 @@ constexpr int kBlocksPerCU = 8;
 constexpr int kMaxPartBufs = 16;              // device buffers for streamed parts and chunks (round-robin)
 constexpr int kDefaultPartBufs = 4;
 constexpr uint32_t kNoValue = 0xFFFFFFFFu;      // `done` before a vertex was ever expanded
+// limits of a step that k_narrow (narrow.hip) runs in one workgroup: frontier
+// vertices (its LDS), their edges (a CU takes ~4 ns an edge, a wide step ~40 us
+// whatever its size, so the two meet near 8192), far-pile entries of a split
+constexpr uint32_t kNarrowCap = 3072;
+constexpr uint32_t kNarrowEdges = 8192;
+constexpr uint32_t kNarrowFar = 8192;
 constexpr uint32_t kMaxChunks = 4096;           // dense on-demand chunks (LDS histogram size)
 
 // Per-level counters, in a ring of four: level L reads slot L%4, appends to
@@ -135,7 +141,25 @@ struct RunCounters {
 struct LevelPub {
     Slot slot;
     Piles piles;
+    unsigned long long edges;       // edges of a frontier of at most kNarrowCap vertices (else ~0)
     unsigned long long seq;
+};
+
+// A run of narrow steps as k_narrow publishes it (seq last).
+struct NarrowPub {
+    uint32_t level;                 // level reached; its frontier is in q[level & 1]
+    uint32_t n;                     // that frontier's vertices
+    uint32_t n_far, fcur, theta;    // far pile and band
+    uint32_t splits;
+    unsigned long long edges;       // that frontier's edges
+    unsigned long long nodes, expanded;   // vertices and edges expanded
+    unsigned long long seq;
+};
+
+struct NarrowState {
+    uint32_t level = 0, fcur = 0;   // in and out
+    uint32_t n = 0, n_far = 0, theta = 0, splits = 0;
+    uint64_t edges = 0, nodes = 0, expanded = 0;
 };
 
 // Waits until the device has written `want` to *seq (mapped host memory),
@@ -194,6 +218,9 @@ struct TravState {
     HostBuf<LevelPub> h_pub;        // written by the device through d_pub (mapped)
     LevelPub* d_pub = nullptr;
     unsigned long long lvl_seq = 0;
+    HostBuf<NarrowPub> h_narrow;    // written by the device through d_narrow (mapped)
+    NarrowPub* d_narrow = nullptr;
+    unsigned long long narrow_seq = 0;
     HostBuf<DevStats> h_stats;
     // the host gather's index of a round's sparse segment: first record of
     // each listed vertex in the gathered array (written by the device through
@@ -264,6 +291,15 @@ int timed_launch(TravState* t, bool prof, int kind, hipStream_t s, F&& launch) {
     }
     return ASC_OK;
 }
+
+// Runs narrow steps of a fully resident graph from the frontier of io.level
+// (n_in <= kNarrowCap vertices in q[level & 1], or none and a far pile of n_far
+// entries in far[fcur]) until the traversal ends or a step outgrows the narrow
+// limits; the wide kernels can go on from the state left behind.  The band
+// starts at a.theta and advances by `delta`.
+template <int ALGO, class OffT, class EdgeT>
+int narrow_run(asc_graph* g, const TravArgs<OffT, EdgeT>& a, uint32_t n_in, uint32_t n_far, uint32_t delta,
+               NarrowState& io);
 
 // Shared end of a traversal run: kernel statistics from the recorded events
 // and DevStats, the values copied to `out` (value convention applied), and
