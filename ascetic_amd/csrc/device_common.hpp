@@ -40,6 +40,27 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
+// Publishing to mapped host memory that the host polls.  The words before the
+// sequence number are written through to the host (system-scope stores) and
+// the number itself is a releasing store.  Plain stores followed by
+// __threadfence_system() are not enough: the host then saw a new number beside
+// a cache line that still held old words in 30 of 7.4 M publishes (none in
+// 2.5 M this way), and a run that reads an old frontier size ends early.
+template <class T>
+__device__ __forceinline__ void host_store(T* p, T v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+template <class T>
+__device__ __forceinline__ void host_store_words(T* dst, const T& v) {
+    static_assert(sizeof(T) % 4 == 0, "whole words");
+    const uint32_t* s = (const uint32_t*)&v;
+#pragma unroll
+    for (uint32_t i = 0; i < sizeof(T) / 4; i++) host_store((uint32_t*)dst + i, s[i]);
+}
+__device__ __forceinline__ void host_publish(unsigned long long* seq, unsigned long long v) {
+    __hip_atomic_store(seq, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // Inclusive wave scan (Kogge-Stone over cross-lane shuffles).
 template <class T>
 __device__ __forceinline__ T wave_scan_incl(T x) {

@@ -286,6 +286,10 @@ int asc_ctx_create(const asc_config* cfg, asc_ctx** out) {
     ctx->device = c.device;
     ctx->num_cus = prop.multiProcessorCount > 0 ? prop.multiProcessorCount : 1;
     ctx->total_mem = prop.totalGlobalMem;
+    if (hipDeviceGetAttribute(&ctx->wall_khz, hipDeviceAttributeWallClockRate, c.device) != hipSuccess) {
+        (void)hipGetLastError();
+        ctx->wall_khz = 0;
+    }
     if (hipStreamCreateWithFlags(&ctx->s_main, hipStreamNonBlocking) != hipSuccess ||
         hipStreamCreateWithFlags(&ctx->s_copy, hipStreamNonBlocking) != hipSuccess) {
         delete ctx;

@@ -162,6 +162,7 @@ __device__ __forceinline__ void expand_local_body(const TravArgs<OffT, EdgeT>& a
         Slot* z = a.slots + ((level + 2) & 3);
         z->n_res = 0;
         z->heavy = 0;
+        a.stats->t_begin = wall_clock64();
     }
     const uint32_t n = cur->n_res;
     const uint32_t tid = threadIdx.x, lane = lane_id(), w = wave_id();

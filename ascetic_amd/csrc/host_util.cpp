@@ -54,6 +54,7 @@ void ThreadPool::loop(int id) {
 }
 
 void ThreadPool::run(const std::function<void(int, int)>& fn) {
+    std::lock_guard<std::mutex> one(run_mu_);   // one job at a time: the pool is shared by calling threads
     if (workers_.empty()) {
         fn(0, 1);
         return;

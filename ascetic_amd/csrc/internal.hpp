@@ -130,6 +130,35 @@ struct DevTmp {
     }
 };
 
+// Several device arrays in one allocation (one of a megabyte or more takes
+// ~270 us): add() each, then alloc() once; freed with the arena.
+struct DevArena {
+    std::vector<std::pair<void**, size_t>> parts;
+    char* p = nullptr;
+    size_t bytes = 0;
+    DevArena() = default;
+    DevArena(const DevArena&) = delete;
+    DevArena& operator=(const DevArena&) = delete;
+    ~DevArena() {
+        if (p) (void)hipFree(p);
+    }
+    template <class T>
+    void add(T** at, size_t count) {
+        parts.push_back({(void**)at, bytes});
+        bytes += (count * sizeof(T) + 255) & ~size_t(255);
+    }
+    int alloc() {
+        if (hipMalloc(&p, bytes ? bytes : 256) != hipSuccess) {
+            (void)hipGetLastError();
+            p = nullptr;
+            set_last_error("device allocation of %zu bytes failed", bytes);
+            return ASC_ERR_DEVICE;
+        }
+        for (auto& x : parts) *x.first = p + x.second;
+        return ASC_OK;
+    }
+};
+
 // A timing event destroyed when it leaves scope.
 struct ScopedEvent {
     hipEvent_t e = nullptr;
@@ -174,6 +203,7 @@ public:
 private:
     void loop(int id);
     std::vector<std::thread> workers_;
+    std::mutex run_mu_;             // held by run()
     std::mutex mu_;
     std::condition_variable cv_, done_cv_;
     const std::function<void(int, int)>* job_ = nullptr;
@@ -199,6 +229,7 @@ struct asc_ctx {
     int device = 0;
     int num_cus = 0;
     uint64_t total_mem = 0;
+    int wall_khz = 0;               // rate of the devices' constant clock (wall_clock64)
     hipStream_t s_main = nullptr;   // kernels
     hipStream_t s_copy = nullptr;   // host<->device transfers of on-demand parts
     asc::ThreadPool* pool = nullptr;  // gather threads

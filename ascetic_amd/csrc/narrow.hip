@@ -64,6 +64,7 @@ __global__ __launch_bounds__(kNwBlock) void k_narrow(TravArgs<OffT, EdgeT> a, Na
     __shared__ unsigned long long s_cnt[3];
     __shared__ uint32_t s_nfar[2], s_min;
     const uint32_t tid = threadIdx.x;
+    const unsigned long long t_begin = wall_clock64();
     uint32_t level = na.level, fcur = na.fcur, theta = na.theta;
     unsigned long long nodes = 0, edges = 0;
     uint32_t steps = 0, splits = 0;
@@ -287,18 +288,18 @@ __global__ __launch_bounds__(kNwBlock) void k_narrow(TravArgs<OffT, EdgeT> a, Na
         na.piles->n_far[fcur ^ 1] = 0;
         a.stats->edges_local += edges;
         a.stats->verts_local += nodes;
+        a.stats->ticks += wall_clock64() - t_begin;
         NarrowPub* o = na.pub;
-        o->level = level;
-        o->n = (uint32_t)(c >> kNwCntShift);
-        o->edges = c & kNwCntMask;
-        o->n_far = s_nfar[fcur];
-        o->fcur = fcur;
-        o->theta = theta;
-        o->splits = splits;
-        o->nodes = nodes;
-        o->expanded = edges;
-        __threadfence_system();
-        o->seq = na.seq;
+        host_store(&o->level, level);
+        host_store(&o->n, (uint32_t)(c >> kNwCntShift));
+        host_store(&o->edges, c & kNwCntMask);
+        host_store(&o->n_far, s_nfar[fcur]);
+        host_store(&o->fcur, fcur);
+        host_store(&o->theta, theta);
+        host_store(&o->splits, splits);
+        host_store(&o->nodes, nodes);
+        host_store(&o->expanded, edges);
+        host_publish(&o->seq, na.seq);
     }
 }
 
@@ -314,7 +315,7 @@ int narrow_run(asc_graph* g, const TravArgs<OffT, EdgeT>& a, uint32_t n_in, uint
         na.far[i] = t->far[i];
     }
     na.piles = t->piles;
-    na.pub = t->d_narrow;
+    na.pub = &t->d_h->narrow;
     na.seq = ++t->narrow_seq;
     na.level = io.level;
     na.n_in = n_in;
@@ -324,25 +325,14 @@ int narrow_run(asc_graph* g, const TravArgs<OffT, EdgeT>& a, uint32_t n_in, uint
     na.delta = delta;
     na.edge_limit = kNarrowEdges;
     na.V = (uint32_t)g->h.V;
-    hipEvent_t e0 = nullptr, e1 = nullptr;
-    if (!prof) {
-        e0 = next_event(t);
-        e1 = next_event(t);
-        if (!e0 || !e1) return ASC_ERR_DEVICE;
-        ASC_HIP(hipEventRecord(e0, s));
-    }
     ASC_TRY(timed_launch(t, prof, KERN_LOCAL, s, [&] {
         if (ALGO == ALG_BFS && g->h.V <= kNwLdsBits)
             hipLaunchKernelGGL((k_narrow<ALGO, OffT, EdgeT, ALGO == ALG_BFS>), dim3(1), dim3(kNwBlock), 0, s, a, na);
         else
             hipLaunchKernelGGL((k_narrow<ALGO, OffT, EdgeT, false>), dim3(1), dim3(kNwBlock), 0, s, a, na);
     }));
-    if (!prof) {
-        ASC_HIP(hipEventRecord(e1, s));
-        t->timed.push_back({-1, e0, e1});
-    }
-    ASC_TRY(wait_host_seq(&t->h_narrow.p->seq, na.seq, s));
-    const volatile NarrowPub* o = t->h_narrow.p;
+    ASC_TRY(wait_host_seq(&t->h[0].narrow.seq, na.seq, s));
+    const volatile NarrowPub* o = &t->h[0].narrow;
     io.level = o->level;
     io.n = o->n;
     io.edges = o->edges;

@@ -37,6 +37,11 @@ struct PrState {
     double* acc = nullptr;        // ring of kAccSlots slots of kAccSlot sums (PrArgs::acc_in / acc_out)
     double* resid = nullptr;      // residual of each iteration
     int resid_iters = 0;
+    HostBuf<double> h_resid;      // the same on the host, and a sequence number behind them (mapped)
+    double* d_hresid = nullptr;
+    unsigned long long resid_seq = 0;
+    hipEvent_t ev[2] = {nullptr, nullptr};   // first and last kernel of a run
+    OutStage out;
     // reference mode
     double* val64 = nullptr;
     double* contrib64[2] = {nullptr, nullptr};   // read by / written for the next iteration
@@ -98,6 +103,7 @@ void pr_free(PrState* p) {
     f(p->pb_src); f(p->pb_pos); f(p->pb_dl); f(p->pb_vals); f(p->pb_bin_start); f(p->pb_cnt);
     f(p->tl_edges); f(p->tl_off); f(p->tl_heavy);
     for (int i = 0; i < 2; i++) {
+        if (p->ev[i]) (void)hipEventDestroy(p->ev[i]);
         if (p->ev_copy[i]) (void)hipEventDestroy(p->ev_copy[i]);
         if (p->ev_kern[i]) (void)hipEventDestroy(p->ev_kern[i]);
     }
@@ -429,10 +435,14 @@ __global__ __launch_bounds__(kBlock) void k_pr_init(float* rank, float* contrib,
     acc_add<kBlock>(0.0, dang, acc);
 }
 
-// The last iteration's residual (one wave).
-__global__ void k_pr_last_residual(const double* slot, double* resid) {
+// The last iteration's residual, then all of them to mapped host memory and
+// the sequence number the host polls for behind them (one wave).
+__global__ void k_pr_residuals(const double* slot, double* resid, int iters, double* host, unsigned long long seq) {
     const double r = acc_lines(slot);
-    if (threadIdx.x == 0) *resid = r;
+    for (int i = threadIdx.x; i < iters; i += kWave) host_store(host + i, i == iters - 1 ? r : resid[i]);
+    __threadfence_system();   // every lane's, before the one lane publishes
+    __builtin_amdgcn_wave_barrier();
+    if (threadIdx.x == 0) host_publish((unsigned long long*)(host + iters), seq);
 }
 
 struct PrArgs {
@@ -1053,9 +1063,8 @@ __global__ void k_prref_publish(uint32_t* count, PrRefPub* host, unsigned long l
     }
     n = wave_sum(n);
     if (threadIdx.x == 0) {
-        host->moved = n;
-        __threadfence_system();
-        host->seq = seq;
+        host_store(&host->moved, (unsigned long long)n);
+        host_publish(&host->seq, seq);
     }
 }
 
@@ -1117,12 +1126,17 @@ static int pr_ensure(asc_graph* g, int iters, bool ref) {
             ASC_HIP(hipMalloc(&p->contrib[i], 4 * V));
         }
     }
+    for (int i = 0; i < 2; i++)
+        if (!p->ev[i]) ASC_HIP(hipEventCreate(&p->ev[i]));
     if (!ref && !p->acc) ASC_HIP(hipMalloc(&p->acc, sizeof(double) * kAccSlots * kAccSlot));
     if (!ref && p->resid_iters < iters) {
         if (p->resid) (void)hipFree(p->resid);
         p->resid = nullptr;
         p->resid_iters = 0;
         ASC_HIP(hipMalloc(&p->resid, sizeof(double) * (size_t)iters));
+        ASC_TRY(p->h_resid.alloc((size_t)iters + 1, true));
+        std::memset((void*)p->h_resid.p, 0, sizeof(double) * ((size_t)iters + 1));
+        ASC_HIP(hipHostGetDevicePointer((void**)&p->d_hresid, p->h_resid.p, 0));
         p->resid_iters = iters;
     }
     if (ref && !p->val64) {
@@ -1332,7 +1346,6 @@ static int pr_normalised(asc_graph* g, const asc_pr_opts* o, float* rank_out, do
     hipLaunchKernelGGL(k_pr_init, dim3(std::max<uint64_t>(1, std::min<uint64_t>((V + kBlock - 1) / kBlock, (uint64_t)grid))), dim3(kBlock), 0,
                        s, p->rank[0], p->contrib[0], g->d_outdeg, V, slot(0));
     ASC_HIP(hipGetLastError());
-    ASC_HIP(hipStreamSynchronize(s));
     const int G = g->pr_group > 0 ? g->pr_group : 0;
     if (o->method == ASC_PR_BLOCKED) ASC_TRY(pr_blocked_build<OffT>(g, p));
     const bool blocked = o->method == ASC_PR_BLOCKED && p->pb_state == 1;
@@ -1361,11 +1374,8 @@ static int pr_normalised(asc_graph* g, const asc_pr_opts* o, float* rank_out, do
         set_last_error("source-segmented PageRank needs every edge resident, V <= 2^31 and room for its tiles");
         return ASC_ERR_UNSUPPORTED;
     }
-    ScopedEvent e0, e1;
-    ASC_HIP(hipEventCreate(&e0.e));
-    ASC_HIP(hipEventCreate(&e1.e));
     const double t0 = now_ms();
-    ASC_HIP(hipEventRecord(e0.e, s));
+    ASC_HIP(hipEventRecord(p->ev[0], s));
     for (int it = 0; it < iters; it++) {
         PrArgs a{};
         a.off = g->d_off;
@@ -1437,18 +1447,26 @@ static int pr_normalised(asc_graph* g, const asc_pr_opts* o, float* rank_out, do
             return launch_pull<OffT>(G, ctx->num_cus, s, c, p);
         }));
     }
-    hipLaunchKernelGGL(k_pr_last_residual, dim3(1), dim3(kWave), 0, s, (const double*)slot(iters),
-                       p->resid + iters - 1);
+    ASC_HIP(hipEventRecord(p->ev[1], s));
+    // the host copies hold `iters` residuals and the sequence number right
+    // behind them, whatever their capacity
+    volatile unsigned long long* seq = (volatile unsigned long long*)(p->h_resid.p + iters);
+    *seq = 0;
+    const unsigned long long want = ++p->resid_seq;
+    hipLaunchKernelGGL(k_pr_residuals, dim3(1), dim3(kWave), 0, s, (const double*)slot(iters), p->resid, iters,
+                       p->d_hresid, want);
     ASC_HIP(hipGetLastError());
-    ASC_HIP(hipEventRecord(e1.e, s));
-    ASC_HIP(hipStreamSynchronize(s));
+    ASC_TRY(wait_host_seq(seq, want, s));
     const double t1 = now_ms();
+    const double* hres = p->h_resid.p;
+    if (residual_out) std::memcpy(residual_out, hres, sizeof(double) * iters);
+    if (rank_out) ASC_TRY(out_copy(p->out, (const uint32_t*)p->rank[iters & 1], V, (uint32_t*)rank_out, s));
     float kms = 0;
-    (void)hipEventElapsedTime(&kms, e0.e, e1.e);
-    std::vector<double> hres(iters);
-    ASC_HIP(hipMemcpy(hres.data(), p->resid, sizeof(double) * iters, hipMemcpyDeviceToHost));
-    if (residual_out) std::memcpy(residual_out, hres.data(), sizeof(double) * iters);
-    if (rank_out) ASC_HIP(hipMemcpy(rank_out, p->rank[iters & 1], 4 * V, hipMemcpyDeviceToHost));
+    if (hipEventElapsedTime(&kms, p->ev[0], p->ev[1]) != hipSuccess) {   // not yet seen by the runtime
+        (void)hipGetLastError();
+        ASC_HIP(hipEventSynchronize(p->ev[1]));
+        (void)hipEventElapsedTime(&kms, p->ev[0], p->ev[1]);
+    }
     if (st) {
         std::memset(st, 0, sizeof(*st));
         st->total_ms = t1 - t0;
@@ -1491,7 +1509,6 @@ static int pr_reference(asc_graph* g, const asc_pr_opts* o, double* rank_out, as
     hipLaunchKernelGGL(k_prref_init, dim3(grid), dim3(256), 0, s, p->val64, p->contrib64[0], p->active, g->d_outdeg,
                        V);
     ASC_HIP(hipGetLastError());
-    ASC_HIP(hipStreamSynchronize(s));
     const double t0 = now_ms();
     // Queues iteration `it` (from 1) and the publish of its count.
     const unsigned long long seq0 = p->ref_seq;
@@ -1548,8 +1565,9 @@ static int pr_reference(asc_graph* g, const asc_pr_opts* o, double* rank_out, as
         node_sum += active;
     }
     const double t1 = now_ms();
-    ASC_HIP(hipStreamSynchronize(s));   // a queued iteration past the last
-    if (rank_out) ASC_HIP(hipMemcpy(rank_out, p->val64, 8 * V, hipMemcpyDeviceToHost));
+    // (a queued iteration past the last runs ahead of the copy and changes nothing)
+    if (rank_out) ASC_TRY(out_copy(p->out, (const uint32_t*)p->val64, 2 * V, (uint32_t*)rank_out, s));
+    else ASC_HIP(hipStreamSynchronize(s));
     if (st) {
         std::memset(st, 0, sizeof(*st));
         st->total_ms = t1 - t0;

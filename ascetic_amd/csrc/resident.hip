@@ -21,7 +21,6 @@
 // Symmetry is decided once per upload from order-independent 64-bit hash
 // sums of (u, v) and of (v, u) over all edges, under two seeds.
 #include <algorithm>
-#include <unordered_map>
 
 #include "device_common.hpp"
 #include "internal.hpp"
@@ -273,6 +272,7 @@ __global__ __launch_bounds__(kBlock) void k_bfs_bottom_up(const OffT* off, const
                                                           uint32_t* visited, const uint32_t* front, uint32_t* next,
                                                           uint32_t V, uint32_t level, DoCounters* c,
                                                           DevStats* stats) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) stats->t_begin = wall_clock64();
     bottom_up_body(off, edges, val, visited, front, next, V, level, c, stats, (uint32_t*)nullptr,
                    (uint32_t*)nullptr, blockIdx.x, gridDim.x);
 }
@@ -323,22 +323,22 @@ __global__ __launch_bounds__(kBlock) void k_do_fill(uint32_t* p, uint64_t n, uin
 // End of a level: the level's counters (and the next top-down frontier's
 // size, in `pad`) are written to mapped host memory, and the device counters
 // are cleared for the next level (no copy or memset dispatch per level).
-__global__ void k_do_publish(DoCounters* c, const Slot* next_slot, DoCounters* host, unsigned long long seq) {
+__global__ void k_do_publish(DoCounters* c, const Slot* next_slot, DevStats* stats, DoCounters* host,
+                             unsigned long long seq) {
     if (threadIdx.x != 0 || blockIdx.x != 0) return;
     const DoCounters v = *c;
-    host->n_found = v.n_found;
-    host->m_found = v.m_found;
-    host->m_frontier = v.m_frontier;
-    host->pad = next_slot ? next_slot->n_res : 0;
-    __threadfence_system();
-    host[1].n_found = seq;   // the counters above are complete (the host polls this word)
+    host_store(&host->n_found, v.n_found);
+    host_store(&host->m_found, v.m_found);
+    host_store(&host->m_frontier, v.m_frontier);
+    host_store(&host->pad, (unsigned long long)(next_slot ? next_slot->n_res : 0));
+    host_publish(&host[1].n_found, seq);   // the counters above are complete (the host polls this word)
     c->n_found = 0;
     c->m_found = 0;
     c->m_frontier = 0;
     c->pad = 0;
+    stats->ticks += wall_clock64() - stats->t_begin;
 }
 
-// Level-0 frontier: the source alone, value 1 (level + 1).
 // ---- persistent direction-optimizing BFS -----------------------------------
 // The whole traversal in one cooperative launch: every level runs between
 // grid barriers, and every workgroup takes the same direction decision from
@@ -498,32 +498,36 @@ __global__ __launch_bounds__(kBlock) void k_bfs_persistent(TravArgs<OffT, EdgeT>
 
 __global__ void k_set_u64(unsigned long long* p, unsigned long long v) { *p = v; }
 
-__global__ void k_do_source(uint32_t* val, uint32_t* visited, uint32_t* q, Slot* slot, uint32_t src) {
-    val[src] = 1;
-    visited[src >> 5] |= 1u << (src & 31);
-    q[0] = src;
-    slot->n_res = 1;
-}
-
 static int ensure_fast_state(asc_graph* g) {
     ASC_TRY(trav_ensure(g));
     TravState* t = g->trav;
     const uint64_t words = (g->h.V + 31) / 32 + 2;
-    if (!t->bm[0]) {
-        ASC_HIP(hipMalloc(&t->bm[0], 4 * words));
-        ASC_HIP(hipMalloc(&t->bm[1], 4 * words));
-        ASC_HIP(hipMalloc(&t->bm[2], 4 * words));
-        ASC_HIP(hipMalloc(&t->pctl, 4 * kPctlWords));
-    }
-    if (!t->dcnt) {
-        ASC_HIP(hipMalloc(&t->dcnt, sizeof(DoCounters)));
-        ASC_TRY(t->h_dcnt.alloc(2, true));   // [0] counters, [1].n_found the publish sequence
-        t->h_dcnt[1].n_found = 0;
-        t->pub_seq = 0;
-        ASC_HIP(hipHostGetDevicePointer((void**)&t->d_hdcnt, t->h_dcnt.p, 0));
-        ASC_TRY(t->h_sample.alloc(kSamples, true));
+    if (!t->mem_fast.p) {
+        t->mem_fast.parts.clear();
+        t->mem_fast.bytes = 0;
+        for (uint32_t** p : {&t->bm[0], &t->bm[1], &t->bm[2]}) t->mem_fast.add(p, words);
+        t->mem_fast.add(&t->pctl, kPctlWords);
+        t->mem_fast.add(&t->dcnt, 1);
+        ASC_TRY(t->mem_fast.alloc());
     }
     return ASC_OK;
+}
+
+static RunInit bfs_init(asc_graph* g, uint32_t src) {
+    TravState* t = g->trav;
+    RunInit ri{};
+    ri.V = g->h.V;
+    ri.val = t->val;
+    ri.visited = t->visited;
+    ri.slots = t->slots;
+    ri.piles = t->piles;
+    ri.stats = t->stats;
+    ri.dcnt = t->dcnt;
+    ri.q0 = t->q[0];
+    ri.src = src;
+    ri.unreached = (uint32_t)(g->h.V + 1);
+    ri.n_res0 = 1;
+    return ri;
 }
 
 template <class OffT, class EdgeT>
@@ -540,14 +544,7 @@ static int run_bfs_do(asc_graph* g, uint32_t src, uint32_t* out, asc_stats* st) 
     const int grid = ctx->num_cus * (g->blocks_per_cu > 0 ? g->blocks_per_cu : kBlocksPerCU);
     const int bu_grid = (int)std::max<uint64_t>(1, std::min<uint64_t>((V + kBlock - 1) / kBlock, (uint64_t)grid));
 
-    hipLaunchKernelGGL(k_do_fill, dim3(1), dim3(kBlock), 0, s, (uint32_t*)t->slots, sizeof(Slot) * 4 / 4, 0u);
-    hipLaunchKernelGGL(k_do_fill, dim3(1), dim3(kBlock), 0, s, (uint32_t*)t->stats, sizeof(DevStats) / 4, 0u);
-    hipLaunchKernelGGL(k_do_fill, dim3(1), dim3(kBlock), 0, s, (uint32_t*)t->dcnt, sizeof(DoCounters) / 4, 0u);
-    hipLaunchKernelGGL(k_do_fill, dim3(fill_grid), dim3(kBlock), 0, s, t->val, V, (uint32_t)(V + 1));
-    hipLaunchKernelGGL(k_do_fill, dim3(fill_grid), dim3(kBlock), 0, s, t->visited, words, 0u);
-    hipLaunchKernelGGL(k_do_source, dim3(1), dim3(1), 0, s, t->val, t->visited, t->q[0], t->slots, src);
-    ASC_HIP(hipGetLastError());
-    ASC_HIP(hipStreamSynchronize(s));
+    ASC_TRY(launch_run_init(bfs_init(g, src), ctx->num_cus, s));
 
     TravArgs<OffT, EdgeT> a{};
     a.off = (const OffT*)g->d_off;
@@ -577,12 +574,6 @@ static int run_bfs_do(asc_graph* g, uint32_t src, uint32_t* out, asc_stats* st) 
     uint32_t level = 0;
     const double t0 = now_ms();
     while (nf > 0) {
-        hipEvent_t e0 = nullptr;
-        if (!prof) {
-            e0 = next_event(t);
-            if (!e0) return ASC_ERR_DEVICE;
-            ASC_HIP(hipEventRecord(e0, s));
-        }
         if (bottom_up && nf < V / kBeta && nf < prev_nf) {
             // bitmap -> queue, slot ring restarted at this level
             hipLaunchKernelGGL(k_do_fill, dim3(1), dim3(kBlock), 0, s, (uint32_t*)t->slots, sizeof(Slot) * 4 / 4, 0u);
@@ -626,23 +617,21 @@ static int run_bfs_do(asc_graph* g, uint32_t src, uint32_t* out, asc_stats* st) 
             ASC_TRY(timed_launch(t, prof, KERN_LOCAL, s, [&] {
                 hipLaunchKernelGGL((k_expand_local<ALG_BFS, OffT, EdgeT>), dim3(lgrid), dim3(kBlock), 0, s, a, level);
             }));
-            ASC_TRY(timed_launch(t, prof, KERN_HEAVY, s, [&] {
-                hipLaunchKernelGGL((k_expand_heavy<ALG_BFS, OffT, EdgeT>), dim3(grid), dim3(kBlock), 0, s, a, level);
-            }));
-        }
-        if (!prof) {
-            hipEvent_t e1 = next_event(t);
-            if (!e1) return ASC_ERR_DEVICE;
-            ASC_HIP(hipEventRecord(e1, s));
-            t->timed.push_back({-1, e0, e1});
+            if (g->max_degree >= a.heavy_thr) {
+                ASC_TRY(timed_launch(t, prof, KERN_HEAVY, s, [&] {
+                    hipLaunchKernelGGL((k_expand_heavy<ALG_BFS, OffT, EdgeT>), dim3(grid), dim3(kBlock), 0, s, a,
+                                       level);
+                }));
+            }
         }
         const unsigned long long want = ++t->pub_seq;
         hipLaunchKernelGGL(k_do_publish, dim3(1), dim3(64), 0, s, t->dcnt,
-                           bottom_up ? (const Slot*)nullptr : t->slots + ((level + 1) & 3), t->d_hdcnt, want);
+                           bottom_up ? (const Slot*)nullptr : t->slots + ((level + 1) & 3), t->stats, t->d_h->bfs,
+                           want);
         ASC_HIP(hipGetLastError());
-        ASC_TRY(wait_host_seq(&t->h_dcnt.p[1].n_found, want, s));
+        ASC_TRY(wait_host_seq(&t->h[0].bfs[1].n_found, want, s));
         prev_nf = nf;
-        const volatile DoCounters* pub = t->h_dcnt.p;   // written by k_do_publish
+        const volatile DoCounters* pub = t->h[0].bfs;   // written by k_do_publish
         if (bottom_up) {
             nf = pub->n_found;
             mf = pub->m_found;
@@ -683,15 +672,10 @@ static int run_bfs_persistent(asc_graph* g, uint32_t src, uint32_t* out, asc_sta
     const int grid = ctx->num_cus * std::min(per_cu, kPersistPerCU);
     DoCounters* ring = (DoCounters*)(t->pctl + kRingWord);
 
-    hipLaunchKernelGGL(k_do_fill, dim3(1), dim3(kBlock), 0, s, (uint32_t*)t->slots, sizeof(Slot) * 4 / 4, 0u);
-    hipLaunchKernelGGL(k_do_fill, dim3(1), dim3(kBlock), 0, s, (uint32_t*)t->stats, sizeof(DevStats) / 4, 0u);
-    hipLaunchKernelGGL(k_do_fill, dim3(1), dim3(kBlock), 0, s, (uint32_t*)t->dcnt, sizeof(DoCounters) / 4, 0u);
+    ASC_TRY(launch_run_init(bfs_init(g, src), ctx->num_cus, s));
     hipLaunchKernelGGL(k_do_fill, dim3(1), dim3(kBlock), 0, s, t->pctl, (uint64_t)kPctlWords, 0u);
-    hipLaunchKernelGGL(k_do_fill, dim3(fill_grid), dim3(kBlock), 0, s, t->val, V, (uint32_t)(V + 1));
-    hipLaunchKernelGGL(k_do_fill, dim3(fill_grid), dim3(kBlock), 0, s, t->visited, words, 0u);
     for (int i = 0; i < 3; i++)
         hipLaunchKernelGGL(k_do_fill, dim3(fill_grid), dim3(kBlock), 0, s, t->bm[i], words, 0u);
-    hipLaunchKernelGGL(k_do_source, dim3(1), dim3(1), 0, s, t->val, t->visited, t->q[0], t->slots, src);
     hipLaunchKernelGGL(k_set_u64, dim3(1), dim3(1), 0, s, &ring[0].m_found,
                        (unsigned long long)(g->h.off[src + 1] - g->h.off[src]));
     ASC_HIP(hipGetLastError());
@@ -785,7 +769,13 @@ __device__ __forceinline__ void uf_link(uint32_t* comp, uint32_t u, uint32_t v) 
     }
 }
 
-__global__ __launch_bounds__(kBlock) void k_uf_init(uint32_t* comp, uint32_t V) {
+__global__ __launch_bounds__(kBlock) void k_uf_init(uint32_t* comp, uint32_t V, DevStats* stats) {
+    if (blockIdx.x == 0) {
+        uint32_t* st = (uint32_t*)stats;
+        for (uint32_t i = threadIdx.x; i < sizeof(DevStats) / 4; i += kBlock) st[i] = 0;
+        __syncthreads();
+        if (threadIdx.x == 0) stats->t_begin = wall_clock64();
+    }
     for (uint32_t v = blockIdx.x * kBlock + threadIdx.x; v < V; v += gridDim.x * kBlock) comp[v] = v;
 }
 
@@ -818,9 +808,23 @@ __global__ __launch_bounds__(kBlock) void k_uf_compress(uint32_t* comp, uint32_t
     }
 }
 
-__global__ void k_uf_gather(const uint32_t* comp, const uint32_t* idx, uint32_t n, uint32_t* out) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] = comp[idx[i]];
+// Most common component among kSamples vertices (a fixed SplitMix64 sequence,
+// so runs are repeatable; the smallest label of those tied).  One workgroup of
+// kSamples lanes, each counting its own label among all.
+__global__ __launch_bounds__(kSamples) void k_uf_giant(const uint32_t* comp, uint64_t V, uint32_t* giant) {
+    __shared__ uint32_t s_label[kSamples];
+    __shared__ unsigned long long s_best;
+    const uint32_t i = threadIdx.x;
+    const uint64_t z = mix64(0x243f6a8885a308d3ull + (i + 1) * 0x9e3779b97f4a7c15ull);
+    const uint32_t label = comp[z % V];
+    s_label[i] = label;
+    if (i == 0) s_best = 0;
+    __syncthreads();
+    uint32_t n = 0;
+    for (int j = 0; j < kSamples; j++) n += s_label[j] == label;
+    atomicMax(&s_best, ((unsigned long long)n << 32) | (0xFFFFFFFFu - label));
+    __syncthreads();
+    if (i == 0) *giant = 0xFFFFFFFFu - (uint32_t)s_best;
 }
 
 // Links the edges from position `skip` on of every vertex whose component
@@ -829,7 +833,8 @@ __global__ void k_uf_gather(const uint32_t* comp, const uint32_t* idx, uint32_t 
 // Edges of giant-component vertices are covered from their other endpoint.
 template <class OffT, class EdgeT>
 __global__ __launch_bounds__(kBlock) void k_uf_rest(const OffT* off, const EdgeT* edges, uint32_t* comp, uint32_t V,
-                                                    uint32_t giant, uint32_t skip, DevStats* stats) {
+                                                    const uint32_t* giant_p, uint32_t skip, DevStats* stats) {
+    const uint32_t giant = *giant_p;
     __shared__ unsigned long long s_pref[kBlock];
     __shared__ OffT s_beg[kBlock];
     __shared__ unsigned long long s_scan[kWavesPerBlock];
@@ -884,33 +889,12 @@ static int run_cc_uf(asc_graph* g, uint32_t* out, asc_stats* st) {
     const EdgeT* edges = (const EdgeT*)g->d_edges;
     uint32_t* comp = t->val;
 
-    // sampled vertices: a fixed SplitMix64 sequence, so runs are repeatable
-    const uint32_t ns = (uint32_t)std::min<uint64_t>(kSamples, V);
-    uint64_t x = 0x243f6a8885a308d3ull;
-    for (uint32_t i = 0; i < ns; i++) {
-        uint64_t z = (x += 0x9e3779b97f4a7c15ull);
-        z = (z ^ (z >> 30)) * 0xbf58476d1ce4e5b9ull;
-        z = (z ^ (z >> 27)) * 0x94d049bb133111ebull;
-        z ^= z >> 31;
-        t->h_sample[i] = (uint32_t)(z % V);
-    }
-    uint32_t* d_idx = t->heavy_u;              // kHeavyCap >= kSamples * 2 entries of scratch
-    uint32_t* d_lab = t->heavy_u + kSamples;
-    ASC_HIP(hipMemcpyAsync(d_idx, t->h_sample.p, 4 * (size_t)ns, hipMemcpyHostToDevice, s));
-    ASC_HIP(hipMemsetAsync(t->stats, 0, sizeof(DevStats), s));
-    ASC_HIP(hipStreamSynchronize(s));
-
+    uint32_t* d_giant = t->heavy_u;            // scratch
     RunCounters rc{};
     t->timed.clear();
     t->ev_next = 0;
     const double t0 = now_ms();
-    hipEvent_t e0 = nullptr;
-    if (!prof) {
-        e0 = next_event(t);
-        if (!e0) return ASC_ERR_DEVICE;
-        ASC_HIP(hipEventRecord(e0, s));
-    }
-    hipLaunchKernelGGL(k_uf_init, dim3(vgrid), dim3(kBlock), 0, s, comp, (uint32_t)V);
+    hipLaunchKernelGGL(k_uf_init, dim3(vgrid), dim3(kBlock), 0, s, comp, (uint32_t)V, t->stats);
     for (int r = 0; r < kSampleRounds; r++) {
         ASC_TRY(timed_launch(t, prof, KERN_UF, s, [&] {
             hipLaunchKernelGGL((k_uf_sample<OffT, EdgeT>), dim3(vgrid), dim3(kBlock), 0, s, off, edges, comp,
@@ -918,33 +902,17 @@ static int run_cc_uf(asc_graph* g, uint32_t* out, asc_stats* st) {
         }));
         hipLaunchKernelGGL(k_uf_compress, dim3(vgrid), dim3(kBlock), 0, s, comp, (uint32_t)V);
     }
-    hipLaunchKernelGGL(k_uf_gather, dim3((ns + 255) / 256), dim3(256), 0, s, comp, d_idx, ns, d_lab);
-    ASC_HIP(hipGetLastError());
-    ASC_HIP(hipMemcpyAsync(t->h_sample.p, d_lab, 4 * (size_t)ns, hipMemcpyDeviceToHost, s));
-    ASC_HIP(hipStreamSynchronize(s));
-    // most common sampled label (ties: the smallest)
-    std::unordered_map<uint32_t, uint32_t> freq;
-    uint32_t giant = t->h_sample[0], best = 0;
-    for (uint32_t i = 0; i < ns; i++) {
-        const uint32_t c = ++freq[t->h_sample[i]];
-        if (c > best || (c == best && t->h_sample[i] < giant)) {
-            best = c;
-            giant = t->h_sample[i];
-        }
-    }
+    hipLaunchKernelGGL(k_uf_giant, dim3(1), dim3(kSamples), 0, s, comp, V, d_giant);
     ASC_TRY(timed_launch(t, prof, KERN_UF, s, [&] {
         hipLaunchKernelGGL((k_uf_rest<OffT, EdgeT>), dim3(vgrid), dim3(kBlock), 0, s, off, edges, comp, (uint32_t)V,
-                           giant, (uint32_t)kSampleRounds, t->stats);
+                           (const uint32_t*)d_giant, (uint32_t)kSampleRounds, t->stats);
     }));
     hipLaunchKernelGGL(k_uf_compress, dim3(vgrid), dim3(kBlock), 0, s, comp, (uint32_t)V);
+    const unsigned long long want = ++t->pub_seq;
+    hipLaunchKernelGGL(k_do_publish, dim3(1), dim3(64), 0, s, t->dcnt, (const Slot*)nullptr, t->stats, t->d_h->bfs,
+                       want);
     ASC_HIP(hipGetLastError());
-    if (!prof) {
-        hipEvent_t e1 = next_event(t);
-        if (!e1) return ASC_ERR_DEVICE;
-        ASC_HIP(hipEventRecord(e1, s));
-        t->timed.push_back({-1, e0, e1});
-    }
-    ASC_HIP(hipStreamSynchronize(s));
+    ASC_TRY(wait_host_seq(&t->h[0].bfs[1].n_found, want, s));
     const double t1 = now_ms();
     rc.node_sum = V;
     return finish_traversal(g, ALG_CC, PATH_UNION_FIND, out, st, rc, t1 - t0, kSampleRounds + 1);

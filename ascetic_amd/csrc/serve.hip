@@ -727,12 +727,25 @@ __global__ void k_seed(BatchArgs<OffT, EdgeT> a, SeedArgs sa, uint32_t step, uin
     }
 }
 
-// Result column of one BFS lane, unreached (seen bit clear) as V + 1; the
-// level bytes of vertices the lane did not reach may hold an earlier query's.
-__global__ void k_extract_lev(const uint8_t* lev, const unsigned long long* seen, uint64_t V, uint32_t stride,
-                              uint32_t lane, uint32_t* out) {
-    for (uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v < V; v += (uint64_t)gridDim.x * blockDim.x)
-        out[v] = ((seen[v] >> lane) & 1ull) ? (uint32_t)lev[v * stride + lane] : (uint32_t)(V + 1);
+// The lanes whose result columns are being sent: lane of part p.
+struct SendLanes {
+    uint8_t q[kMaxLanes];
+};
+
+// Pieces of BFS lanes' result columns for the host: unreached (seen bit clear)
+// as V + 1, or the zero-based convention; the level bytes of vertices a lane
+// did not reach may hold an earlier query's.
+__global__ __launch_bounds__(kBlock) void k_extract_lev(const uint8_t* lev, const unsigned long long* seen, uint64_t V,
+                                                        uint32_t stride, SendLanes lanes, int zero_based, OutGroup g) {
+    const OutSlot s = out_slot(g);
+    const uint32_t lane = lanes.q[s.part];
+    for (uint32_t i = s.block * kBlock + threadIdx.x; i < s.n; i += s.blocks * kBlock) {
+        const uint64_t v = s.first + i;
+        const bool hit = (seen[v] >> lane) & 1ull;
+        const uint32_t x = hit ? (uint32_t)lev[v * stride + lane] : 0;
+        s.dst[i] = hit ? x - (zero_based ? 1u : 0u) : zero_based ? 0xFFFFFFFFu : (uint32_t)(V + 1);
+    }
+    out_done(s);
 }
 
 __global__ void k_lane_fill(uint32_t* p, uint64_t n, uint32_t v) {
@@ -740,16 +753,22 @@ __global__ void k_lane_fill(uint32_t* p, uint64_t n, uint32_t v) {
         p[i] = v;
 }
 
-// Result column of one lane, unreached as V + 1.  The lanes relax without the
-// reference's cap: there a value starts at V + 1 and only a smaller candidate
-// lowers it (GraphMeta.cuh:440-446, gpu_kernels.cuh:499), so a vertex whose
-// distance + 1 reaches V + 1 keeps V + 1.  With non-negative weights that
-// schedule ends at min(exact value, V + 1), which is applied here.
-__global__ void k_extract_lane(const uint16_t* dist, uint64_t V, uint32_t stride, uint32_t lane, uint32_t* out) {
-    for (uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v < V; v += (uint64_t)gridDim.x * blockDim.x) {
-        const uint32_t d = dist[v * stride + lane];
-        out[v] = d == kD16Inf || (uint64_t)d > V ? (uint32_t)(V + 1) : d;
+// Pieces of SSSP lanes' result columns, unreached as V + 1 (or the zero-based
+// convention).  The lanes relax without the reference's cap: there a value
+// starts at V + 1 and only a smaller candidate lowers it (GraphMeta.cuh:440-446,
+// gpu_kernels.cuh:499), so a vertex whose distance + 1 reaches V + 1 keeps
+// V + 1.  With non-negative weights that schedule ends at min(exact value,
+// V + 1), which is applied here.
+__global__ __launch_bounds__(kBlock) void k_extract_lane(const uint16_t* dist, uint64_t V, uint32_t stride,
+                                                         SendLanes lanes, int zero_based, OutGroup g) {
+    const OutSlot s = out_slot(g);
+    const uint32_t lane = lanes.q[s.part];
+    for (uint32_t i = s.block * kBlock + threadIdx.x; i < s.n; i += s.blocks * kBlock) {
+        const uint32_t d = dist[(s.first + i) * stride + lane];
+        const bool hit = d != kD16Inf && (uint64_t)d <= V;
+        s.dst[i] = hit ? d - (zero_based ? 1u : 0u) : zero_based ? 0xFFFFFFFFu : (uint32_t)(V + 1);
     }
+    out_done(s);
 }
 
 // -- host -----------------------------------------------------------------------
@@ -782,7 +801,7 @@ struct Engine {
     unsigned long long* heavy_bits = nullptr;
     unsigned long long* heavy_base = nullptr;
     uint32_t* s0 = nullptr;
-    uint32_t* staging = nullptr;      // SSSP result column
+    OutStage out;                     // result columns on their way to the host
     HostBuf<Slot> h_slot;
     SQuery* lane_q[kMaxLanes] = {};
     unsigned long long busy = 0;
@@ -842,7 +861,7 @@ static void engine_free(Engine& e) {
         x = nullptr;
     }
     f(e.bits[0]); f(e.bits[1]); f(e.seen); f(e.lanes_state); f(e.q[0]); f(e.q[1]); f(e.slots);
-    f(e.heavy_u); f(e.heavy_bits); f(e.heavy_base); f(e.s0); f(e.staging); f(e.d_cnt); f(e.d_ovf); f(e.d_sp);
+    f(e.heavy_u); f(e.heavy_bits); f(e.heavy_base); f(e.s0); f(e.d_cnt); f(e.d_ovf); f(e.d_sp);
     if (e.stream) (void)hipStreamDestroy(e.stream);
     e.stream = nullptr;
 }
@@ -862,7 +881,6 @@ static int engine_init(Engine& e, int kind, int lanes, uint64_t V) {
         ASC_HIP(hipMalloc(&e.seen, 8 * V));
         ASC_HIP(hipMemsetAsync(e.seen, 0, 8 * V, e.stream));
     }
-    ASC_HIP(hipMalloc(&e.staging, 4 * V));
     // rows of whole 16-byte units: 16 lanes for the u8 BFS levels, 8 for the u16 SSSP distances
     e.stride = kind == ASC_QUERY_BFS ? (uint32_t)((lanes + 15) / 16 * 16) : (uint32_t)((lanes + 7) / 8 * 8);
     hipError_t r = hipMalloc(&e.lanes_state, (kind == ASC_QUERY_SSSP ? 2 : 1) * V * (size_t)e.stride);
@@ -1067,36 +1085,39 @@ static int engine_finish(asc_server* s, Engine& e, std::vector<SQuery*>& done) {
             e.mu[q] = e.mu[q] > e.mf[q] ? e.mu[q] - e.mf[q] : 0;
         }
     }
-    const bool zero_based = s->g->ctx->cfg.value_convention == ASC_VALUES_ZERO_BASED;
-    const uint32_t unreached = (uint32_t)(e.V + 1);
+    const int zero_based = s->g->ctx->cfg.value_convention == ASC_VALUES_ZERO_BASED ? 1 : 0;
+    // the result columns of all lanes that finished, sent together
+    uint32_t* parts[kMaxLanes];
+    SendLanes lanes{};
+    uint32_t n_parts = 0;
     for (int q = 0; q < e.lanes; q++) {
         SQuery* qq = e.lane_q[q];
         if (!qq) continue;
         qq->steps++;
-        if (act & (1ull << q)) continue;
-        const bool overflowed = (e.h_ovf[0] >> q) & 1ull;
-        if (qq->out && overflowed) {
+        if ((act & (1ull << q)) || !qq->out) continue;
+        if ((e.h_ovf[0] >> q) & 1ull) {
             // a level left 8 bits / a distance left 16 bits: the single-query
             // engine answers exactly (value convention applied there)
             ASC_TRY(traverse(s->g, e.kind == ASC_QUERY_SSSP ? ALG_SSSP : ALG_BFS, qq->src, qq->out, nullptr));
             s->fallbacks++;
-        } else if (qq->out) {
-            const int grid = s->g->ctx->num_cus * 4;
-            if (e.kind == ASC_QUERY_BFS)
-                hipLaunchKernelGGL(k_extract_lev, dim3(grid), dim3(256), 0, e.stream, (const uint8_t*)e.lanes_state,
-                                   (const unsigned long long*)e.seen, e.V, e.stride, (uint32_t)q, e.staging);
-            else
-                hipLaunchKernelGGL(k_extract_lane, dim3(grid), dim3(256), 0, e.stream,
-                                   (const uint16_t*)e.lanes_state, e.V, e.stride, (uint32_t)q, e.staging);
-            ASC_HIP(hipMemcpyAsync(qq->out, e.staging, 4 * e.V, hipMemcpyDeviceToHost, e.stream));
-            ASC_HIP(hipStreamSynchronize(e.stream));
-            if (zero_based) {
-                uint32_t* o = qq->out;
-                host_pool().parallel_for(e.V, [&](uint64_t b, uint64_t en) {
-                    for (uint64_t v = b; v < en; v++) o[v] = o[v] == unreached ? 0xFFFFFFFFu : o[v] - 1;
-                });
-            }
+        } else {
+            lanes.q[n_parts] = (uint8_t)q;
+            parts[n_parts++] = qq->out;
         }
+    }
+    ASC_TRY(out_send(e.out, parts, n_parts, e.V, e.stream, [&](const OutGroup& og, int blocks) -> int {
+        if (e.kind == ASC_QUERY_BFS)
+            hipLaunchKernelGGL(k_extract_lev, dim3(blocks), dim3(kBlock), 0, e.stream, (const uint8_t*)e.lanes_state,
+                               (const unsigned long long*)e.seen, e.V, e.stride, lanes, zero_based, og);
+        else
+            hipLaunchKernelGGL(k_extract_lane, dim3(blocks), dim3(kBlock), 0, e.stream, (const uint16_t*)e.lanes_state,
+                               e.V, e.stride, lanes, zero_based, og);
+        ASC_HIP(hipGetLastError());
+        return ASC_OK;
+    }));
+    for (int q = 0; q < e.lanes; q++) {
+        SQuery* qq = e.lane_q[q];
+        if (!qq || (act & (1ull << q))) continue;
         qq->t_done = now_ms();
         e.lane_q[q] = nullptr;
         e.busy &= ~(1ull << q);

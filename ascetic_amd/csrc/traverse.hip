@@ -417,10 +417,14 @@ __global__ void k_set_u32(uint32_t* p, uint32_t v) { *p = v; }
 
 // Publishes a level's counters (the next step's slot and the piles, and the
 // edges of a small frontier) to mapped host memory, then the sequence number
-// the host polls for.  One workgroup.
+// the host polls for; the far pile not in use and min_far are reset for the
+// next split.  With `split`, that slot is this step's own frontier, filled by
+// a split ahead of it.  One workgroup.
 template <class OffT>
-__global__ __launch_bounds__(kBlock) void k_trav_publish(const Slot* slot, const Piles* piles, const OffT* off,
-                                                         const uint32_t* q, LevelPub* host, unsigned long long seq) {
+__global__ __launch_bounds__(kBlock) void k_trav_publish(const Slot* slot, const Slot* split, Piles* piles,
+                                                         uint32_t far_other, DevStats* stats, int timed,
+                                                         const OffT* off, const uint32_t* q, LevelPub* host,
+                                                         unsigned long long seq) {
     __shared__ unsigned long long s_m[kWavesPerBlock];
     const uint32_t n = slot->n_res;
     unsigned long long m = 0;
@@ -435,11 +439,14 @@ __global__ __launch_bounds__(kBlock) void k_trav_publish(const Slot* slot, const
     if (threadIdx.x != 0) return;
     m = 0;
     for (int i = 0; i < kWavesPerBlock; i++) m += s_m[i];
-    host->slot = *slot;
-    host->piles = *piles;
-    host->edges = n <= kNarrowCap ? m : ~0ull;
-    __threadfence_system();
-    host->seq = seq;
+    host_store_words(&host->slot, *slot);
+    host_store_words(&host->piles, *piles);
+    host_store(&host->n_split, (unsigned long long)(split ? split->n_res : 0));
+    host_store(&host->edges, n <= kNarrowCap ? m : ~0ull);
+    host_publish(&host->seq, seq);
+    piles->n_far[far_other] = 0;
+    piles->min_far = 0xFFFFFFFFu;
+    if (timed) stats->ticks += wall_clock64() - stats->t_begin;
 }
 
 __global__ void k_fill_u32(uint32_t* p, uint64_t n, uint32_t v) {
@@ -447,24 +454,49 @@ __global__ void k_fill_u32(uint32_t* p, uint64_t n, uint32_t v) {
         p[i] = v;
 }
 
-// Step-0 frontier for BFS / SSSP: the source alone (GraphMeta.cuh:432-446).
-__global__ void k_init_source(uint32_t* val, uint32_t* visited, uint32_t* pstamp, uint32_t* q, uint32_t* pend,
-                              Slot* slots, Piles* piles, uint32_t src, uint32_t vs) {
-    val[src] = 1;
-    if (visited) visited[src >> 5] |= 1u << (src & 31);
-    if (src < vs) {
-        q[0] = src;
-        slots[0].n_res = 1;
-    } else {
-        pend[0] = src;
-        piles->n_pend[0] = 1;
-        if (pstamp) pstamp[src] = 1;
+// Start of a run in one launch: every array at its initial value, the step-0
+// frontier of BFS / SSSP the source alone (GraphMeta.cuh:432-446).
+__global__ __launch_bounds__(kBlock) void k_run_init(RunInit a) {
+    const uint64_t i0 = blockIdx.x * (uint64_t)kBlock + threadIdx.x, step = (uint64_t)gridDim.x * kBlock;
+    if (a.val)
+        for (uint64_t i = i0; i < a.V; i += step) a.val[i] = i == a.src ? 1u : a.unreached;
+    for (uint32_t* z : {a.stamp, a.pstamp, a.fstamp})
+        if (z)
+            for (uint64_t i = i0; i < a.V; i += step) z[i] = 0;
+    if (a.done)
+        for (uint64_t i = i0; i < a.V; i += step) a.done[i] = kNoValue;
+    if (a.visited)
+        for (uint64_t i = i0; i < (a.V + 31) / 32; i += step) a.visited[i] = i == a.src >> 5 ? 1u << (a.src & 31) : 0u;
+    if (a.val16)
+        for (uint64_t i = i0; i < (a.V + 1) / 2; i += step) a.val16[i] = 0xFFFFFFFFu;
+    if (blockIdx.x != 0) return;
+    uint32_t* st = (uint32_t*)a.stats;
+    for (uint32_t i = threadIdx.x; i < sizeof(DevStats) / 4; i += kBlock) st[i] = 0;
+    if (threadIdx.x < 4) {
+        Slot z{};
+        if (threadIdx.x == 0) z.n_res = a.n_res0;
+        a.slots[threadIdx.x] = z;
     }
+    if (threadIdx.x == 4) {
+        Piles z{};
+        z.n_pend[0] = a.n_pend0;
+        z.min_far = 0xFFFFFFFFu;
+        *a.piles = z;
+    }
+    if (threadIdx.x == 5 && a.dcnt) *a.dcnt = DoCounters{};
+    if (threadIdx.x == 6 && a.q0 && a.n_res0) a.q0[0] = a.src;
+    if (threadIdx.x == 7 && a.pend0 && a.n_pend0) a.pend0[0] = a.src;
+}
+
+int launch_run_init(const RunInit& a, int num_cus, hipStream_t s) {
+    const int grid = (int)std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)num_cus * 8, (a.V + kBlock - 1) / kBlock));
+    hipLaunchKernelGGL(k_run_init, dim3(grid), dim3(kBlock), 0, s, a);
+    ASC_HIP(hipGetLastError());
+    return ASC_OK;
 }
 
 // CC: every vertex starts with its own id and active (GraphMeta.cuh:448-452).
-__global__ void k_init_cc(uint32_t* val, uint32_t* pstamp, uint32_t* q, uint32_t* pend, Slot* slots, Piles* piles,
-                          uint32_t V, uint32_t vs) {
+__global__ void k_init_cc(uint32_t* val, uint32_t* pstamp, uint32_t* q, uint32_t* pend, uint32_t V, uint32_t vs) {
     for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x; v < V; v += gridDim.x * blockDim.x) {
         val[v] = v;
         if (v < vs) {
@@ -474,10 +506,71 @@ __global__ void k_init_cc(uint32_t* val, uint32_t* pstamp, uint32_t* q, uint32_t
             pstamp[v] = 1;
         }
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        slots[0].n_res = vs;
-        piles->n_pend[0] = V - vs;
+}
+
+// Pieces of the run's values for the host: value convention applied, and
+// (BFS, SSSP: `off` given) the reached vertices and their degrees added up.
+template <class OffT>
+__global__ __launch_bounds__(kBlock) void k_finish_values(const uint32_t* val, const OffT* off, uint32_t unreached,
+                                                          int zero_based, unsigned long long* reach, OutGroup g) {
+    __shared__ unsigned long long s_r[kWavesPerBlock], s_d[kWavesPerBlock];
+    const OutSlot s = out_slot(g);
+    unsigned long long r = 0, d = 0;
+    auto one = [&](uint64_t v, uint32_t x) {
+        const bool hit = x != unreached;
+        if (off) {
+            const unsigned long long deg = (unsigned long long)(off[v + 1] - off[v]);
+            r += hit;
+            d += hit ? deg : 0;
+        }
+        return zero_based ? (hit ? x - 1 : 0xFFFFFFFFu) : x;
+    };
+    const uint32_t n4 = s.n / 4, i0 = s.block * kBlock + threadIdx.x, step = s.blocks * kBlock;
+    const uint4* in = (const uint4*)(val + s.first);   // pieces start at multiples of 128 KiB
+    for (uint32_t i = i0; i < n4; i += step) {
+        uint4 x = in[i];
+        const uint64_t v = s.first + 4 * i;
+        x.x = one(v, x.x);
+        x.y = one(v + 1, x.y);
+        x.z = one(v + 2, x.z);
+        x.w = one(v + 3, x.w);
+        ((uint4*)s.dst)[i] = x;
     }
+    for (uint32_t i = 4 * n4 + i0; i < s.n; i += step) s.dst[i] = one(s.first + i, val[s.first + i]);
+    if (off) {
+        r = wave_sum(r);
+        d = wave_sum(d);
+        if (lane_id() == 0) {
+            s_r[wave_id()] = r;
+            s_d[wave_id()] = d;
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            r = d = 0;
+            for (int i = 0; i < kWavesPerBlock; i++) {
+                r += s_r[i];
+                d += s_d[i];
+            }
+            if (r) {
+                atomicAdd(reach, r);
+                atomicAdd(reach + 1, d);
+            }
+        }
+    }
+    out_done(s);
+}
+
+// Behind the last values: the statistics of the run, and the counts above
+// (cleared for the next run).  One lane.
+__global__ void k_finish_stats(const DevStats* stats, unsigned long long* reach, FinishPub* pub,
+                               unsigned long long seq) {
+    if (threadIdx.x != 0) return;
+    host_store_words(&pub->stats, *stats);
+    host_store(&pub->reached, reach[0]);
+    host_store(&pub->degree_sum, reach[1]);
+    reach[0] = 0;
+    reach[1] = 0;
+    host_publish(&pub->seq, seq);
 }
 
 // ---------------------------------------------------------------------------
@@ -489,14 +582,10 @@ void trav_free(TravState* t) {
     auto f = [](void* p) {
         if (p) (void)hipFree(p);
     };
-    f(t->val); f(t->val16); f(t->stamp); f(t->pstamp); f(t->fstamp); f(t->done); f(t->visited);
-    for (int i = 0; i < 2; i++) {
-        f(t->q[i]); f(t->pend[i]); f(t->far[i]);
-    }
+    f(t->val16);
+    for (int i = 0; i < 2; i++) f(t->pend[i]);
     for (int i = 0; i < kMaxPartBufs; i++) f(t->part[i]);
-    f(t->heavy_u); f(t->heavy_sv); f(t->heavy_base);
-    f(t->od_list); f(t->od_prefix); f(t->scan_tmp); f(t->slots); f(t->piles); f(t->stats);
-    f(t->bm[0]); f(t->bm[1]); f(t->bm[2]); f(t->pctl); f(t->dcnt); f(t->d_ch_v); f(t->d_ch_edges); f(t->d_ch_count); f(t->d_ch_dense);
+    f(t->od_list); f(t->od_prefix); f(t->scan_tmp); f(t->d_ch_v); f(t->d_ch_edges); f(t->d_ch_count); f(t->d_ch_dense);
     f(t->d_cursor);
     for (int i = 0; i < kMaxPartBufs; i++) {
         if (t->ev_copy[i]) (void)hipEventDestroy(t->ev_copy[i]);
@@ -570,29 +659,24 @@ int trav_ensure(asc_graph* g) {
     if (t) trav_free(t);
     t = new TravState();
     g->trav = t;
-    t->V = V;
     ASC_HIP(hipSetDevice(g->ctx->device));
-    for (uint32_t** p : {&t->val, &t->stamp, &t->pstamp, &t->fstamp, &t->done, &t->far[0], &t->far[1]})
-        ASC_HIP(hipMalloc(p, 4 * V));
+    t->mem.add(&t->val, V);
     // a narrow step may list a vertex more than once
     for (uint32_t** p : {&t->q[0], &t->q[1]})
-        ASC_HIP(hipMalloc(p, 4 * std::max<uint64_t>(V, std::max(kNarrowEdges, kNarrowFar))));
-    ASC_HIP(hipMalloc(&t->visited, 4 * ((V + 31) / 32)));
-    ASC_HIP(hipMalloc(&t->heavy_u, 4 * (size_t)kHeavyCap));
-    ASC_HIP(hipMalloc(&t->heavy_sv, 4 * (size_t)kHeavyCap));
-    ASC_HIP(hipMalloc(&t->heavy_base, 8 * (size_t)kHeavyCap));
-    ASC_HIP(hipMalloc(&t->slots, sizeof(Slot) * 4));
-    ASC_HIP(hipMalloc(&t->piles, sizeof(Piles)));
-    ASC_HIP(hipMalloc(&t->stats, sizeof(DevStats)));
-    ASC_TRY(t->h_slot.alloc(4, true));
-    ASC_TRY(t->h_piles.alloc(1, true));
-    ASC_TRY(t->h_pub.alloc(1, true));
-    t->h_pub[0].seq = 0;
-    ASC_HIP(hipHostGetDevicePointer((void**)&t->d_pub, t->h_pub.p, 0));
-    ASC_TRY(t->h_narrow.alloc(1, true));
-    t->h_narrow[0].seq = 0;
-    ASC_HIP(hipHostGetDevicePointer((void**)&t->d_narrow, t->h_narrow.p, 0));
-    ASC_TRY(t->h_stats.alloc(1, true));
+        t->mem.add(p, std::max<uint64_t>(V, std::max(kNarrowEdges, kNarrowFar)));
+    t->mem.add(&t->visited, (V + 31) / 32);
+    t->mem.add(&t->heavy_u, kHeavyCap);
+    t->mem.add(&t->heavy_sv, kHeavyCap);
+    t->mem.add(&t->heavy_base, kHeavyCap);
+    t->mem.add(&t->slots, 4);
+    t->mem.add(&t->piles, 1);
+    t->mem.add(&t->stats, 1);
+    t->mem.add(&t->d_reach, 2);
+    ASC_TRY(t->mem.alloc());
+    ASC_HIP(hipMemsetAsync(t->d_reach, 0, 16, g->ctx->s_main));
+    ASC_TRY(t->h.alloc(1, true));
+    std::memset((void*)t->h.p, 0, sizeof(HostPubs));
+    ASC_HIP(hipHostGetDevicePointer((void**)&t->d_h, t->h.p, 0));
     if (need_parts) {
         const uint64_t nod = V - g->static_vertices;
         ASC_HIP(hipMalloc(&t->pend[0], 4 * nod));
@@ -626,7 +710,20 @@ int trav_ensure(asc_graph* g) {
         ASC_HIP(hipEventCreateWithFlags(&t->ev_meta, hipEventDisableTiming));
         ASC_TRY(plan_dense_chunks(g, t));
     }
+    t->V = V;   // last: a state that could not be set up whole is set up again
     return ASC_OK;
+}
+
+int trav_ensure_relax(asc_graph* g) {
+    ASC_TRY(trav_ensure(g));
+    TravState* t = g->trav;
+    if (t->mem_relax.p) return ASC_OK;
+    const uint64_t V = g->h.V;
+    t->mem_relax.parts.clear();
+    t->mem_relax.bytes = 0;
+    for (uint32_t** p : {&t->stamp, &t->pstamp, &t->fstamp, &t->done, &t->far[0], &t->far[1]})
+        t->mem_relax.add(p, V);
+    return t->mem_relax.alloc();
 }
 
 static hipEvent_t pooled_event(TravState* t, size_t i) {
@@ -965,9 +1062,9 @@ static int stream_pile(asc_graph* g, TravArgs<OffT, EdgeT>& a, uint32_t& level, 
         hipLaunchKernelGGL((k_filter_pile<ALGO, OffT>), dim3(pile_grid), dim3(kBlock), 0, s, a.off, pile, npile,
                            a.val, a.done, t->od_list, list_deg, &t->piles->n_list);
         ASC_HIP(hipGetLastError());
-        ASC_HIP(hipMemcpyAsync(t->h_piles.p, t->piles, sizeof(Piles), hipMemcpyDeviceToHost, s));
+        ASC_HIP(hipMemcpyAsync(&t->h[0].piles, t->piles, sizeof(Piles), hipMemcpyDeviceToHost, s));
         ASC_HIP(hipStreamSynchronize(s));
-        m = t->h_piles[0].n_list;
+        m = t->h[0].piles.n_list;
         n_sparse = m;
         if (m) {
             ASC_TRY(scan_degrees(t, list_deg, m, s));
@@ -1209,12 +1306,12 @@ static int stream_pile(asc_graph* g, TravArgs<OffT, EdgeT>& a, uint32_t& level, 
 template <int ALGO, class OffT, class EdgeT>
 static int run_traversal(asc_graph* g, uint32_t src, uint32_t* out, asc_stats* st) {
     asc_ctx* ctx = g->ctx;
-    ASC_TRY(trav_ensure(g));
+    ASC_HIP(hipSetDevice(ctx->device));
+    ASC_TRY(ALGO == ALG_BFS ? trav_ensure(g) : trav_ensure_relax(g));
     TravState* t = g->trav;
     const uint64_t V = g->h.V;
     const uint32_t vs = (uint32_t)g->static_vertices;
     hipStream_t s = ctx->s_main;
-    ASC_HIP(hipSetDevice(ctx->device));
     const int fill_grid = ctx->num_cus * 4;
     const int grid = ctx->num_cus * (g->blocks_per_cu > 0 ? g->blocks_per_cu : kBlocksPerCU);
     const bool prof = ctx->cfg.profile != 0;
@@ -1222,37 +1319,44 @@ static int run_traversal(asc_graph* g, uint32_t src, uint32_t* out, asc_stats* s
     const bool use16 = ALGO == ALG_SSSP && vs == V && sssp_filter_pays(g);
 
     // initial state
-    ASC_HIP(hipMemsetAsync(t->slots, 0, sizeof(Slot) * 4, s));
-    ASC_HIP(hipMemsetAsync(t->piles, 0, sizeof(Piles), s));
-    ASC_HIP(hipMemsetAsync(t->stats, 0, sizeof(DevStats), s));
-    if (ALGO == ALG_BFS) {
-        hipLaunchKernelGGL(k_fill_u32, dim3(fill_grid), dim3(256), 0, s, t->val, V, (uint32_t)(V + 1));
-        hipLaunchKernelGGL(k_fill_u32, dim3(fill_grid), dim3(256), 0, s, t->visited, (V + 31) / 32, 0u);
-        hipLaunchKernelGGL(k_init_source, dim3(1), dim3(1), 0, s, t->val, t->visited, (uint32_t*)nullptr, t->q[0],
-                           t->pend[0], t->slots, t->piles, src, vs);
+    if (use16 && !t->val16) ASC_HIP(hipMalloc(&t->val16, 4 * ((V + 1) / 2)));
+    RunInit ri{};
+    ri.V = V;
+    ri.slots = t->slots;
+    ri.piles = t->piles;
+    ri.stats = t->stats;
+    ri.src = src;
+    ri.unreached = (uint32_t)(V + 1);
+    if (ALGO == ALG_CC) {
+        ri.n_res0 = vs;
+        ri.n_pend0 = (uint32_t)(V - vs);
     } else {
-        for (uint32_t* p : {t->stamp, t->pstamp, t->fstamp})
-            hipLaunchKernelGGL(k_fill_u32, dim3(fill_grid), dim3(256), 0, s, p, V, 0u);
-        hipLaunchKernelGGL(k_fill_u32, dim3(fill_grid), dim3(256), 0, s, t->done, V, kNoValue);
-        if (ALGO == ALG_CC) {
-            hipLaunchKernelGGL(k_init_cc, dim3(fill_grid), dim3(256), 0, s, t->val, t->pstamp, t->q[0], t->pend[0],
-                               t->slots, t->piles, (uint32_t)V, vs);
-        } else {
-            hipLaunchKernelGGL(k_fill_u32, dim3(fill_grid), dim3(256), 0, s, t->val, V, (uint32_t)(V + 1));
-            if (use16) {
-                // the value filter serves fully resident graphs (narrow bands:
-                // few improvements per vertex); with on-demand edges (wide
-                // bands, more stores to it) it measured slower
-                if (!t->val16) ASC_HIP(hipMalloc(&t->val16, 4 * ((V + 1) / 2)));
-                hipLaunchKernelGGL(k_fill_u32, dim3(fill_grid), dim3(256), 0, s, (uint32_t*)t->val16, (V + 1) / 2,
-                                   0xFFFFFFFFu);
-            }
-            hipLaunchKernelGGL(k_init_source, dim3(1), dim3(1), 0, s, t->val, (uint32_t*)nullptr, t->pstamp, t->q[0],
-                               t->pend[0], t->slots, t->piles, src, vs);
-        }
+        ri.val = t->val;
+        ri.q0 = t->q[0];
+        ri.pend0 = t->pend[0];
+        ri.n_res0 = src < vs ? 1 : 0;
+        ri.n_pend0 = src < vs ? 0 : 1;
+    }
+    if (ALGO == ALG_BFS) {
+        ri.visited = t->visited;
+    } else {
+        ri.stamp = t->stamp;
+        ri.pstamp = vs < V ? t->pstamp : nullptr;   // on-demand vertices only
+        ri.fstamp = ALGO == ALG_SSSP ? t->fstamp : nullptr;
+        ri.done = t->done;
+    }
+    // the value filter serves fully resident graphs (narrow bands: few
+    // improvements per vertex); with on-demand edges (wide bands, more stores
+    // to it) it measured slower
+    if (use16) ri.val16 = (uint32_t*)t->val16;
+    ASC_TRY(launch_run_init(ri, ctx->num_cus, s));
+    if (ALGO == ALG_CC) {
+        hipLaunchKernelGGL(k_init_cc, dim3(fill_grid), dim3(256), 0, s, t->val, t->pstamp, t->q[0], t->pend[0],
+                           (uint32_t)V, vs);
+    } else if (src >= vs && ALGO == ALG_SSSP) {
+        hipLaunchKernelGGL(k_set_u32, dim3(1), dim3(1), 0, s, t->pstamp + src, 1u);
     }
     ASC_HIP(hipGetLastError());
-    ASC_HIP(hipStreamSynchronize(s));
 
     TravArgs<OffT, EdgeT> a{};
     a.off = (const OffT*)g->d_off;
@@ -1292,11 +1396,12 @@ static int run_traversal(asc_graph* g, uint32_t src, uint32_t* out, asc_stats* s
     if (g->static_vertices < V && t->part[0]) ASC_TRY(prefetch_chunks(g, t));
     uint32_t level = 0;
     bool last_split_empty = false;
+    const bool resident = vs == V;
     // edges of the frontier where known (the source, a small published one)
     uint64_t nedges = ALGO == ALG_CC ? g->h.E : g->h.off[src + 1] - g->h.off[src];
     for (;;) {
         // small steps of a resident graph run back to back in one workgroup
-        if (vs == V && ((nr > 0 && nr <= kNarrowCap && nedges <= kNarrowEdges) ||
+        if (resident && ((nr > 0 && nr <= kNarrowCap && nedges <= kNarrowEdges) ||
                         (nr == 0 && nfar > 0 && nfar <= kNarrowFar && delta))) {
             NarrowState io;
             io.level = level;
@@ -1343,27 +1448,30 @@ static int run_traversal(asc_graph* g, uint32_t src, uint32_t* out, asc_stats* s
         a.far_count = &t->piles->n_far[fcur];
         if (mode == M_SPLIT) {
             // advance the band; entries still beyond it move to the other far pile
-            const uint64_t th = (uint64_t)(last_split_empty ? std::max(a.theta, t->h_piles[0].min_far) : a.theta) + delta;
+            const uint64_t th = (uint64_t)(last_split_empty ? std::max(a.theta, t->h[0].piles.min_far) : a.theta) + delta;
             a.theta = (uint32_t)std::min<uint64_t>(th, 0xFFFFFFFFull);
             const uint32_t old = fcur;
             fcur ^= 1;
             a.far_out = t->far[fcur];
-            a.far_count = &t->piles->n_far[fcur];
-            hipLaunchKernelGGL(k_set_u32, dim3(1), dim3(1), 0, s, &t->piles->n_far[fcur], 0u);
-            hipLaunchKernelGGL(k_set_u32, dim3(1), dim3(1), 0, s, &t->piles->min_far, 0xFFFFFFFFu);
+            a.far_count = &t->piles->n_far[fcur];   // zero: the last publish cleared it
             hipLaunchKernelGGL((k_split_far<OffT, EdgeT>),
                                dim3(std::min<uint32_t>((nfar + kBlock - 1) / kBlock, (uint32_t)grid)), dim3(kBlock), 0,
                                s, a, t->far[old], nfar, level, t->q[level & 1], t->piles);
             ASC_HIP(hipGetLastError());
             rc.splits++;
-        } else {
+            nr = nfar;   // at most; a resident graph expands what the split leaves at once
+        }
+        const bool expand = mode != M_SPLIT || resident;
+        if (expand) {
             // one step: expand the resident frontier (possibly empty), then
             // stream the pile
-            rc.node_sum += nr;
+            if (mode != M_SPLIT) rc.node_sum += nr;
             a.q_in = t->q[level & 1];
             a.q_out = t->q[(level + 1) & 1];
+            // streamed runs time the resident kernels by events, resident ones
+            // by the device's clock (an event costs a few us of each step)
             hipEvent_t e0 = nullptr;
-            if (!prof) {
+            if (!prof && !resident) {
                 e0 = next_event(t);
                 if (!e0) return ASC_ERR_DEVICE;
                 ASC_HIP(hipEventRecord(e0, s));
@@ -1373,12 +1481,12 @@ static int run_traversal(asc_graph* g, uint32_t src, uint32_t* out, asc_stats* s
             ASC_TRY(timed_launch(t, prof, KERN_LOCAL, s, [&] {
                 hipLaunchKernelGGL((k_expand_local<ALGO, OffT, EdgeT>), dim3(lgrid), dim3(kBlock), 0, s, a, level);
             }));
-            if (nr) {
+            if (nr && g->max_degree >= a.heavy_thr) {
                 ASC_TRY(timed_launch(t, prof, KERN_HEAVY, s, [&] {
                     hipLaunchKernelGGL((k_expand_heavy<ALGO, OffT, EdgeT>), dim3(grid), dim3(kBlock), 0, s, a, level);
                 }));
             }
-            if (!prof) {
+            if (!prof && !resident) {
                 hipEvent_t e1 = next_event(t);
                 if (!e1) return ASC_ERR_DEVICE;
                 ASC_HIP(hipEventRecord(e1, s));
@@ -1388,12 +1496,14 @@ static int run_traversal(asc_graph* g, uint32_t src, uint32_t* out, asc_stats* s
             level++;
         }
         const unsigned long long want = ++t->lvl_seq;
-        hipLaunchKernelGGL((k_trav_publish<OffT>), dim3(1), dim3(kBlock), 0, s, t->slots + (level & 3), t->piles, a.off,
-                           (const uint32_t*)t->q[level & 1], t->d_pub, want);
+        hipLaunchKernelGGL((k_trav_publish<OffT>), dim3(1), dim3(kBlock), 0, s, t->slots + (level & 3),
+                           mode == M_SPLIT && resident ? (const Slot*)(t->slots + ((level - 1) & 3)) : (const Slot*)nullptr,
+                           t->piles, fcur ^ 1u, t->stats, resident && expand ? 1 : 0, a.off,
+                           (const uint32_t*)t->q[level & 1], &t->d_h->level, want);
         ASC_HIP(hipGetLastError());
-        ASC_TRY(wait_host_seq(&t->h_pub.p->seq, want, s));
+        ASC_TRY(wait_host_seq(&t->h[0].level.seq, want, s));
         {
-            const volatile LevelPub* pb = t->h_pub.p;
+            const volatile LevelPub* pb = &t->h[0].level;
             nr = pb->slot.n_res;
             nedges = pb->edges;
             Piles pl;
@@ -1404,11 +1514,13 @@ static int run_traversal(asc_graph* g, uint32_t src, uint32_t* out, asc_stats* s
             pl.n_list = pb->piles.n_list;
             pl.min_far = pb->piles.min_far;
             pl.pad[0] = pl.pad[1] = 0;
-            t->h_piles[0] = pl;   // min_far is read when the band advances
+            t->h[0].piles = pl;   // min_far is read when the band advances
         }
-        npend = t->h_piles[0].n_pend[pcur];
-        nfar = ALGO == ALG_SSSP ? t->h_piles[0].n_far[fcur] : 0;
-        last_split_empty = mode == M_SPLIT && nr == 0 && npend == 0;
+        npend = t->h[0].piles.n_pend[pcur];
+        nfar = ALGO == ALG_SSSP ? t->h[0].piles.n_far[fcur] : 0;
+        if (mode == M_SPLIT && resident) rc.node_sum += ((const volatile LevelPub*)&t->h[0].level)->n_split;
+        last_split_empty = mode == M_SPLIT && nr == 0 && npend == 0 &&
+                           (!resident || ((const volatile LevelPub*)&t->h[0].level)->n_split == 0);
     }
     const double t1 = now_ms();
     return finish_traversal(g, ALGO, PATH_FRONTIER, out, st, rc, t1 - t0, level);
@@ -1436,8 +1548,36 @@ int finish_traversal(asc_graph* g, int algo, int path, uint32_t* out, asc_stats*
     if (prof)
         static_ms = kern[KERN_LOCAL].ms + kern[KERN_HEAVY].ms + kern[KERN_BU].ms + kern[KERN_UF].ms +
                     kern[KERN_PERSIST].ms;
-    ASC_HIP(hipMemcpy(t->h_stats.p, t->stats, sizeof(DevStats), hipMemcpyDeviceToHost));
-    const DevStats& ds = t->h_stats[0];
+    // the values go out in pieces, the statistics behind the last of them
+    DevStats ds{};
+    const bool count = algo != ALG_CC;
+    const bool zero_based = count && ctx->cfg.value_convention == ASC_VALUES_ZERO_BASED;
+    const unsigned long long want = ++t->finish_seq;
+    auto send_stats = [&]() -> int {
+        hipLaunchKernelGGL(k_finish_stats, dim3(1), dim3(kWave), 0, ctx->s_main, t->stats, t->d_reach, &t->d_h->finish,
+                           want);
+        ASC_HIP(hipGetLastError());
+        return ASC_OK;
+    };
+    if (out) {
+        ASC_TRY(out_send(t->out, &out, 1, V, ctx->s_main, [&](const OutGroup& og, int blocks) -> int {
+            if (g->off_bytes == 4)
+                hipLaunchKernelGGL((k_finish_values<uint32_t>), dim3(blocks), dim3(kBlock), 0, ctx->s_main, t->val,
+                                   count ? (const uint32_t*)g->d_off : nullptr, (uint32_t)(V + 1), zero_based ? 1 : 0,
+                                   t->d_reach, og);
+            else
+                hipLaunchKernelGGL((k_finish_values<uint64_t>), dim3(blocks), dim3(kBlock), 0, ctx->s_main, t->val,
+                                   count ? (const uint64_t*)g->d_off : nullptr, (uint32_t)(V + 1), zero_based ? 1 : 0,
+                                   t->d_reach, og);
+            ASC_HIP(hipGetLastError());
+            return (uint64_t)(og.piece + kOutGroup) * kOutPiece >= V ? send_stats() : ASC_OK;
+        }));
+    } else {
+        ASC_TRY(send_stats());
+    }
+    ASC_TRY(wait_host_seq(&t->h[0].finish.seq, want, ctx->s_main));
+    ds = t->h[0].finish.stats;
+    if (!prof) static_ms += ctx->wall_khz > 0 ? (double)ds.ticks / ctx->wall_khz : 0;
     kern[KERN_LOCAL].edges = ds.edges_local;
     kern[KERN_LOCAL].vertices = ds.verts_local;
     kern[KERN_HEAVY].edges = ds.edges_heavy;
@@ -1449,7 +1589,6 @@ int finish_traversal(asc_graph* g, int algo, int path, uint32_t* out, asc_stats*
     kern[KERN_BU].vertices = ds.verts_bu;
     kern[KERN_UF].edges = ds.edges_uf;
     kern[KERN_UF].vertices = path == PATH_UNION_FIND ? V : 0;
-    if (out) ASC_HIP(hipMemcpy(out, t->val, 4 * V, hipMemcpyDeviceToHost));
 
     if (st) {
         std::memset(st, 0, sizeof(*st));
@@ -1473,34 +1612,15 @@ int finish_traversal(asc_graph* g, int algo, int path, uint32_t* out, asc_stats*
         st->path = path;
         std::memcpy(st->kern, kern, sizeof(kern));
     }
-    if (out) {
+    if (out && st) {
         // reached vertices and their degree sum (Graph500 TEPS numerator)
-        const uint32_t unreached = (uint32_t)(V + 1);
-        std::atomic<uint64_t> reached{0}, dsum{0};
-        const uint64_t* off = g->h.off.p;
-        const int conv = ctx->cfg.value_convention;
-        host_pool().parallel_for(V, [&](uint64_t b, uint64_t e) {
-            uint64_t r = 0, d = 0;
-            for (uint64_t v = b; v < e; v++) {
-                if (algo == ALG_CC || out[v] != unreached) {
-                    r++;
-                    d += off[v + 1] - off[v];
-                }
-                if (algo != ALG_CC && conv == ASC_VALUES_ZERO_BASED)
-                    out[v] = out[v] == unreached ? 0xFFFFFFFFu : out[v] - 1;
-            }
-            reached += r;
-            dsum += d;
-        });
-        if (st) {
-            st->reached = reached;
-            st->reached_degree_sum = dsum;
-            // BFS is level-synchronous: each reached vertex is active in
-            // exactly one iteration, so the reference's nodeSum (actives summed
-            // over iterations, CalculateOpt.cu:183-190) is the reached count,
-            // whichever direction each level took
-            if (algo == ALG_BFS) st->node_sum = reached;
-        }
+        st->reached = count ? t->h[0].finish.reached : V;
+        st->reached_degree_sum = count ? t->h[0].finish.degree_sum : g->h.E;
+        // BFS is level-synchronous: each reached vertex is active in
+        // exactly one iteration, so the reference's nodeSum (actives summed
+        // over iterations, CalculateOpt.cu:183-190) is the reached count,
+        // whichever direction each level took
+        if (algo == ALG_BFS) st->node_sum = st->reached;
     }
     if (ctx->cfg.verbose && st) {
         printf("totalProcess time is %.3f ms\npreProcess time is %.3f ms\nstaticProcess time is %.3f ms\n"

@@ -3,6 +3,7 @@
 
 #include "device_common.hpp"
 #include "internal.hpp"
+#include "output.hpp"
 
 namespace asc {
 
@@ -55,6 +56,17 @@ struct DevStats {
     unsigned long long edges_bu;      // k_bfs_bottom_up: edge records read
     unsigned long long verts_bu;      //   unvisited vertices scanned
     unsigned long long edges_uf;      // union-find link passes: edge records read
+    // device time of the resident kernels, in ticks of the constant-rate clock:
+    // a level's first kernel notes when it began, its publish adds the time
+    // since (fully resident runs; streamed ones are timed by events)
+    unsigned long long t_begin, ticks;
+};
+
+// What the end of a run hands to the host beside the values (seq last).
+struct FinishPub {
+    DevStats stats;
+    unsigned long long reached, degree_sum;
+    unsigned long long seq;
 };
 
 enum {
@@ -142,8 +154,22 @@ struct LevelPub {
     Slot slot;
     Piles piles;
     unsigned long long edges;       // edges of a frontier of at most kNarrowCap vertices (else ~0)
+    unsigned long long n_split;     // vertices a split put into the step's own frontier
     unsigned long long seq;
 };
+
+// Arrays to set at the start of a run (null: not used by it).
+struct RunInit {
+    uint32_t *val, *stamp, *pstamp, *fstamp, *done, *visited, *val16;
+    uint64_t V;
+    Slot* slots;
+    Piles* piles;
+    DevStats* stats;
+    DoCounters* dcnt;
+    uint32_t *q0, *pend0;           // get the source when n_res0 / n_pend0 (BFS, SSSP)
+    uint32_t src, unreached, n_res0, n_pend0;
+};
+int launch_run_init(const RunInit& a, int num_cus, hipStream_t s);
 
 // A run of narrow steps as k_narrow publishes it (seq last).
 struct NarrowPub {
@@ -183,7 +209,19 @@ inline int wait_host_seq(const volatile unsigned long long* seq, unsigned long l
     return ASC_OK;
 }
 
+// Host side of the published blocks; each is complete once its sequence number
+// holds the value the host waits for.
+struct HostPubs {
+    LevelPub level;
+    NarrowPub narrow;
+    FinishPub finish;
+    DoCounters bfs[2];              // [0] a level's counters, [1].n_found the sequence number
+    Piles piles;                    // the host's copy
+};
+
 struct TravState {
+    // device arrays below are cut out of these allocations
+    DevArena mem, mem_relax, mem_fast;
     uint64_t V = 0;
     uint32_t* val = nullptr;
     uint16_t* val16 = nullptr;        // SSSP value filter (TravArgs::val16)
@@ -213,15 +251,12 @@ struct TravState {
     int buf_chunk[kMaxPartBufs] = {};
     bool buf_counted[kMaxPartBufs] = {};
     uint64_t part_edges = 0;
-    HostBuf<Slot> h_slot;
-    HostBuf<Piles> h_piles;
-    HostBuf<LevelPub> h_pub;        // written by the device through d_pub (mapped)
-    LevelPub* d_pub = nullptr;
-    unsigned long long lvl_seq = 0;
-    HostBuf<NarrowPub> h_narrow;    // written by the device through d_narrow (mapped)
-    NarrowPub* d_narrow = nullptr;
-    unsigned long long narrow_seq = 0;
-    HostBuf<DevStats> h_stats;
+    // what the device publishes to the host, one page-locked block (mapped)
+    HostBuf<HostPubs> h;
+    HostPubs* d_h = nullptr;
+    unsigned long long lvl_seq = 0, narrow_seq = 0, pub_seq = 0, finish_seq = 0;
+    unsigned long long* d_reach = nullptr;   // reached vertices and their degrees while values are sent
+    OutStage out;
     // the host gather's index of a round's sparse segment: first record of
     // each listed vertex in the gathered array (written by the device through
     // d_hsrc, mapped) and the u64 exclusive prefix of their degrees
@@ -246,14 +281,10 @@ struct TravState {
     // copies (measured once) and the host gather (running estimate)
     double link_bps = 0, gather_bps = 30e9;
     // resident fast paths: frontier bitmaps (the persistent BFS keeps three in
-    // a ring), counters, sampled labels, the persistent kernel's control words
+    // a ring), counters, the persistent kernel's control words
     uint32_t* bm[3] = {nullptr, nullptr, nullptr};
     uint32_t* pctl = nullptr;
     DoCounters* dcnt = nullptr;
-    HostBuf<DoCounters> h_dcnt;     // written by the device through d_hdcnt (mapped): [0] the
-    DoCounters* d_hdcnt = nullptr;  // counters, [1].n_found the sequence number of the last publish
-    unsigned long long pub_seq = 0;
-    HostBuf<uint32_t> h_sample;
     // device part buffer b: copy into it done / last kernel reading it done;
     // staging buffer i: copy out of it done
     hipEvent_t ev_copy[kMaxPartBufs] = {}, ev_kern[kMaxPartBufs] = {}, ev_meta = nullptr;
@@ -270,6 +301,7 @@ struct TravState {
 
 int traverse(asc_graph* g, int algo, uint32_t src, uint32_t* out, asc_stats* st);
 int trav_ensure(asc_graph* g);
+int trav_ensure_relax(asc_graph* g);   // and what SSSP / label propagation add
 hipEvent_t next_event(TravState* t);
 
 // Launches through `launch`; when profiling, brackets it with an event pair on
