@@ -54,7 +54,7 @@ struct PrState {
     void* rows_blocks = nullptr;
     uint32_t* rows_heavy = nullptr;
     uint32_t rows_n = 0, rows_cap = 0, rows_front = 0, rows_back = 0;
-    bool rows_built = false;
+    bool heavy_built = false, rows_built = false;
     // on-demand in-edges: vertex-range chunks [v0, v1) whose in-edges
     // [off[v0], off[v1]) fit one part buffer, copied from the pinned tail
     struct Chunk {
@@ -65,20 +65,17 @@ struct PrState {
     uint64_t part_edges = 0;
     hipEvent_t ev_copy[2] = {nullptr, nullptr}, ev_kern[2] = {nullptr, nullptr};
     uint64_t streamed_edges = 0;  // per pull sweep
-    // propagation-blocked normalised mode (every edge resident): out-edge e
-    // of source src_of[e] writes its contribution to slot pos[e] (or none,
-    // kPbSkip, when its destination is heavy); the slots of destination bin
-    // b and source range r form one region, slot k feeding bin-local vertex
-    // dl[k]
+    // propagation-blocked normalised mode (every edge resident): the light
+    // in-edges regrouped by (source slice, destination bin) into runs, each
+    // padded to whole quads of edges
     int pb_state = 0;             // 0 not built, 1 built, -1 not possible
-    uint32_t pb_nbins = 0;
-    uint64_t pb_edges = 0;        // out-edges (= E)
-    uint32_t* pb_src = nullptr;
-    uint32_t* pb_pos = nullptr;
-    uint16_t* pb_dl = nullptr;
-    float* pb_vals = nullptr;
-    unsigned long long* pb_bin_start = nullptr;   // region bases [b * R + r]
-    uint32_t* pb_cnt = nullptr;                   // region sizes [b * R + r]
+    bool outdeg_sums = false;     // the out-degrees were found to sum to E
+    uint32_t pb_sbits = 0, pb_dbits = 0, pb_nbins = 0, pb_nitems = 0;
+    void* pb_src = nullptr;       // u16 slice-local sources, in slice order
+    void* pb_dst = nullptr;       // u16 bin-local destinations, in bin order
+    uint32_t* pb_pos = nullptr;   // in bin order: an oct's place in slice order
+    float* pb_vals = nullptr;     // contributions on their way, in slice order
+    void *pb_bins = nullptr, *pb_items = nullptr;
     // source-segmented normalised mode (every edge resident): the light
     // in-edges regrouped into tiles (destination block d, source segment s),
     // tile (d, s) at tl_edges[tl_off[d * tl_ns + s] ...], one u32 word per
@@ -100,7 +97,7 @@ void pr_free(PrState* p) {
     f(p->acc); f(p->resid); f(p->val64); f(p->contrib64[0]); f(p->contrib64[1]); f(p->active);
     f(p->count); f(p->rows_heavy); f(p->rows_blocks);
     f(p->part[0]); f(p->part[1]);
-    f(p->pb_src); f(p->pb_pos); f(p->pb_dl); f(p->pb_vals); f(p->pb_bin_start); f(p->pb_cnt);
+    f(p->pb_src); f(p->pb_dst); f(p->pb_vals); f(p->pb_pos); f(p->pb_bins); f(p->pb_items);
     f(p->tl_edges); f(p->tl_off); f(p->tl_heavy);
     for (int i = 0; i < 2; i++) {
         if (p->ev[i]) (void)hipEventDestroy(p->ev[i]);
@@ -287,6 +284,7 @@ struct RowBlock {
 template <class OffT>
 __global__ __launch_bounds__(kBlock) void k_row_blocks(const OffT* off, uint64_t n, RowBlock* blocks, uint32_t* cnt) {
     __shared__ uint64_t s_break[kWavesPerBlock];
+    __shared__ uint32_t s_count[kWavesPerBlock], s_at;
     const uint32_t lane = lane_id(), w = wave_id();
     for (uint64_t base = (uint64_t)blockIdx.x * kBlock; base < n; base += (uint64_t)gridDim.x * kBlock) {
         const uint64_t v = base + threadIdx.x;
@@ -302,11 +300,18 @@ __global__ __launch_bounds__(kBlock) void k_row_blocks(const OffT* off, uint64_t
         }
         const uint64_t brk = wave_ballot(starts || heavy || v >= n);
         if (lane == 0) s_break[w] = brk;
-        __syncthreads();
         const uint64_t m = wave_ballot(starts);
-        uint32_t at = 0;
-        if (lane == 0 && m) at = atomicAdd(cnt, (uint32_t)__popcll(m));
-        at = __shfl(at, 0, kWave);
+        // one global atomic per 256 vertices
+        if (lane == 0) s_count[w] = (uint32_t)__popcll(m);
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            uint32_t all = 0;
+            for (int i = 0; i < kWavesPerBlock; i++) all += s_count[i];
+            s_at = all ? atomicAdd(cnt, all) : 0;
+        }
+        __syncthreads();
+        uint32_t at = s_at;
+        for (uint32_t i = 0; i < w; i++) at += s_count[i];
         if (starts) {
             // the next break after this lane ends the block
             uint32_t end = kBlock;
@@ -386,10 +391,12 @@ struct RowPlan {
 // whole grid take ~9 ns each, 18 us for 2048 workgroups), and the readers add
 // the lines up.  Slot it & 3 holds the dangling mass of the ranks iteration
 // `it` reads and the residual of iteration it - 1; iteration `it` clears slot
-// (it + 2) & 3.
+// (it + 2) & 3.  Beside them, the largest contribution that iteration `it`
+// gathers (float bits; the blocked schedule's scale).
 constexpr int kAccLine = 16;                            // doubles per 128-byte line
 constexpr int kAccDang = kPrLines * kAccLine;           // the dangling lines follow the residual lines
-constexpr int kAccSlot = 2 * kAccDang;
+constexpr int kAccMax = 2 * kAccDang;                   // and the maximum's follow those
+constexpr int kAccSlot = 3 * kAccDang;
 constexpr int kAccSlots = 4;
 
 // Sum of a slot's lines (the residual's at `p`, the dangling mass's at
@@ -399,40 +406,61 @@ __device__ __forceinline__ double acc_lines(const double* p) {
     return wave_sum(l < (uint32_t)kPrLines ? p[l * kAccLine] : 0.0);
 }
 
-// Workgroup sums of res and dang, added to this workgroup's lines of `acc`.
+// What a lane adds up over the vertices it finishes.
+struct PrSums {
+    double res = 0, dang = 0;
+    uint32_t most = 0;           // float bits of the largest contribution written (they order as the values do)
+    __device__ __forceinline__ void wrote(float c) { most = max(most, __float_as_uint(c)); }
+};
+
+// Workgroup sums, added to this workgroup's lines of `acc`.
 template <int THREADS>
-__device__ __forceinline__ void acc_add(double res, double dang, double* acc) {
+__device__ __forceinline__ void acc_add(const PrSums& a, double* acc) {
     __shared__ double s_r[THREADS / kWave], s_d[THREADS / kWave];
-    res = wave_sum(res);
-    dang = wave_sum(dang);
+    __shared__ uint32_t s_m[THREADS / kWave];
+    const double res = wave_sum(a.res), dang = wave_sum(a.dang);
+    uint32_t most = a.most;
+#pragma unroll
+    for (int d = kWave / 2; d > 0; d >>= 1) most = max(most, (uint32_t)__shfl_xor(most, d, kWave));
     if (lane_id() == 0) {
         s_r[wave_id()] = res;
         s_d[wave_id()] = dang;
+        s_m[wave_id()] = most;
     }
     __syncthreads();
     if (threadIdx.x == 0) {
         double r = 0, d = 0;
+        uint32_t m = 0;
         for (int i = 0; i < THREADS / kWave; i++) {
             r += s_r[i];
             d += s_d[i];
+            m = max(m, s_m[i]);
         }
         double* line = acc + (blockIdx.x % kPrLines) * kAccLine;
         if (r != 0) atomicAdd(line, r);
         if (d != 0) atomicAdd(line + kAccDang, d);
+        if (m) atomicMax((uint32_t*)(line + kAccMax), m);
     }
+}
+
+__global__ void k_pr_fill(uint32_t* p, uint64_t n, uint32_t v) {
+    for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
+        p[i] = v;
 }
 
 __global__ __launch_bounds__(kBlock) void k_pr_init(float* rank, float* contrib, const uint32_t* outdeg, uint64_t V,
                                                     double* acc) {
     const float r0 = (float)(1.0 / (double)V);
-    double dang = 0;
+    PrSums sums;
     for (uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v < V; v += (uint64_t)gridDim.x * blockDim.x) {
         const uint32_t d = outdeg[v];
+        const float c = d ? r0 / (float)d : 0.0f;
         rank[v] = r0;
-        contrib[v] = d ? r0 / (float)d : 0.0f;
-        if (!d) dang += (double)r0;
+        contrib[v] = c;
+        sums.wrote(c);
+        if (!d) sums.dang += (double)r0;
     }
-    acc_add<kBlock>(0.0, dang, acc);
+    acc_add<kBlock>(sums, acc);
 }
 
 // The last iteration's residual, then all of them to mapped host memory and
@@ -475,17 +503,18 @@ struct PrOwn {
 __device__ __forceinline__ PrOwn pr_own(const PrArgs& a, uint64_t v) { return PrOwn{a.outdeg[v], a.rank_in[v]}; }
 
 __device__ __forceinline__ void pr_finish_vertex(const PrArgs& a, uint64_t v, double s, const PrOwn& own, double base,
-                                                 double& res, double& dang) {
+                                                 PrSums& sums) {
     const float nr = (float)(base + a.damping64 * s);
-    res += fabs((double)nr - (double)own.rank);
+    const float c = own.outdeg ? nr / (float)own.outdeg : 0.0f;
+    sums.res += fabs((double)nr - (double)own.rank);
+    sums.wrote(c);
     a.rank_out[v] = nr;
-    a.contrib_out[v] = own.outdeg ? nr / (float)own.outdeg : 0.0f;
-    if (!own.outdeg) dang += (double)nr;
+    a.contrib_out[v] = c;
+    if (!own.outdeg) sums.dang += (double)nr;
 }
 
-__device__ __forceinline__ void pr_finish_vertex(const PrArgs& a, uint64_t v, double s, double base, double& res,
-                                                 double& dang) {
-    pr_finish_vertex(a, v, s, pr_own(a, v), base, res, dang);
+__device__ __forceinline__ void pr_finish_vertex(const PrArgs& a, uint64_t v, double s, double base, PrSums& sums) {
+    pr_finish_vertex(a, v, s, pr_own(a, v), base, sums);
 }
 
 // Rank of a vertex whose in-sum is zero, in every lane; called by the whole
@@ -564,33 +593,33 @@ __global__ __launch_bounds__(kBlock) void k_pr_rows(PrArgs a, RowPlan rows, uint
     const OffT* off = (const OffT*)a.off;
     const uint32_t* src = a.src - a.e_base;
     const double base = pr_base(a);
-    double res = 0, dang = 0;
+    PrSums sums;
     if (HEAVY && blockIdx.x < hb) {
         for (uint32_t i = blockIdx.x; i < rows.n_front; i += hb) {
             const uint32_t v = rows.front(i);
             const double s = pull_long_row<OffT>(src, a.contrib_in, off[v], off[v + 1], s_sum);
-            if (threadIdx.x == 0) pr_finish_vertex(a, v, s, base, res, dang);
+            if (threadIdx.x == 0) pr_finish_vertex(a, v, s, base, sums);
         }
         for (uint32_t i = blockIdx.x * kWavesPerBlock + wave_id(); i < rows.n_back; i += hb * kWavesPerBlock) {
             const uint32_t v = rows.back(i);
             const double s = pull_wave_row<OffT>(src, a.contrib_in, off[v], off[v + 1]);
-            if (lane_id() == 0) pr_finish_vertex(a, v, s, base, res, dang);
+            if (lane_id() == 0) pr_finish_vertex(a, v, s, base, sums);
         }
     } else {
         const uint32_t bid = blockIdx.x - (HEAVY ? hb : 0), nblk = gridDim.x - (HEAVY ? hb : 0);
         if (HEAVY) {
             auto pre = [&](uint64_t v) { return pr_own(a, v); };
-            auto fin = [&](uint64_t v, double s, const PrOwn& own) { pr_finish_vertex(a, v, s, own, base, res, dang); };
+            auto fin = [&](uint64_t v, double s, const PrOwn& own) { pr_finish_vertex(a, v, s, own, base, sums); };
             for (uint32_t i = bid; i < rows.n_blocks; i += nblk)
                 pull_block(off, src, a.contrib_in, rows.blocks[i], s_val, pre, fin);
         } else {
             auto take = [](uint64_t) { return true; };
-            auto fin = [&](uint64_t v, double s) { pr_finish_vertex(a, v, s, base, res, dang); };
+            auto fin = [&](uint64_t v, double s) { pr_finish_vertex(a, v, s, base, sums); };
             for (uint64_t v = a.v_begin + (uint64_t)bid * kBlock; v < a.v_end; v += (uint64_t)nblk * kBlock)
                 pull_rows(off, src, a.contrib_in, v, a.v_end, s_val, take, fin);
         }
     }
-    acc_add<kBlock>(res, dang, a.acc_out);
+    acc_add<kBlock>(sums, a.acc_out);
 }
 
 // G lanes per vertex (asc_config.pr_group or a tuned graph); vertices with
@@ -602,7 +631,7 @@ __global__ __launch_bounds__(kBlock) void k_pr_pull(PrArgs a) {
     const uint32_t sub = threadIdx.x % G;
     const uint64_t groups_per_grid = (uint64_t)gridDim.x * (blockDim.x / G);
     const uint32_t* src = a.src - a.e_base;
-    double res = 0, dang = 0;
+    PrSums sums;
     for (uint64_t v = a.v_begin + blockIdx.x * (uint64_t)(blockDim.x / G) + threadIdx.x / G; v < a.v_end;
          v += groups_per_grid) {
         const OffT b = off[v], e = off[v + 1];
@@ -626,9 +655,9 @@ __global__ __launch_bounds__(kBlock) void k_pr_pull(PrArgs a) {
         }
 #pragma unroll
         for (int d = G / 2; d > 0; d >>= 1) s += __shfl_xor(s, d, G);
-        if (sub == 0 && !heavy) pr_finish_vertex(a, v, s, base, res, dang);
+        if (sub == 0 && !heavy) pr_finish_vertex(a, v, s, base, sums);
     }
-    acc_add<kBlock>(res, dang, a.acc_out);
+    acc_add<kBlock>(sums, a.acc_out);
 }
 
 template <class OffT>
@@ -636,140 +665,309 @@ __global__ __launch_bounds__(kBlock) void k_pr_pull_heavy(PrArgs a, const uint32
     __shared__ double s_sum[kWavesPerBlock];
     const OffT* off = (const OffT*)a.off;
     const double base = pr_base(a);
-    double res = 0, dang = 0;
+    PrSums sums;
     for (uint32_t i = blockIdx.x; i < n_heavy; i += gridDim.x) {
         const uint32_t v = heavy[i];
         const double s = pull_long_row<OffT>(a.src, a.contrib_in, off[v], off[v + 1], s_sum);
-        if (threadIdx.x == 0) pr_finish_vertex(a, v, s, base, res, dang);
+        if (threadIdx.x == 0) pr_finish_vertex(a, v, s, base, sums);
     }
-    acc_add<kBlock>(res, dang, a.acc_out);
+    acc_add<kBlock>(sums, a.acc_out);
 }
 
 // ---- propagation-blocked normalised mode -----------------------------------
-// The pull gathers one random 4-byte contribution per in-edge and is bound by
-// the lines those gathers move.  This schedule streams instead (selected by
-// ASC_PR_BLOCKED; on Erdos-Renyi 2^26 / 2^31 edges it measured 46 ms scatter +
-// 11.5 ms gather per iteration against 42 ms for the pull, the scattered
-// 4-byte slot writes evicting partly filled lines):
-//   scatter  out-edge e of source u writes contrib[u] to its slot pos[e]
-//            (sources in order, so contrib is read sequentially; the slots of
-//            one source range and destination bin are contiguous);
-//   gather   one workgroup per bin of 32768 destinations adds its slots into
-//            LDS (FP32) and finishes those vertices.
-// The slot layout is fixed by the graph and built once.  Destinations with
-// in-degree >= the heavy threshold keep the FP64 pull (k_pr_pull_heavy).
-constexpr int kPbBinBits = 15;
-constexpr uint32_t kPbBin = 1u << kPbBinBits;   // destinations per bin (128 KB of sums)
-constexpr uint32_t kPbSkip = 0xFFFFFFFFu;       // out-edge into a heavy destination
-constexpr uint32_t kPbRanges = 2048;            // source ranges of the slot layout
-constexpr int kPbBlock = 1024;                  // gather workgroup
-constexpr uint32_t kPbMaxBins = 8192;           // build histograms live in LDS
+// A pull's random 4-byte gathers each bring a 128-byte line from L2 into L1,
+// and a CU takes 64 bytes a clock: 3.3 ps an edge over the chip at best (the
+// row blocks measure 5.2 to 6.8 while the contributions fit the L2s, 16 at V =
+// 2^23 Erdos-Renyi), and the tiled pull below measures 5.8 to 400.  Here every
+// random access is to LDS and memory is only streamed, 12.5 bytes an edge:
+//   scatter  a workgroup loads the contributions of one slice of sources into
+//            LDS and writes, for each of a stretch of the slice's edges, the
+//            contribution of its source (2-byte local id) to the edge's place;
+//   gather   a workgroup per bin of destinations adds the values of the bin's
+//            edges into LDS sums (2-byte local ids) and finishes its vertices.
+// A slice's edges of one bin are a run, padded to octs.  Sources and values
+// lie in slice order, so the scatter reads and writes straight through;
+// destinations lie in bin order, with each oct's place in slice order, so the
+// gather's lanes are busy whatever the runs' lengths and its value reads are
+// runs of a few KB.  Bins are cut by vertices and by edges, so skewed graphs
+// get bins of equal work; a row of kRowsLong edges and more is a bin of its
+// own, summed in registers.  The layout depends on the graph alone and is
+// built once (2^28 edges: 14 ms).
+// 20 iterations in ms, this / tiled / row blocks:
+//   Erdos-Renyi V = 2^23, 2^28 edges  14.8 / 31.3 / 86.2 (scatter 328 us and
+//                                     gather 408 us an iteration, both at the
+//                                     ~5 TB/s that memory gives)
+//   R-MAT scale 23, 2.6e8 edges       17.1 / 152 / 41.0
+//   R-MAT scale 20, 3.1e7 edges       2.27 / 109 / 3.28
+//   Erdos-Renyi V = 2^18, 2^23 edges  0.66 / 13.5 / 1.07
+//   R-MAT scale 18, 7.6e6 edges       0.91 / 46.0 / 0.80
+//   Erdos-Renyi V = 2^22, 8.4e6 edges 0.75 / 2.19 / 2.94
+constexpr int kPbBlock = 1024;
+constexpr uint32_t kPbOct = 8;                  // edges a lane moves at a time; runs are padded to it
+constexpr uint32_t kPbItemOcts = 1u << 14;      // octs per scatter workgroup, at most
+constexpr uint32_t kPbMaxSlices = 8192;         // build histograms in LDS
 
-// out_dst[cursor[u]++] = v for every in-edge (u -> v): the out-CSR of a
-// graph given as in-CSR (order within an out-list is arbitrary).
+struct PbBin {
+    uint32_t v, n;               // vertices [v, v + n)
+    uint32_t o, octs;            // octs [o, o + octs) in bin order
+    uint32_t kind;               // kPbPlain / kPbAround / kPbHeavy
+};
+constexpr uint32_t kPbPlain = 0;
+constexpr uint32_t kPbAround = 1;   // holds rows of kRowsLong edges and more, which are not its own
+constexpr uint32_t kPbHeavy = 2;    // is one such row: summed in registers
+struct PbRun {
+    uint32_t q, n, o;            // octs [q, q + n) in slice order, [o, o + n) in bin order
+};
+struct PbItem {
+    uint32_t slice, q0, q1;
+};
+typedef unsigned short PbIds __attribute__((ext_vector_type(8)));   // the ids of an oct
+
+// cnt[b * ns + s]: edges of bin b from slice s.  A workgroup per bin.
 template <class OffT>
-__global__ __launch_bounds__(kBlock) void k_pb_transpose(const OffT* in_off, const uint32_t* in_src, uint64_t V,
-                                                         unsigned long long* cursor, uint32_t* out_dst) {
-    for (uint64_t v = blockIdx.x * (uint64_t)kBlock + threadIdx.x; v < V; v += (uint64_t)gridDim.x * kBlock)
-        for (OffT k = in_off[v]; k < in_off[v + 1]; k++)
-            out_dst[atomicAdd(cursor + in_src[k], 1ull)] = (uint32_t)v;
-}
-
-// src[e] = u for the out-edges e of u.
-template <class OffT>
-__global__ __launch_bounds__(kBlock) void k_pb_src(const OffT* out_off, uint64_t V, uint32_t* src) {
-    for (uint64_t u = blockIdx.x * (uint64_t)kBlock + threadIdx.x; u < V; u += (uint64_t)gridDim.x * kBlock)
-        for (OffT e = out_off[u]; e < out_off[u + 1]; e++) src[e] = (uint32_t)u;
-}
-
-__device__ __forceinline__ uint64_t pb_range_begin(uint64_t E, uint32_t r) { return E * r / kPbRanges; }
-
-// cnt[b * kPbRanges + r]: out-edges of range r (edges [E r / R, E (r+1) / R))
-// into light destinations of bin b.
-template <class OffT>
-__global__ __launch_bounds__(kBlock) void k_pb_count(const uint32_t* out_dst, uint64_t E, const OffT* in_off,
-                                                     uint32_t heavy_thr, uint32_t nb, uint32_t* cnt) {
-    __shared__ uint32_t h[kPbMaxBins];
-    for (uint32_t r = blockIdx.x; r < kPbRanges; r += gridDim.x) {
-        for (uint32_t b = threadIdx.x; b < nb; b += kBlock) h[b] = 0;
-        __syncthreads();
-        for (uint64_t e = pb_range_begin(E, r) + threadIdx.x; e < pb_range_begin(E, r + 1); e += kBlock) {
-            const uint32_t v = out_dst[e];
-            if ((uint64_t)(in_off[v + 1] - in_off[v]) < heavy_thr) atomicAdd(&h[v >> kPbBinBits], 1u);
+__global__ __launch_bounds__(kPbBlock) void k_pb_count(const OffT* off, const uint32_t* src, const PbBin* bins,
+                                                       uint32_t ns, uint32_t bits, uint32_t* cnt) {
+    __shared__ uint32_t h[kPbMaxSlices];
+    const PbBin b = bins[blockIdx.x];
+    for (uint32_t i = threadIdx.x; i < ns; i += kPbBlock) h[i] = 0;
+    __syncthreads();
+    if (b.kind == kPbAround) {
+        constexpr uint32_t L = 8;
+        for (uint32_t r = threadIdx.x / L; r < b.n; r += kPbBlock / L) {
+            const OffT e0 = off[b.v + r], e1 = off[b.v + r + 1];
+            if (e1 - e0 >= kRowsLong) continue;
+            for (OffT e = e0 + threadIdx.x % L; e < e1; e += L) atomicAdd(&h[src[e] >> bits], 1u);
         }
+    } else {
+        const OffT e1 = off[b.v + b.n];
+        for (OffT e = off[b.v] + threadIdx.x; e < e1; e += kPbBlock) atomicAdd(&h[src[e] >> bits], 1u);
+    }
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < ns; i += kPbBlock) cnt[(size_t)blockIdx.x * ns + i] = h[i];
+}
+
+// Octs of every slice (SLICES: a workgroup per slice, else per bin).
+template <bool SLICES>
+__global__ __launch_bounds__(kBlock) void k_pb_totals(const uint32_t* cnt, uint32_t nb, uint32_t ns, uint32_t* out) {
+    __shared__ uint32_t s_sum[kWavesPerBlock];
+    uint32_t sum = 0;
+    for (uint32_t i = threadIdx.x; i < (SLICES ? nb : ns); i += kBlock)
+        sum += (cnt[SLICES ? (size_t)i * ns + blockIdx.x : (size_t)blockIdx.x * ns + i] + kPbOct - 1) / kPbOct;
+    sum = wave_sum(sum);
+    if (lane_id() == 0) s_sum[wave_id()] = sum;
+    __syncthreads();
+    if (threadIdx.x == 0) out[blockIdx.x] = s_sum[0] + s_sum[1] + s_sum[2] + s_sum[3];
+}
+
+// The runs' places: in slice order (SLICES: a workgroup per slice goes through
+// the bins), else in bin order (a workgroup per bin goes through the slices).
+template <bool SLICES>
+__global__ __launch_bounds__(kBlock) void k_pb_place(const uint32_t* cnt, uint32_t nb, uint32_t ns,
+                                                     const uint32_t* first, PbRun* runs) {
+    __shared__ uint32_t s_sum[kWavesPerBlock];
+    uint32_t at = first[blockIdx.x];
+    for (uint32_t i0 = 0; i0 < (SLICES ? nb : ns); i0 += kBlock) {
+        const uint32_t i = i0 + threadIdx.x;
+        const bool in = i < (SLICES ? nb : ns);
+        const size_t k = SLICES ? (size_t)i * ns + blockIdx.x : (size_t)blockIdx.x * ns + i;
+        const uint32_t n = in ? (cnt[k] + kPbOct - 1) / kPbOct : 0;
+        uint32_t x = n;   // inclusive sum over the wave
+#pragma unroll
+        for (int d = 1; d < kWave; d <<= 1) {
+            const uint32_t y = __shfl_up(x, d, kWave);
+            if (lane_id() >= (uint32_t)d) x += y;
+        }
+        if (lane_id() == kWave - 1) s_sum[wave_id()] = x;
         __syncthreads();
-        for (uint32_t b = threadIdx.x; b < nb; b += kBlock) cnt[(size_t)b * kPbRanges + r] = h[b];
+        uint32_t before = 0, all = 0;
+        for (uint32_t w = 0; w < (uint32_t)kWavesPerBlock; w++) {
+            if (w < wave_id()) before += s_sum[w];
+            all += s_sum[w];
+        }
+        const uint32_t place = at + before + x - n;
+        if (in && SLICES) {
+            runs[k].q = place;
+            runs[k].n = n;
+        } else if (in) {
+            runs[k].o = place;
+        }
+        at += all;
         __syncthreads();
     }
 }
 
-// pos[e] for every out-edge (slots of (bin, range) handed out from
-// base[b * kPbRanges + r]) and dl[slot] = bin-local destination.
+// The local ids of every edge of a bin (source in the low half of a word,
+// destination in the high), in arrival order within its runs.  Eight lanes
+// share a row.  The LDS array is larger than the cursors need: one workgroup a
+// CU keeps the runs' open lines (128 bytes a run) within the XCD's L2.
 template <class OffT>
-__global__ __launch_bounds__(kBlock) void k_pb_assign(const uint32_t* out_dst, uint64_t E, const OffT* in_off,
-                                                      uint32_t heavy_thr, uint32_t nb,
-                                                      const unsigned long long* base, uint32_t* pos, uint16_t* dl) {
-    __shared__ unsigned long long cur[kPbMaxBins];
-    for (uint32_t r = blockIdx.x; r < kPbRanges; r += gridDim.x) {
-        for (uint32_t b = threadIdx.x; b < nb; b += kBlock) cur[b] = base[(size_t)b * kPbRanges + r];
-        __syncthreads();
-        for (uint64_t e = pb_range_begin(E, r) + threadIdx.x; e < pb_range_begin(E, r + 1); e += kBlock) {
-            const uint32_t v = out_dst[e];
-            if ((uint64_t)(in_off[v + 1] - in_off[v]) < heavy_thr) {
-                const unsigned long long k = atomicAdd(&cur[v >> kPbBinBits], 1ull);
-                pos[e] = (uint32_t)k;
-                dl[k] = (uint16_t)(v & (kPbBin - 1));
-            } else {
-                pos[e] = kPbSkip;
-            }
+__global__ __launch_bounds__(kPbBlock) void k_pb_fill(const OffT* off, const uint32_t* src, const PbBin* bins,
+                                                      const PbRun* runs, uint32_t ns, uint32_t bits, uint32_t* out) {
+    constexpr uint32_t L = 8;
+    __shared__ unsigned long long cur[kPbMaxSlices + kPbMaxSlices / 4 + 128];
+    const PbBin b = bins[blockIdx.x];
+    for (uint32_t i = threadIdx.x; i < ns; i += kPbBlock) cur[i] = (uint64_t)kPbOct * runs[(size_t)blockIdx.x * ns + i].q;
+    __syncthreads();
+    const uint32_t mask = (1u << bits) - 1;
+    if (b.kind == kPbHeavy) {
+        const OffT e1 = off[b.v + 1];
+        for (OffT e = off[b.v] + threadIdx.x; e < e1; e += kPbBlock) {
+            const uint32_t u = src[e];
+            out[atomicAdd(&cur[u >> bits], 1ull)] = u & mask;
         }
-        __syncthreads();
+        return;
     }
-}
-
-// Workgroups are dealt to the 8 XCDs round-robin (blockIdx % 8), and each
-// XCD walks the source ranges x, x + 8, ... with all of its workgroups on one
-// range at a time: a range writes 2048 slot regions (one per bin), whose
-// partly filled lines then stay in that XCD's L2 until they are whole instead
-// of being written back from every XCD.  The grid is a multiple of 8.
-__global__ __launch_bounds__(kBlock) void k_pb_scatter(const uint32_t* src, const uint32_t* pos, uint64_t E,
-                                                       const float* contrib, float* vals) {
-    const uint32_t xcd = blockIdx.x & 7u, local = blockIdx.x >> 3, nloc = gridDim.x >> 3;
-    for (uint32_t r = xcd; r < kPbRanges; r += 8) {
-        const uint64_t e1 = pb_range_begin(E, r + 1);
-        for (uint64_t e = pb_range_begin(E, r) + (uint64_t)local * kBlock + threadIdx.x; e < e1;
-             e += (uint64_t)nloc * kBlock) {
-            const uint32_t k = pos[e];
-            if (k != kPbSkip) vals[k] = contrib[src[e]];
+    for (uint32_t r = threadIdx.x / L; r < b.n; r += kPbBlock / L) {
+        const OffT e0 = off[b.v + r], e1 = off[b.v + r + 1];
+        if (b.kind == kPbAround && e1 - e0 >= kRowsLong) continue;
+        for (OffT e = e0 + threadIdx.x % L; e < e1; e += L) {
+            const uint32_t u = src[e];
+            out[atomicAdd(&cur[u >> bits], 1ull)] = (u & mask) | (r << 16);
         }
     }
 }
 
-// The slots of bin b are the regions (b, r) of every source range r, at
-// reg_base[b * R + r] with cnt[b * R + r] slots; a wave adds one region at a
-// time.
-template <class OffT>
-__global__ __launch_bounds__(kPbBlock) void k_pb_gather(PrArgs a, const unsigned long long* reg_base,
-                                                        const uint32_t* cnt, const uint16_t* dl, const float* vals) {
-    __shared__ float acc[kPbBin];
+// Splits the pairs: sources stay in slice order, destinations go to bin order,
+// where `pos` has each oct's place in slice order.  Eight lanes take a run.
+__global__ __launch_bounds__(kPbBlock) void k_pb_unzip(const PbRun* runs, uint32_t ns, const uint4* in, PbIds* src,
+                                                       PbIds* dst, uint32_t* pos) {
+    constexpr uint32_t L = 8;
+    for (uint32_t i = threadIdx.x / L; i < ns; i += kPbBlock / L) {
+        const PbRun r = runs[(size_t)blockIdx.x * ns + i];
+        for (uint32_t k = threadIdx.x % L; k < r.n; k += L) {
+            const uint32_t q = r.q + k;
+            const uint4 x = in[2 * (size_t)q], y = in[2 * (size_t)q + 1];
+            src[q] = PbIds{(unsigned short)x.x, (unsigned short)x.y, (unsigned short)x.z, (unsigned short)x.w,
+                           (unsigned short)y.x, (unsigned short)y.y, (unsigned short)y.z, (unsigned short)y.w};
+            dst[r.o + k] = PbIds{(unsigned short)(x.x >> 16), (unsigned short)(x.y >> 16), (unsigned short)(x.z >> 16),
+                                 (unsigned short)(x.w >> 16), (unsigned short)(y.x >> 16), (unsigned short)(y.y >> 16),
+                                 (unsigned short)(y.z >> 16), (unsigned short)(y.w >> 16)};
+            pos[r.o + k] = q;
+        }
+    }
+}
+
+// Consecutive items (of one slice, mostly) go to one XCD, so a slice comes
+// into one L2.
+template <int BITS>
+__global__ __launch_bounds__(kPbBlock) void k_pb_scatter(const float* __restrict__ contrib, uint64_t V,
+                                                         const PbItem* __restrict__ items, uint32_t n_items,
+                                                         const ushort4* __restrict__ src, float4* __restrict__ vals) {
+    __shared__ float s_c[1u << BITS];
+    const uint32_t per = (n_items + 7) / 8, id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if ((blockIdx.x >> 3) >= per || id >= n_items) return;
+    const PbItem it = items[id];
+    const uint64_t base = (uint64_t)it.slice << BITS;
+    const uint32_t have = (uint32_t)min<uint64_t>(1u << BITS, V - base);
+    for (uint32_t i = threadIdx.x; i < have / 4; i += kPbBlock)
+        ((float4*)s_c)[i] = ((const float4*)(contrib + base))[i];
+    for (uint32_t i = (have & ~3u) + threadIdx.x; i < have; i += kPbBlock) s_c[i] = contrib[base + i];
+    __syncthreads();
+    // half an oct a lane: whole lines per store
+    constexpr int U = 4;
+    const uint32_t q1 = 2 * it.q1;
+    for (uint32_t q = 2 * it.q0 + threadIdx.x; q < q1; q += U * kPbBlock) {
+        ushort4 u[U];
+#pragma unroll
+        for (int j = 0; j < U; j++) u[j] = src[min(q + j * kPbBlock, q1 - 1)];
+#pragma unroll
+        for (int j = 0; j < U; j++)
+            if (q + j * kPbBlock < q1)
+                vals[q + j * kPbBlock] = make_float4(s_c[u[j].x], s_c[u[j].y], s_c[u[j].z], s_c[u[j].w]);
+    }
+}
+
+// Sums in LDS are 64-bit fixed point: a 64-lane FP32 LDS add takes 136 clocks
+// on gfx950 (the lanes one after the other; FP32 sums ran 1363 us an iteration
+// at V = 2^23, 2^28 edges, all of it those adds), an integer one a few.  With
+// the largest contribution c below 2^e and fewer than 2^12 edges a row, units
+// of 2^(e - 51) cannot overflow, a contribution of 2^-27 of the largest still
+// keeps its 24 bits, and sums are exact in these units whatever their order.
+// Every rank is at least its base, so a contribution of kPbSpread bases at
+// most keeps an edge's rounding below 2^-32 of the rank.  Beyond that (a
+// vertex with a large share of all rank and few out-edges, or out-degrees too
+// small for the edges, whose ranks grow to infinity) sums are FP64.
+constexpr double kPbSpread = 1 << 20;
+__device__ __forceinline__ uint32_t pb_most(const double* slot) {
+    const uint32_t l = lane_id();
+    uint32_t m = l < (uint32_t)kPrLines ? *(const uint32_t*)(slot + kAccMax + l * kAccLine) : 0u;
+#pragma unroll
+    for (int d = kWave / 2; d > 0; d >>= 1) m = max(m, (uint32_t)__shfl_xor(m, d, kWave));
+    return m;
+}
+__device__ __forceinline__ unsigned long long pb_fixed(float x, int shift) {
+    const uint32_t bits = __float_as_uint(x);
+    const int s = max((int)(bits >> 23), 1) + shift;
+    const unsigned long long m = (bits & 0x7FFFFFu) | (bits >> 23 ? 0x800000u : 0u);
+    return s >= 0 ? m << s : s > -25 ? (m + (1ull << (-s - 1))) >> -s : 0ull;
+}
+
+// A lane takes an oct at a time, wherever its run begins or ends (a wave per
+// run left most lanes idle on R-MAT graphs, whose runs are mostly short: 1040
+// us at V = 2^23).  The padding of a run adds to one sum past the bin's.
+template <class OffT, int BITS>
+__global__ __launch_bounds__(kPbBlock) void k_pb_gather(PrArgs a, const PbBin* __restrict__ bins,
+                                                        const uint32_t* __restrict__ pos,
+                                                        const ushort4* __restrict__ dst,
+                                                        const float4* __restrict__ vals) {
+    __shared__ unsigned long long acc[(1u << BITS) + 1];
+    const PbBin b = bins[blockIdx.x];
     const OffT* off = (const OffT*)a.off;
-    const uint32_t b = blockIdx.x;
-    for (uint32_t i = threadIdx.x; i < kPbBin; i += kPbBlock) acc[i] = 0.0f;
-    __syncthreads();
-    for (uint32_t r = threadIdx.x / kWave; r < kPbRanges; r += kPbBlock / kWave) {
-        const unsigned long long k0 = reg_base[(size_t)b * kPbRanges + r];
-        const uint32_t n = cnt[(size_t)b * kPbRanges + r];
-        for (uint32_t k = lane_id(); k < n; k += kWave) atomicAdd(&acc[dl[k0 + k]], vals[k0 + k]);
+    for (uint32_t i = threadIdx.x; i < b.n; i += kPbBlock) acc[i] = 0;
+    const uint32_t big = pb_most(a.acc_in);
+    // shift of a 24-bit mantissa, less its exponent field: the largest
+    // contribution is below 2^(field - 126)
+    const int shift = 27 - (int)max(big >> 23, 1u);
+    const double base = pr_base(a);   // (ends with a barrier)
+    const bool fixed = (double)__uint_as_float(big) <= kPbSpread * base, heavy = b.kind == kPbHeavy;
+    double sum = 0;                   // a heavy row's (id 0; the padding has another)
+    auto add = [&](uint32_t at, float x) {
+        if (heavy) sum += at == 0 ? (double)x : 0.0;
+        else if (fixed) atomicAdd(&acc[at], pb_fixed(x, shift));
+        else atomicAdd((double*)&acc[at], (double)x);
+    };
+    constexpr int U = 4;
+    const uint32_t end = 2 * (b.o + b.octs);
+    for (uint32_t o = 2 * b.o + threadIdx.x; o < end; o += U * kPbBlock) {
+        uint32_t q[U];
+        ushort4 d[U];
+        float4 x[U];
+#pragma unroll
+        for (int j = 0; j < U; j++) {
+            const uint32_t at = min(o + j * kPbBlock, end - 1);
+            q[j] = 2 * pos[at >> 1] + (at & 1);
+            d[j] = dst[at];
+        }
+#pragma unroll
+        for (int j = 0; j < U; j++) x[j] = vals[q[j]];
+#pragma unroll
+        for (int j = 0; j < U; j++) {
+            if (o + j * kPbBlock >= end) continue;
+            add(d[j].x, x[j].x);
+            add(d[j].y, x[j].y);
+            add(d[j].z, x[j].z);
+            add(d[j].w, x[j].w);
+        }
     }
     __syncthreads();
-    const double base = pr_base(a);
-    double res = 0, dang = 0;
-    for (uint32_t i = threadIdx.x; i < kPbBin; i += kPbBlock) {
-        const uint64_t v = (uint64_t)b * kPbBin + i;
-        if (v >= a.V || (uint64_t)(off[v + 1] - off[v]) >= a.heavy_thr) continue;
-        pr_finish_vertex(a, v, (double)acc[i], base, res, dang);
+    // a unit is 2^(field - 126 - 51)
+    const double unit = ldexp(1.0, 27 - shift - 177);
+    PrSums sums;
+    if (heavy) {
+        __shared__ double s_sum[kPbBlock / kWave];
+        sum = wave_sum(sum);
+        if (lane_id() == 0) s_sum[wave_id()] = sum;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            for (int i = 1; i < kPbBlock / kWave; i++) sum += s_sum[i];
+            pr_finish_vertex(a, b.v, sum, base, sums);
+        }
     }
-    acc_add<kPbBlock>(res, dang, a.acc_out);
+    for (uint32_t i = threadIdx.x; !heavy && i < b.n; i += kPbBlock) {
+        if (b.kind == kPbAround && off[b.v + i + 1] - off[b.v + i] >= kRowsLong) continue;
+        pr_finish_vertex(a, b.v + i, fixed ? (double)acc[i] * unit : __longlong_as_double((long long)acc[i]), base, sums);
+    }
+    acc_add<kPbBlock>(sums, a.acc_out);
 }
 
 // ---- source-segmented normalised mode --------------------------------------
@@ -864,7 +1062,7 @@ __global__ __launch_bounds__(kTlBlock) void k_pr_tiled(PrArgs a, const uint32_t*
     const uint32_t nb = blockIdx.x < ts.nd ? (ts.nd - blockIdx.x + G - 1) / G : 0;   // blocks of this workgroup
     const uint32_t dsz = 1u << ts.db, smask = (1u << ts.sb) - 1;
     const double base = pr_base(a);
-    double res = 0, dang = 0;
+    PrSums sums;
     for (uint32_t r = 0; r < nb; r++) {
         const uint64_t d = blockIdx.x + (uint64_t)r * G;
         for (uint32_t i = threadIdx.x; i < dsz; i += kTlBlock) acc[i] = 0.0f;
@@ -918,11 +1116,11 @@ __global__ __launch_bounds__(kTlBlock) void k_pr_tiled(PrArgs a, const uint32_t*
             const uint64_t v = v0 + i;
             if (v >= a.V) break;
             if (heavy_bits && (heavy_bits[v >> 5] >> (v & 31) & 1u)) continue;
-            pr_finish_vertex(a, v, (double)acc[i], base, res, dang);
+            pr_finish_vertex(a, v, (double)acc[i], base, sums);
         }
         __syncthreads();
     }
-    acc_add<kTlBlock>(res, dang, a.acc_out);
+    acc_add<kTlBlock>(sums, a.acc_out);
 }
 
 // ---- reference mode --------------------------------------------------------
@@ -1072,27 +1270,22 @@ __global__ void k_prref_publish(uint32_t* count, PrRefPub* host, unsigned long l
 
 constexpr int kRefRing = 4;   // published iterations of the reference mode
 
-// Cuts the resident vertices into row blocks and lists their heavy rows, once
-// per graph.
+// Lists the heavy rows of the resident vertices, once per graph.
 template <class OffT>
-static int pr_rows_build(asc_graph* g, PrState* p) {
-    if (p->rows_built) return ASC_OK;
+static int pr_heavy_build(asc_graph* g, PrState* p) {
+    if (p->heavy_built) return ASC_OK;
     const uint64_t n = g->static_vertices;
     const uint64_t cap = std::min<uint64_t>(n, g->static_edges / kRowsHeavy) + 1;
-    const uint64_t bcap = std::min<uint64_t>(n, (n + kBlock - 1) / kBlock + g->static_edges / kRowsWindow + cap) + 1;
     hipStream_t s = g->ctx->s_main;
     DevTmp<uint32_t> d_cnt;
-    uint32_t cnt[3] = {0, 0, 0};
+    uint32_t cnt[2] = {0, 0};
     if (!p->rows_heavy) ASC_HIP(hipMalloc(&p->rows_heavy, 4 * cap));
-    if (!p->rows_blocks) ASC_HIP(hipMalloc(&p->rows_blocks, sizeof(RowBlock) * bcap));
     ASC_HIP(hipMalloc(&d_cnt.p, sizeof(cnt)));
     ASC_HIP(hipMemsetAsync(d_cnt.p, 0, sizeof(cnt), s));
     if (n) {
         const int grid = (int)std::min<uint64_t>((n + kBlock - 1) / kBlock, (uint64_t)g->ctx->num_cus * 8);
         hipLaunchKernelGGL((k_rows_heavy_list<OffT>), dim3(grid), dim3(kBlock), 0, s, (const OffT*)g->d_off, n,
                            p->rows_heavy, (uint32_t)cap, d_cnt.p);
-        hipLaunchKernelGGL((k_row_blocks<OffT>), dim3(grid), dim3(kBlock), 0, s, (const OffT*)g->d_off, n,
-                           (RowBlock*)p->rows_blocks, d_cnt.p + 2);
         ASC_HIP(hipGetLastError());
     }
     ASC_HIP(hipMemcpyAsync(cnt, d_cnt.p, sizeof(cnt), hipMemcpyDeviceToHost, s));
@@ -1100,7 +1293,33 @@ static int pr_rows_build(asc_graph* g, PrState* p) {
     p->rows_cap = (uint32_t)cap;
     p->rows_front = cnt[0];
     p->rows_back = cnt[1];
-    p->rows_n = cnt[2];
+    p->heavy_built = true;
+    return ASC_OK;
+}
+
+// Cuts the resident vertices into row blocks too, once per graph.
+template <class OffT>
+static int pr_rows_build(asc_graph* g, PrState* p) {
+    ASC_TRY(pr_heavy_build<OffT>(g, p));
+    if (p->rows_built) return ASC_OK;
+    const uint64_t n = g->static_vertices;
+    const uint64_t bcap = std::min<uint64_t>(n, (n + kBlock - 1) / kBlock + g->static_edges / kRowsWindow +
+                                                    p->rows_cap) + 1;
+    hipStream_t s = g->ctx->s_main;
+    DevTmp<uint32_t> d_cnt;
+    uint32_t cnt = 0;
+    if (!p->rows_blocks) ASC_HIP(hipMalloc(&p->rows_blocks, sizeof(RowBlock) * bcap));
+    ASC_HIP(hipMalloc(&d_cnt.p, sizeof(cnt)));
+    ASC_HIP(hipMemsetAsync(d_cnt.p, 0, sizeof(cnt), s));
+    if (n) {
+        const int grid = (int)std::min<uint64_t>((n + kBlock - 1) / kBlock, (uint64_t)g->ctx->num_cus * 8);
+        hipLaunchKernelGGL((k_row_blocks<OffT>), dim3(grid), dim3(kBlock), 0, s, (const OffT*)g->d_off, n,
+                           (RowBlock*)p->rows_blocks, d_cnt.p);
+        ASC_HIP(hipGetLastError());
+    }
+    ASC_HIP(hipMemcpyAsync(&cnt, d_cnt.p, sizeof(cnt), hipMemcpyDeviceToHost, s));
+    ASC_HIP(hipStreamSynchronize(s));
+    p->rows_n = cnt;
     p->rows_built = true;
     return ASC_OK;
 }
@@ -1188,86 +1407,176 @@ static int launch_pull(int G, int num_cus, hipStream_t s, const PrArgs& a, const
     return ASC_OK;
 }
 
-// Builds the propagation-blocked slot layout once (every edge resident,
-// E < 2^32, at most kPbMaxBins bins, slot arrays within free device memory);
-// pb_state = -1 when it cannot be built.
-template <class OffT>
-static int pr_blocked_build(asc_graph* g, PrState* p) {
-    if (p->pb_state != 0) return ASC_OK;
-    p->pb_state = -1;
-    const uint64_t V = g->h.V, E = g->h.E;
-    const uint64_t nb = (V + kPbBin - 1) / kPbBin;
-    if (g->static_vertices != V || E == 0 || E >= 0xFFFFFFFFull || nb > kPbMaxBins) return ASC_OK;
-    const bool sym = g->symmetric == 1;
-    size_t free_b = 0, total_b = 0;
-    ASC_HIP(hipMemGetInfo(&free_b, &total_b));
-    const uint64_t keep = E * (4 + 4 + 2 + 4) + 12 * (uint64_t)kPbRanges * nb;
-    const uint64_t temp = 8 * (uint64_t)kPbRanges * nb + 8 * (V + 1) + (sym ? 0 : 4 * E + 8 * (V + 1));
-    if (keep + temp + (uint64_t(1) << 30) > free_b) return ASC_OK;
-    hipStream_t s = g->ctx->s_main;
-    const int grid = g->ctx->num_cus * 8;
-    const OffT* in_off = (const OffT*)g->d_off;
-    // out-CSR: the in-CSR itself when symmetric, else a transpose
-    HostBuf<uint64_t> h_out;
-    ASC_TRY(h_out.alloc(V + 1));
-    h_out[0] = 0;
-    for (uint64_t u = 0; u < V; u++) h_out[u + 1] = h_out[u] + g->h.outdeg[u];
-    if (h_out[V] != E) {
-        set_last_error("out-degrees sum to %llu, not E = %llu", (unsigned long long)h_out[V], (unsigned long long)E);
+// ASC_PR_BLOCKED asked for by name refuses out-degrees that do not sum to E.
+static int pr_check_outdeg(const asc_graph* g, PrState* p) {
+    if (p->outdeg_sums) return ASC_OK;
+    std::atomic<uint64_t> sum{0};
+    host_pool().parallel_for(g->h.V, [&](uint64_t b, uint64_t e) {
+        uint64_t x = 0;
+        for (uint64_t u = b; u < e; u++) x += g->h.outdeg[u];
+        sum += x;
+    });
+    if (sum != g->h.E) {
+        set_last_error("out-degrees sum to %llu, not E = %llu", (unsigned long long)sum.load(),
+                       (unsigned long long)g->h.E);
         return ASC_ERR_FORMAT;
     }
-    // set-up temporaries (freed on every return): out-offsets, the transpose
-    // of a directed graph and its fill cursors, the slot counts
-    DevTmp<unsigned long long> d_out_off, cursor;
-    DevTmp<uint32_t> transposed, d_cnt;
-    ASC_HIP(hipMalloc(&d_out_off.p, 8 * (V + 1)));
-    ASC_HIP(hipMemcpy(d_out_off.p, h_out.p, 8 * (V + 1), hipMemcpyHostToDevice));
-    const uint32_t* out_dst = (const uint32_t*)g->d_edges;
-    if (!sym) {
-        ASC_HIP(hipMalloc(&transposed.p, 4 * E));
-        ASC_HIP(hipMalloc(&cursor.p, 8 * (V + 1)));
-        ASC_HIP(hipMemcpyAsync(cursor.p, d_out_off.p, 8 * (V + 1), hipMemcpyDeviceToDevice, s));
-        hipLaunchKernelGGL((k_pb_transpose<OffT>), dim3(grid), dim3(kBlock), 0, s, in_off,
-                           (const uint32_t*)g->d_edges, V, cursor.p, transposed.p);
-        ASC_HIP(hipGetLastError());
-        ASC_HIP(hipStreamSynchronize(s));
-        out_dst = transposed.p;
-    }
-    ASC_HIP(hipMalloc(&p->pb_src, 4 * E));
-    hipLaunchKernelGGL((k_pb_src<unsigned long long>), dim3(grid), dim3(kBlock), 0, s, d_out_off.p, V, p->pb_src);
-    ASC_HIP(hipGetLastError());
-    // slot layout: counts per (bin, range), exclusive scan in bin-major order
-    const uint32_t thr = kRowsLong;
-    ASC_HIP(hipMalloc(&d_cnt.p, 4 * (size_t)kPbRanges * nb));
-    hipLaunchKernelGGL((k_pb_count<OffT>), dim3(std::min<uint32_t>(kPbRanges, grid)), dim3(kBlock), 0, s, out_dst, E,
-                       in_off, thr, (uint32_t)nb, d_cnt.p);
-    ASC_HIP(hipGetLastError());
-    std::vector<uint32_t> cnt((size_t)kPbRanges * nb);
-    ASC_HIP(hipMemcpyAsync(cnt.data(), d_cnt.p, 4 * cnt.size(), hipMemcpyDeviceToHost, s));
-    ASC_HIP(hipStreamSynchronize(s));
-    // range-major slots: the regions of one source range are adjacent, so
-    // the scatter of a range writes one contiguous stretch
-    std::vector<unsigned long long> base(cnt.size());
-    unsigned long long acc = 0;
-    for (uint32_t r = 0; r < kPbRanges; r++)
-        for (uint64_t b = 0; b < nb; b++) {
-            base[b * kPbRanges + r] = acc;
-            acc += cnt[b * kPbRanges + r];
+    p->outdeg_sums = true;
+    return ASC_OK;
+}
+
+// Smallest graph of the blocked schedule under ASC_PR_AUTO.
+// Below, the row blocks' gathers come out of the L2s and two launches an
+// iteration on few workgroups cost more (ms of 20 iterations, blocked / row
+// blocks: R-MAT scale 18, 7.6e6 edges 0.91 / 0.80, Erdos-Renyi V = 2^18, 8.4e6
+// edges 0.66 / 1.07, V = 2^17, 1.7e7 edges 0.85 / 1.82); from V = 2^20 on the
+// lines hold however few the edges (V = 2^20, 4.2e6 edges: 0.53 / 0.96, R-MAT
+// 0.86 / 0.79).
+constexpr uint64_t kPbMinV = uint64_t(1) << 17, kPbMinE = uint64_t(1) << 23;
+
+// Builds the propagation-blocked layout once (every edge resident, at most
+// kPbMaxSlices slices, fewer than 2^31 octs, its arrays within free device
+// memory); pb_state = -1 when it cannot be built.
+template <class OffT>
+static int pr_blocked_build(asc_graph* g, PrState* p, bool by_name) {
+    if (p->pb_state != 0) return ASC_OK;
+    const uint64_t V = g->h.V, E = g->h.E;
+    const uint32_t cus = (uint32_t)g->ctx->num_cus;
+    const uint64_t most = std::max<uint64_t>(1u << 16, E / (8 * (uint64_t)cus));   // edges of a bin
+    // 2^14 sources a slice and 2^13 destinations a bin: 64 KB of LDS each, two
+    // workgroups a CU (V = 2^23, 2^28 edges: 14.7 ms for 20 iterations, also
+    // with 2^15 sources, 15.0 with 2^14 destinations; R-MAT scale 20: 2.20,
+    // 2.26, 2.57).  Larger ones where runs would be shorter than 64 edges;
+    // AUTO leaves graphs with less than 16 a run to the tiled pull.
+    uint32_t bits = 14, dbits = 13;
+    auto runs_of = [&] { return ((V >> bits) + 1) * (std::max(V >> dbits, E / most) + 1); };
+    if (E / 64 < runs_of()) bits = 15;
+    if (E / 64 < runs_of()) dbits = 14;
+    if (!by_name && E / 16 < runs_of()) return ASC_OK;
+    p->pb_state = -1;
+    const uint64_t ns = (V + (1ull << bits) - 1) >> bits;
+    if (g->static_vertices != V || E == 0 || E >= 0xFFFFFFFFull || V > (uint64_t(1) << 28) || ns > kPbMaxSlices)
+        return ASC_OK;
+    hipStream_t s = g->ctx->s_main;
+    const OffT* off = (const OffT*)g->d_off;
+    const uint32_t* src = (const uint32_t*)g->d_edges;
+    // rows left to the pull, in order
+    std::vector<uint32_t> heavy(p->rows_front);
+    if (p->rows_front)
+        ASC_HIP(hipMemcpy(heavy.data(), p->rows_heavy, 4 * heavy.size(), hipMemcpyDeviceToHost));
+    std::sort(heavy.begin(), heavy.end());
+    const uint64_t* ho = g->h.off.p;
+    std::vector<PbBin> bins;
+    for (uint32_t v : heavy) bins.push_back({v, 1, 0, 0, kPbHeavy});
+    size_t nh = 0;
+    for (uint64_t v = 0; v < V;) {
+        const uint64_t lim = std::min<uint64_t>(V, v + (1ull << dbits));
+        uint64_t left = most, at = v;   // (a row that is not heavy always fits an empty bin)
+        uint32_t kind = kPbPlain;
+        while (at < lim) {
+            if (nh < heavy.size() && heavy[nh] == at) {
+                kind = kPbAround;
+                nh++;
+                at++;
+                continue;
+            }
+            const uint64_t seg = nh < heavy.size() ? std::min<uint64_t>(lim, heavy[nh]) : lim;
+            const uint64_t* e = std::upper_bound(ho + at + 1, ho + seg + 1, ho[at] + left);
+            const uint64_t v1 = (uint64_t)(e - ho) - 1;
+            left -= ho[v1] - ho[at];
+            at = v1;
+            if (at < seg) break;
         }
-    ASC_HIP(hipMalloc(&p->pb_bin_start, 8 * base.size()));   // region bases, [b * R + r]
-    ASC_HIP(hipMemcpy(p->pb_bin_start, base.data(), 8 * base.size(), hipMemcpyHostToDevice));
-    ASC_HIP(hipMalloc(&p->pb_cnt, 4 * cnt.size()));
-    ASC_HIP(hipMemcpy(p->pb_cnt, cnt.data(), 4 * cnt.size(), hipMemcpyHostToDevice));
-    ASC_HIP(hipMalloc(&p->pb_pos, 4 * E));
-    ASC_HIP(hipMalloc(&p->pb_dl, 2 * std::max<unsigned long long>(acc, 1)));
-    ASC_HIP(hipMalloc(&p->pb_vals, 4 * std::max<unsigned long long>(acc, 1)));
-    hipLaunchKernelGGL((k_pb_assign<OffT>), dim3(std::min<uint32_t>(kPbRanges, grid)), dim3(kBlock), 0, s, out_dst,
-                       E, in_off, thr, (uint32_t)nb, p->pb_bin_start, p->pb_pos, p->pb_dl);
+        bins.push_back({(uint32_t)v, (uint32_t)(at - v), 0, 0, kind});
+        v = at;
+    }
+    const uint64_t nb = bins.size();
+    size_t free_b = 0, total_b = 0;
+    ASC_HIP(hipMemGetInfo(&free_b, &total_b));
+    const uint64_t padded = E + (kPbOct - 1) * nb * ns;
+    if (nb == 0 || padded / kPbOct >= (uint64_t(1) << 31) || 9 * padded + 16 * nb * ns + (uint64_t(1) << 30) > free_b) return ASC_OK;
+    DevTmp<uint32_t> d_cnt;
+    ASC_HIP(hipMalloc(&d_cnt.p, 4 * nb * ns));
+    ASC_HIP(hipMalloc(&p->pb_bins, sizeof(PbBin) * nb));
+    ASC_HIP(hipMemcpyAsync(p->pb_bins, bins.data(), sizeof(PbBin) * nb, hipMemcpyHostToDevice, s));
+    hipLaunchKernelGGL((k_pb_count<OffT>), dim3((uint32_t)nb), dim3(kPbBlock), 0, s, off, src,
+                       (const PbBin*)p->pb_bins, (uint32_t)ns, bits, d_cnt.p);
     ASC_HIP(hipGetLastError());
+    DevTmp<uint32_t> d_first;   // octs of the slices, then of the bins; then where they begin
+    ASC_HIP(hipMalloc(&d_first.p, 4 * (ns + nb)));
+    hipLaunchKernelGGL(k_pb_totals<true>, dim3((uint32_t)ns), dim3(kBlock), 0, s, d_cnt.p, (uint32_t)nb, (uint32_t)ns,
+                       d_first.p);
+    hipLaunchKernelGGL(k_pb_totals<false>, dim3((uint32_t)nb), dim3(kBlock), 0, s, d_cnt.p, (uint32_t)nb, (uint32_t)ns,
+                       d_first.p + ns);
+    ASC_HIP(hipGetLastError());
+    std::vector<uint32_t> first(ns + nb);
+    ASC_HIP(hipMemcpyAsync(first.data(), d_first.p, 4 * first.size(), hipMemcpyDeviceToHost, s));
     ASC_HIP(hipStreamSynchronize(s));
+    // slice order: a slice's runs one after the other, bin by bin
+    uint64_t octs = 0;
+    for (uint64_t i = 0; i < ns; i++) octs += first[i];
+    const uint64_t per = std::min<uint64_t>(kPbItemOcts, std::max<uint64_t>(octs / (2 * (uint64_t)cus), 1u << 11));
+    std::vector<PbItem> items;
+    uint32_t at = 0;
+    for (uint64_t i = 0; i < ns; i++) {
+        const uint32_t end = at + first[i];
+        first[i] = at;
+        for (uint64_t q = at; q < end; q += per)
+            items.push_back({(uint32_t)i, (uint32_t)q, (uint32_t)std::min<uint64_t>(end, q + per)});
+        at = end;
+    }
+    at = 0;
+    for (uint64_t b = 0; b < nb; b++) {
+        bins[b].o = at;
+        bins[b].octs = first[ns + b];
+        first[ns + b] = at;
+        at += bins[b].octs;
+    }
+    const uint64_t q1 = std::max<uint64_t>(octs, 1);
+    DevTmp<PbRun> d_runs;
+    ASC_HIP(hipMalloc(&d_runs.p, sizeof(PbRun) * nb * ns));
+    ASC_HIP(hipMemcpyAsync(d_first.p, first.data(), 4 * first.size(), hipMemcpyHostToDevice, s));
+    ASC_HIP(hipMemcpyAsync(p->pb_bins, bins.data(), sizeof(PbBin) * nb, hipMemcpyHostToDevice, s));
+    hipLaunchKernelGGL(k_pb_place<true>, dim3((uint32_t)ns), dim3(kBlock), 0, s, d_cnt.p, (uint32_t)nb, (uint32_t)ns,
+                       d_first.p, d_runs.p);
+    hipLaunchKernelGGL(k_pb_place<false>, dim3((uint32_t)nb), dim3(kBlock), 0, s, d_cnt.p, (uint32_t)nb, (uint32_t)ns,
+                       d_first.p + ns, d_runs.p);
+    ASC_HIP(hipGetLastError());
+    ASC_HIP(hipMalloc(&p->pb_items, sizeof(PbItem) * std::max<size_t>(items.size(), 1)));
+    if (!items.empty())
+        ASC_HIP(hipMemcpyAsync(p->pb_items, items.data(), sizeof(PbItem) * items.size(), hipMemcpyHostToDevice, s));
+    ASC_HIP(hipMalloc(&p->pb_src, sizeof(PbIds) * q1));
+    ASC_HIP(hipMalloc(&p->pb_dst, sizeof(PbIds) * q1));
+    ASC_HIP(hipMalloc(&p->pb_pos, 4 * q1));
+    ASC_HIP(hipMalloc(&p->pb_vals, 4 * kPbOct * q1));
+    // the padding's places: source 0 of the slice, the sum past the bin's.  The
+    // ids are written in pairs first (the values' array holds them meanwhile):
+    // two arrays of scattered 2-byte writes took twice as long
+    hipLaunchKernelGGL(k_pr_fill, dim3(cus * 8), dim3(256), 0, s, (uint32_t*)p->pb_vals, kPbOct * q1,
+                       1u << (dbits + 16));
+    hipLaunchKernelGGL((k_pb_fill<OffT>), dim3((uint32_t)nb), dim3(kPbBlock), 0, s, off, src,
+                       (const PbBin*)p->pb_bins, d_runs.p, (uint32_t)ns, bits, (uint32_t*)p->pb_vals);
+    hipLaunchKernelGGL(k_pb_unzip, dim3((uint32_t)nb), dim3(kPbBlock), 0, s, d_runs.p, (uint32_t)ns,
+                       (const uint4*)p->pb_vals, (PbIds*)p->pb_src, (PbIds*)p->pb_dst, p->pb_pos);
+    ASC_HIP(hipGetLastError());
+    ASC_HIP(hipStreamSynchronize(s));   // the host arrays above are read until here
+    p->pb_sbits = bits;
+    p->pb_dbits = dbits;
     p->pb_nbins = (uint32_t)nb;
-    p->pb_edges = E;
+    p->pb_nitems = (uint32_t)items.size();
     p->pb_state = 1;
+    return ASC_OK;
+}
+
+template <class OffT, int SB, int DB>
+static int launch_blocked(const PrArgs& a, const PrState* p, hipStream_t s) {
+    if (p->pb_nitems)
+        hipLaunchKernelGGL(k_pb_scatter<SB>, dim3((p->pb_nitems + 7) / 8 * 8), dim3(kPbBlock), 0, s, a.contrib_in,
+                           a.V, (const PbItem*)p->pb_items, p->pb_nitems, (const ushort4*)p->pb_src,
+                           (float4*)p->pb_vals);
+    hipLaunchKernelGGL((k_pb_gather<OffT, DB>), dim3(p->pb_nbins), dim3(kPbBlock), 0, s, a, (const PbBin*)p->pb_bins,
+                       p->pb_pos, (const ushort4*)p->pb_dst, (const float4*)p->pb_vals);
+    ASC_HIP(hipGetLastError());
     return ASC_OK;
 }
 
@@ -1340,19 +1649,23 @@ static int pr_normalised(asc_graph* g, const asc_pr_opts* o, float* rank_out, do
     const uint64_t V = g->h.V;
     hipStream_t s = ctx->s_main;
     const int grid = ctx->num_cus * 8;
-    ASC_TRY(pr_rows_build<OffT>(g, p));
+    ASC_TRY(pr_heavy_build<OffT>(g, p));
     auto slot = [&](int it) { return p->acc + (size_t)(it % kAccSlots) * kAccSlot; };
     ASC_HIP(hipMemsetAsync(p->acc, 0, sizeof(double) * kAccSlots * kAccSlot, s));
     hipLaunchKernelGGL(k_pr_init, dim3(std::max<uint64_t>(1, std::min<uint64_t>((V + kBlock - 1) / kBlock, (uint64_t)grid))), dim3(kBlock), 0,
                        s, p->rank[0], p->contrib[0], g->d_outdeg, V, slot(0));
     ASC_HIP(hipGetLastError());
     const int G = g->pr_group > 0 ? g->pr_group : 0;
-    if (o->method == ASC_PR_BLOCKED) ASC_TRY(pr_blocked_build<OffT>(g, p));
-    const bool blocked = o->method == ASC_PR_BLOCKED && p->pb_state == 1;
+    const bool by_name = o->method == ASC_PR_BLOCKED;
+    const bool big = o->method == ASC_PR_AUTO && g->static_vertices == V && V >= (uint64_t(1) << 20);
+    const bool blocks = by_name || big || (o->method == ASC_PR_AUTO && !G && V >= kPbMinV && g->h.E >= kPbMinE);
+    if (blocks) ASC_TRY(pr_blocked_build<OffT>(g, p, by_name));
+    const bool blocked = blocks && p->pb_state == 1;
     if (o->method == ASC_PR_BLOCKED && !blocked) {
         set_last_error("propagation-blocked PageRank needs every edge resident, E < 2^32 and room for its slots");
         return ASC_ERR_UNSUPPORTED;
     }
+    if (o->method == ASC_PR_BLOCKED) ASC_TRY(pr_check_outdeg(g, p));
     // tile shape: 2^15-vertex segments (128 KB contribution slices) measured
     // fastest on Erdos-Renyi 2^26 / 2^31 edges (20 iterations: 496 ms with
     // 2^14-vertex blocks against 557-833 ms for 2^14 or 2^16-2^20-vertex
@@ -1365,15 +1678,15 @@ static int pr_normalised(asc_graph* g, const asc_pr_opts* o, float* rank_out, do
     const uint32_t db_auto = (V >> 15) >= 4 * (uint64_t)ctx->num_cus ? 15u : 14u;
     const uint32_t db = o->tile_dst_bits > 0 ? (uint32_t)o->tile_dst_bits
                         : g->pr_tile_dst_bits > 0 ? (uint32_t)g->pr_tile_dst_bits : db_auto;
-    // AUTO: the tiled pull once the contributions outgrow an XCD's L2
-    const bool want_tiled = o->method == ASC_PR_TILED ||
-                            (o->method == ASC_PR_AUTO && g->static_vertices == V && V >= (uint64_t(1) << 20));
+    // AUTO: the tiled pull where the blocked layout cannot be built
+    const bool want_tiled = o->method == ASC_PR_TILED || (big && !blocked);
     if (want_tiled) ASC_TRY(pr_tiled_build<OffT>(g, p, sb, db));
     const bool tiled = want_tiled && p->tl_state == 1;
     if (o->method == ASC_PR_TILED && !tiled) {
         set_last_error("source-segmented PageRank needs every edge resident, V <= 2^31 and room for its tiles");
         return ASC_ERR_UNSUPPORTED;
     }
+    if (!tiled && !blocked && !G) ASC_TRY(pr_rows_build<OffT>(g, p));
     const double t0 = now_ms();
     ASC_HIP(hipEventRecord(p->ev[0], s));
     for (int it = 0; it < iters; it++) {
@@ -1419,18 +1732,16 @@ static int pr_normalised(asc_graph* g, const asc_pr_opts* o, float* rank_out, do
             ASC_HIP(hipGetLastError());
             led();
         } else if (blocked) {
-            hipLaunchKernelGGL(k_pb_scatter, dim3(grid), dim3(kBlock), 0, s, p->pb_src, p->pb_pos, p->pb_edges,
-                               a.contrib_in, p->pb_vals);
-            hipLaunchKernelGGL((k_pb_gather<OffT>), dim3(p->pb_nbins), dim3(kPbBlock), 0, s, a, p->pb_bin_start,
-                               p->pb_cnt, p->pb_dl, p->pb_vals);
-            ASC_HIP(hipGetLastError());
+            if (p->pb_dbits == 14) ASC_TRY((launch_blocked<OffT, 15, 14>(a, p, s)));
+            else if (p->pb_sbits == 15) ASC_TRY((launch_blocked<OffT, 15, 13>(a, p, s)));
+            else ASC_TRY((launch_blocked<OffT, 14, 13>(a, p, s)));
             led();
         } else if (a.v_end > 0) {
             ASC_TRY(launch_pull<OffT>(G, ctx->num_cus, s, a, p));
             led();
         }
         // rows of kRowsLong edges and more (the row kernel takes them itself)
-        if (p->rows_front && (tiled || blocked || G)) {
+        if (p->rows_front && (tiled || (G && !blocked))) {
             hipLaunchKernelGGL((k_pr_pull_heavy<OffT>), dim3(std::min<uint32_t>(p->rows_front, grid)), dim3(kBlock), 0,
                                s, a, p->rows_heavy, p->rows_front);
             ASC_HIP(hipGetLastError());

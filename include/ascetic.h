@@ -367,13 +367,15 @@ typedef struct {
 
 /* Normalised PageRank schedule (asc_pr_opts.method). */
 typedef enum {
-    ASC_PR_AUTO = 0,     /* ASC_PR_TILED when every edge is resident and
-                            V >= 2^20 (contributions larger than an XCD's
-                            L2), else the pull                              */
-    ASC_PR_PULL = 1,     /* G-lane pull over the in-CSR                      */
-    ASC_PR_BLOCKED = 2,  /* propagation-blocked (scatter to slots by
-                            destination bin, LDS sums per bin); needs every
-                            edge resident, else ASC_ERR_UNSUPPORTED         */
+    ASC_PR_AUTO = 0,     /* ASC_PR_BLOCKED when every edge is resident and
+                            V >= 2^20, or V >= 2^17 with 2^23 edges and no
+                            pr_group set; ASC_PR_TILED where V >= 2^20 and
+                            the blocked layout does not fit; else the pull  */
+    ASC_PR_PULL = 1,     /* pull over the in-CSR                             */
+    ASC_PR_BLOCKED = 2,  /* propagation-blocked (scatter by slices of sources,
+                            LDS sums per bin of destinations); needs every
+                            edge resident, else ASC_ERR_UNSUPPORTED, and
+                            out-degrees that sum to E, else ASC_ERR_FORMAT  */
     ASC_PR_TILED = 3     /* source-segmented: in-edges regrouped once into
                             (destination block, source segment) tiles, a
                             workgroup sums one block in LDS while walking
