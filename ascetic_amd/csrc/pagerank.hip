@@ -171,9 +171,6 @@ constexpr uint32_t kRowsWindow = 1536;
 constexpr uint32_t kRowsHeavy = 512;
 static_assert(kRowsWindow + kRowsHeavy <= kRowsTile, "a row block is one tile");
 constexpr uint32_t kRowsLong = 4096;    // rows summed by a whole workgroup, started before all others
-constexpr int kSeqPer = 4;              // a heavy row's pass of the reference mode
-constexpr int kSeqTile = kBlock * kSeqPer;
-static_assert(2 * kSeqTile <= kRowsTile, "two passes share the row tile's LDS");
 constexpr int kPrLines = 16;            // counters spread over this many 128-byte lines
 constexpr int kPrLineWords = 32;
 
@@ -190,36 +187,6 @@ __device__ __forceinline__ double add_in_order(double s, const T* x, uint32_t n)
     }
     for (; k < n; k++) s += (double)x[k];
     return s;
-}
-
-// The same for a long stretch: 16 values are read while the 16 before them
-// are added (two register sets, so nothing is copied, and a scheduling fence
-// so that the reads are not moved behind the adds), and the chain waits for
-// its adds alone.
-__device__ __forceinline__ double add_chain(double s, const double* x, uint32_t n) {
-    constexpr uint32_t B = 16;
-    uint32_t k = 0;
-    if (n >= 3 * B) {
-        double y[B], z[B];
-#pragma unroll
-        for (uint32_t j = 0; j < B; j++) y[j] = x[j];
-        for (; k + 3 * B <= n; k += 2 * B) {
-#pragma unroll
-            for (uint32_t j = 0; j < B; j++) z[j] = x[k + B + j];
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (uint32_t j = 0; j < B; j++) s += y[j];
-#pragma unroll
-            for (uint32_t j = 0; j < B; j++) y[j] = x[k + 2 * B + j];
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (uint32_t j = 0; j < B; j++) s += z[j];
-        }
-#pragma unroll
-        for (uint32_t j = 0; j < B; j++) s += y[j];
-        k += B;
-    }
-    return add_in_order<8>(s, x + k, n - k);
 }
 
 // Sums the rows of at most 256 vertices [base, end) of any length (streamed
@@ -1168,16 +1135,268 @@ __device__ __forceinline__ uint32_t prref_finish(const PrRefArgs& a, uint64_t v,
     return 0;
 }
 
+// What a stretch of a sequential FP64 sum adds to the running sum s while s
+// stays in its binade, whose numbers are multiples of u: `a` if s is an even
+// multiple, a + d * u if it is an odd one.  A term rounds to a whole number of
+// units whatever s is, unless it lies halfway between two: then to the one that
+// leaves s even.  All sums of units here are exact, and a sum that leaves the
+// binade stays outside whatever is added (nothing added is negative).
+struct Ordered {
+    double a;
+    int d;
+    __device__ __forceinline__ double added(double s, double u) const {
+        return __double_as_longlong(s) & 1 ? a + d * u : a;
+    }
+    // this stretch, then the next; base: the binade's first number, even
+    __device__ __forceinline__ Ordered then(const Ordered& b, double base, double u) const {
+        const double even = base + a, odd = base + u + (a + d * u);
+        const double x = a + b.added(even, u), y = (a + d * u) + b.added(odd, u);
+        return Ordered{x, y > x ? 1 : y < x ? -1 : 0};
+    }
+};
+
+// A term c >= 0.
+__device__ __forceinline__ Ordered ordered_term(double c, double base, double u) {
+    const double r = (base + c) - base, e = c - r;
+    return Ordered{r, fabs(e) == 0.5 * u ? (e > 0 ? 1 : -1) : 0};
+}
+
+constexpr int kOrdPer = 8;                       // terms a lane holds
+constexpr uint32_t kOrdWave = kWave * kOrdPer;   // terms a wave holds
+constexpr int kOrdBlock = kBlock;
+static_assert(kBlock * kOrdPer <= kRowsTile, "the rows' LDS has room");
+
+// The state of an ordered sum's binade.
+struct Binade {
+    double base, u, top;
+    int e;
+    __device__ __forceinline__ explicit Binade(double s) {
+        e = (int)((unsigned long long)__double_as_longlong(s) >> 52);
+        base = __longlong_as_double((long long)e << 52);
+        u = __longlong_as_double((long long)max(e - 52, 0) << 52);
+        top = base + base;
+    }
+    __device__ __forceinline__ bool tiny() const { return e < 64; }     // zero, or too small for units
+    __device__ __forceinline__ bool huge() const { return e >= 2046; }  // next to infinity, or negative
+};
+
+// Inclusive sum over the wave by lane moves within the vector unit (__shfl_up
+// goes through LDS, six times one after the other).
+__device__ __forceinline__ double wave_scan_dpp(double x) {
+#define ASC_STEP(ctrl, rows)                                                                                    \
+    {                                                                                                           \
+        const long long b = __double_as_longlong(x);                                                            \
+        const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)b, ctrl, rows, 0xf, false);           \
+        const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(b >> 32), ctrl, rows, 0xf, false);   \
+        x += __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));                            \
+    }
+    ASC_STEP(0x111, 0xf)   // row_shr:1
+    ASC_STEP(0x112, 0xf)
+    ASC_STEP(0x114, 0xf)
+    ASC_STEP(0x118, 0xf)
+    ASC_STEP(0x142, 0xa)   // row_bcast:15
+    ASC_STEP(0x143, 0xc)   // row_bcast:31
+#undef ASC_STEP
+    return x;
+}
+
+// The terms of the lanes from `skip` on, summed from the wave's first lane.
+__device__ __forceinline__ Ordered ordered_scan(const double (&c)[kOrdPer], bool mine, const Binade& n) {
+    Ordered x{0, 0};
+    bool tie = false;
+#pragma unroll
+    for (int j = 0; j < kOrdPer; j++) {
+        const Ordered t = ordered_term(c[j], n.base, n.u);
+        x.a += t.a;
+        tie |= t.d != 0;
+    }
+    if (!mine) {
+        x.a = 0;
+        tie = false;
+    }
+    if (!wave_ballot(tie)) {
+        x.a = wave_scan_dpp(x.a);
+        return x;
+    }
+    if (tie) {
+        x = ordered_term(c[0], n.base, n.u);
+#pragma unroll
+        for (int j = 1; j < kOrdPer; j++) x = x.then(ordered_term(c[j], n.base, n.u), n.base, n.u);
+    }
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) {
+        const Ordered y{__shfl_up(x.a, d, kWave), __shfl_up(x.d, d, kWave)};
+        if (lane_id() >= (uint32_t)d) x = y.then(x, n.base, n.u);
+    }
+    return x;
+}
+
+__device__ __forceinline__ double add_own(double s, const double (&c)[kOrdPer]) {
+#pragma unroll
+    for (int j = 0; j < kOrdPer; j++) s += c[j];
+    return s;
+}
+
+__device__ __forceinline__ bool ordered_terms(const double (&c)[kOrdPer]) {
+    bool ok = true;
+#pragma unroll
+    for (int j = 0; j < kOrdPer; j++) ok &= ((unsigned long long)__double_as_longlong(c[j]) >> 52) < 2047;
+    return ok;   // neither negative, infinite nor NaN
+}
+
+// s + c[0] + c[1] + ... in this order, each sum rounded to FP64: lane t of the
+// wave holds terms 8t to 8t + 7.  All lanes round their terms to units of s at
+// once and a scan adds them; where the sum leaves its binade that lane adds
+// its terms one by one, and the lanes behind it go on in the new units.
+__device__ __forceinline__ double add_ordered_wave(double s, const double (&c)[kOrdPer]) {
+    const uint32_t lane = lane_id();
+    uint32_t skip = 0, small = 0;
+    if (!wave_ballot(!ordered_terms(c))) {
+        while (skip < (uint32_t)kWave) {
+            const Binade n(s);
+            if (n.huge()) break;
+            if (n.tiny()) {
+                // the first terms of a row, in which the sum doubles often, or zeros
+                if (++small > 4) break;
+                for (const uint32_t to = min(skip + 8, (uint32_t)kWave); skip < to; skip++)
+                    s = __shfl(add_own(s, c), skip, kWave);
+                continue;
+            }
+            const Ordered x = ordered_scan(c, lane >= skip, n);
+            const double F = s + x.added(s, n.u);
+            const uint64_t out = wave_ballot(F >= n.top);
+            if (!out) return __shfl(F, kWave - 1, kWave);
+            const uint32_t first = (uint32_t)__builtin_ctzll(out);
+            const double before = __shfl_up(F, 1, kWave);
+            s = __shfl(add_own(lane ? before : s, c), first, kWave);
+            skip = first + 1;
+        }
+    }
+    for (; skip < (uint32_t)kWave; skip++) s = __shfl(add_own(s, c), skip, kWave);
+    return s;
+}
+
+struct OrderedLds {
+    double a[2][kOrdBlock / kWave];
+    int d[2][kOrdBlock / kWave];
+    double s;
+    uint32_t skip;
+};
+
+// The same over a workgroup of kOrdBlock lanes.
+__device__ __forceinline__ double add_ordered_block(double s, const double (&c)[kOrdPer], OrderedLds& l,
+                                                    uint32_t& round) {
+    constexpr uint32_t W = kOrdBlock / kWave;
+    const uint32_t tid = threadIdx.x, lane = lane_id(), w = wave_id();
+    bool units = !__syncthreads_or(!ordered_terms(c));
+    uint32_t skip = 0, small = 0;
+    while (skip < (uint32_t)kOrdBlock) {
+        const Binade n(s);
+        units = units && !n.huge() && !(n.tiny() && ++small > 4);
+        if (!units || n.tiny()) {   // eight lanes, one after the other
+            const uint32_t to = min(skip + 8, (skip / kWave + 1) * kWave);
+            __syncthreads();
+            if (w == skip / kWave) {
+                for (uint32_t i = skip; i < to; i++) s = __shfl(add_own(s, c), i % kWave, kWave);
+                if (lane == 0) l.s = s;
+            }
+            __syncthreads();
+            s = l.s;
+            skip = to;
+            continue;
+        }
+        const Ordered x = ordered_scan(c, tid >= skip, n);
+        const uint32_t buf = round++ & 1;
+        if (lane == kWave - 1) {
+            l.a[buf][w] = x.a;
+            l.d[buf][w] = x.d;
+        }
+        __syncthreads();
+        double S = s, in = s;     // after the waves so far; before this wave
+        uint32_t out = W;         // the wave in which the sum leaves its binade
+#pragma unroll
+        for (uint32_t i = 0; i < W; i++) {
+            if (i == w) in = S;
+            const double F = S + Ordered{l.a[buf][i], l.d[buf][i]}.added(S, n.u);
+            if (F >= n.top) out = min(out, i);
+            S = F;
+        }
+        if (out == W) return S;
+        if (w == out) {
+            const double F = in + x.added(in, n.u);
+            const double before = __shfl_up(F, 1, kWave);
+            const uint32_t first = (uint32_t)__builtin_ctzll(wave_ballot(F >= n.top));
+            if (lane == first) {
+                l.s = add_own(lane ? before : in, c);
+                l.skip = tid + 1;
+            }
+        }
+        __syncthreads();
+        s = l.s;
+        skip = l.skip;
+    }
+    return s;
+}
+
+// The in-sum of the row [b, e) by `waves` waves, this one the w-th.  While a
+// tile is added (add(s, c)) the contributions of the next are gathered and the
+// ids of the one after loaded.  Neighbouring lanes gather neighbouring edges
+// (sources ascend along a row, so they share lines: with eight edges a lane
+// R-MAT scale 20 took 461 us an iteration), and s_val, kOrdWave values of the
+// wave's own, turns them into eight terms a lane.
+template <class Add>
+__device__ __forceinline__ double pull_ordered(const uint32_t* src, const double* contrib, uint64_t b, uint64_t e,
+                                               uint32_t w, uint32_t waves, double* s_val, Add add) {
+    const uint32_t lane = lane_id();
+    const uint64_t tile = (uint64_t)waves * kOrdWave;
+    uint32_t u[kOrdPer];
+    double c0[kOrdPer], c1[kOrdPer];
+    b += w * kOrdWave;   // (of this wave from here on)
+    auto load_ids = [&](uint64_t t0) {
+#pragma unroll
+        for (int j = 0; j < kOrdPer; j++) u[j] = src[min(t0 + j * kWave + lane, e - 1)];
+    };
+    auto gather = [&](double (&c)[kOrdPer], uint64_t t0) {
+#pragma unroll
+        for (int j = 0; j < kOrdPer; j++) c[j] = t0 + j * kWave + lane < e ? contrib[u[j]] : 0.0;
+    };
+    auto turn = [&](double (&c)[kOrdPer]) {
+#pragma unroll
+        for (int j = 0; j < kOrdPer; j++) s_val[j * kWave + lane] = c[j];
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int j = 0; j < kOrdPer; j++) c[j] = s_val[lane * kOrdPer + j];
+        __builtin_amdgcn_wave_barrier();
+    };
+    double s = 0;
+    load_ids(b);
+    gather(c0, b);
+    load_ids(b + tile);
+    for (uint64_t t0 = b;; t0 += 2 * tile) {
+        gather(c1, t0 + tile);
+        load_ids(t0 + 2 * tile);
+        turn(c0);
+        s = add(s, c0);
+        if (t0 - w * kOrdWave + tile >= e) break;
+        gather(c0, t0 + 2 * tile);
+        load_ids(t0 + 3 * tile);
+        turn(c1);
+        s = add(s, c1);
+        if (t0 - w * kOrdWave + 2 * tile >= e) break;
+    }
+    return s;
+}
+
 // One iteration over [v_begin, v_end): prSumKernel_static / _dynamic
 // (gpu_kernels.cuh:554-594) and prKernel_Opt.  The result must equal a
-// sequential FP64 sum in CSR order, so a row is one chain of adds and the
-// longest row bounds an iteration; everything else is kept off that chain.
-// The first `hb` workgroups take the heavy rows, the longest first: 2048
-// contributions a pass are gathered by all lanes, then added by one lane out
-// of LDS while the next pass's gathers are in flight.  The other workgroups
-// run pull_block.  R-MAT scale 20 (31 M in-edges, longest row 64.8 k): 24.4 ms
-// an iteration with one thread per row loading and adding edge by edge, 0.43
-// ms this way, all of it the longest row's chain (6.6 ns an add).
+// sequential FP64 sum in CSR order.  The first `hb` workgroups take the heavy
+// rows with ordered sums, the longest first and a workgroup each, the others a
+// wave each; the other workgroups run pull_block, where a lane adds a row.
+// R-MAT scale 20 (31 M in-edges, longest row 64.6 k): 24.4 ms an iteration
+// with one thread per row loading and adding edge by edge, 0.43 ms with one
+// lane adding a heavy row out of LDS (6.6 ns an add), 0.29 ms this way, most
+// of it the gathers of 8-byte contributions (8.4 MB, twice an XCD's L2).
+// Launch bounds for more waves spill: 0.50 ms.
 template <class OffT, bool HEAVY>
 __global__ __launch_bounds__(kBlock) void k_prref_rows(PrRefArgs a, uint32_t hb) {
     __shared__ double s_val[kRowsTile];
@@ -1187,41 +1406,28 @@ __global__ __launch_bounds__(kBlock) void k_prref_rows(PrRefArgs a, uint32_t hb)
     const uint32_t tid = threadIdx.x;
     uint32_t moved = 0;
     if (HEAVY && blockIdx.x < hb) {
-        for (uint32_t i = blockIdx.x; i < a.rows.n_front + a.rows.n_back; i += hb) {
-            const uint32_t v = i < a.rows.n_front ? a.rows.front(i) : a.rows.back(i - a.rows.n_front);
-            if (!a.active[v]) continue;   // the same for the whole workgroup: only its own lane 0 clears it, below
-            const OffT b = off[v], e = off[v + 1];
-            // pass t: the ids of pass t + 2 are loaded and the contributions
-            // of pass t + 1 gathered (by the ids loaded a pass ago) while
-            // pass t is added, so that no wave waits for either
-            uint32_t u[kSeqPer];
-            double c[kSeqPer];
-            auto load_ids = [&](OffT t0) {
-#pragma unroll
-                for (int j = 0; j < kSeqPer; j++) u[j] = src[min((OffT)(t0 + j * kBlock + tid), (OffT)(e - 1))];
-            };
-            auto gather = [&] {
-#pragma unroll
-                for (int j = 0; j < kSeqPer; j++) c[j] = a.contrib_in[u[j]];
-            };
-            load_ids(b);
-            gather();
-            load_ids(b + kSeqTile);
-            double s = 0;
-            uint32_t half = 0;   // passes alternate between two halves of s_val: one barrier each
-            __syncthreads();     // the previous row's adds are done
-            for (OffT t0 = b; t0 < e; t0 += kSeqTile, half ^= 1) {
-                double* buf = s_val + half * kSeqTile;
-#pragma unroll
-                for (int j = 0; j < kSeqPer; j++) buf[j * kBlock + tid] = c[j];
-                __syncthreads();
-                if (e - t0 > kSeqTile) {
-                    gather();
-                    load_ids(t0 + 2 * kSeqTile);
-                }
-                if (tid == 0) s = add_chain(s, buf, (uint32_t)min((OffT)kSeqTile, (OffT)(e - t0)));
+        // the longest rows, a workgroup each
+        __shared__ OrderedLds s_ord;
+        uint32_t round = 0;
+        const uint32_t lb = min(a.rows.n_front, hb / 2);
+        if (blockIdx.x < lb) {
+            for (uint32_t i = blockIdx.x; i < a.rows.n_front; i += lb) {
+                const uint32_t v = a.rows.front(i);
+                if (!a.active[v]) continue;   // the same for the whole workgroup: only its own lane 0 clears it, below
+                const double s = pull_ordered(src, a.contrib_in, off[v], off[v + 1], wave_id(), kWavesPerBlock,
+                                              s_val + wave_id() * kOrdWave, [&](double s, const double (&c)[kOrdPer]) {
+                                                  return add_ordered_block(s, c, s_ord, round);
+                                              });
+                if (tid == 0) moved += prref_finish(a, v, s);
             }
-            if (tid == 0) moved += prref_finish(a, v, s);
+        }
+        else for (uint32_t i = (blockIdx.x - lb) * kWavesPerBlock + wave_id(); i < a.rows.n_back; i += (hb - lb) * kWavesPerBlock) {
+            const uint32_t v = a.rows.back(i);
+            if (!a.active[v]) continue;   // the same for the whole wave: only its own lane 0 clears it, below
+            const double s = pull_ordered(src, a.contrib_in, off[v], off[v + 1], 0, 1,
+                                          s_val + wave_id() * kOrdWave,
+                                          [](double s, const double (&c)[kOrdPer]) { return add_ordered_wave(s, c); });
+            if (lane_id() == 0) moved += prref_finish(a, v, s);
         }
     } else {
         const uint32_t bid = blockIdx.x - (HEAVY ? hb : 0), nblk = gridDim.x - (HEAVY ? hb : 0);
@@ -1840,9 +2046,11 @@ static int pr_reference(asc_graph* g, const asc_pr_opts* o, double* rank_out, as
             a.src = (const uint32_t*)g->d_edges;
             a.v_end = g->static_vertices;
             a.rows = row_plan(p);
-            const uint32_t hb = std::min<uint32_t>(p->rows_front + p->rows_back, (uint32_t)grid / 2);
+            const uint32_t hb = std::min<uint32_t>(
+                p->rows_front + (p->rows_back + kWavesPerBlock - 1) / kWavesPerBlock + 1, (uint32_t)grid / 2);
             const uint32_t rb = std::min<uint32_t>(p->rows_n, (uint32_t)grid);
-            hipLaunchKernelGGL((k_prref_rows<OffT, true>), dim3(hb + rb), dim3(kBlock), 0, s, a, hb);
+            if (hb + rb)
+                hipLaunchKernelGGL((k_prref_rows<OffT, true>), dim3(hb + rb), dim3(kBlock), 0, s, a, hb);
             ASC_HIP(hipGetLastError());
         }
         ASC_TRY(pr_stream_chunks(g, p, [&](const uint32_t* src, uint64_t e0, uint64_t v0, uint64_t v1) {
