@@ -28,7 +28,7 @@ __device__ __forceinline__ uint32_t candidate(uint32_t sv, uint32_t w) {
 // relax_commit_batch decides from it and performs the atomics.
 template <int ALGO, class OffT, class EdgeT>
 __device__ __forceinline__ uint32_t relax_probe(const TravArgs<OffT, EdgeT>& a, uint32_t v) {
-    if (ALGO == ALG_BFS) return a.visited[v >> 5];
+    if (ALGO == ALG_BFS) return a.seen8 ? 0u - (uint32_t)a.seen8[v] : a.visited[v >> 5];
     if (ALGO == ALG_SSSP && a.val16) {
         // 0xFFFF: nothing known (not lowered yet, or a value beyond 16 bits),
         // so the atomic is tried
@@ -46,9 +46,12 @@ constexpr int kUnroll = 4;
 // is set).  BFS: a vertex whose visited bit is clear is claimed by an atomic
 // OR of that bit and gets its level; SSSP/CC: a candidate below the probed
 // value is offered by atomicMin, and a vertex it lowers is routed once per
-// step (a far candidate to the far pile, a static vertex to the resident
-// frontier, an on-demand one to the pile) by an atomicMax on the matching
-// stamp.  The value atomics of all edges are issued before any result is
+// step (a static vertex to the resident frontier, an on-demand one to the
+// pile) by an atomicMax on the matching stamp.  A far candidate puts its vertex
+// into the far pile if it is the first to reach it: a value at or above theta
+// was at or above every earlier theta, so a vertex that had one is there
+// already (a stamp for it was every second atomic of a step of R-MAT scale 22,
+// whose steps take 0.1 to 0.17 ns an atomic).  The value atomics of all edges are issued before any result is
 // used, then the stamp atomics of those that improved, so each lane waits for
 // two atomic round trips per pass instead of two per edge.
 template <int ALGO, class OffT, class EdgeT>
@@ -69,7 +72,9 @@ __device__ __forceinline__ void relax_commit_batch(const TravArgs<OffT, EdgeT>& 
     if (ALGO == ALG_BFS) {
 #pragma unroll
         for (int j = 0; j < kUnroll; j++) {
-            if (!try_[j] || (old[j] & (1u << (v[j] & 31)))) continue;
+            if (!try_[j]) continue;
+            if (a.seen8) a.seen8[v[j]] = 1;
+            if (old[j] & (1u << (v[j] & 31))) continue;
             a.val[v[j]] = cand[j];
             to[j] = v[j] < a.vs ? TO_RES : TO_PEND;
         }
@@ -81,13 +86,14 @@ __device__ __forceinline__ void relax_commit_batch(const TravArgs<OffT, EdgeT>& 
 #pragma unroll
     for (int j = 0; j < kUnroll; j++) {
         kind[j] = TO_NONE;
-        if (!try_[j] || old[j] <= cand[j]) continue;
-        if (ALGO == ALG_SSSP && a.val16 && cand[j] < 0xFFFFu) a.val16[v[j]] = (uint16_t)cand[j];
+        if (!try_[j]) continue;
+        if (ALGO == ALG_SSSP && a.val16 && min(old[j], cand[j]) < 0xFFFFu) a.val16[v[j]] = (uint16_t)min(old[j], cand[j]);
+        if (old[j] <= cand[j]) continue;
         if (ALGO == ALG_SSSP && cand[j] >= a.theta) {
-            sp[j] = a.fstamp + v[j];
-            sv[j] = a.fepoch;
-            kind[j] = TO_FAR;
-        } else if (v[j] < a.vs) {
+            if (old[j] == a.unreached) to[j] = TO_FAR;
+            continue;
+        }
+        if (v[j] < a.vs) {
             sp[j] = a.stamp + v[j];
             sv[j] = level + 1;
             kind[j] = TO_RES;
@@ -121,30 +127,79 @@ __device__ __forceinline__ void add_claimed(unsigned long long* dst, unsigned lo
     if (lane_id() == 0 && m) atomicAdd(dst, m);
 }
 
+// Staging entries of a wave for the resident frontier and the far pile, the
+// queues that a step may push millions of entries to.
+constexpr int kQueueCap = 256;
+
+template <int ALGO>
+struct PushLds {
+    uint32_t res[kWavesPerBlock][kQueueCap];
+    uint32_t pend[kWavesPerBlock][kStageCap];
+    uint32_t far[kWavesPerBlock][ALGO == ALG_SSSP ? kQueueCap : 1];
+    uint32_t n[3][kWavesPerBlock], at[3];
+};
+
 template <int ALGO>
 struct Pushes {
-    WaveStage<kStageCap> res, pend, far;
+    WaveStage<kQueueCap> res;
+    WaveStage<kStageCap> pend;
+    WaveStage<kQueueCap> far;
+    PushLds<ALGO>& lds;
+
+    __device__ __forceinline__ explicit Pushes(PushLds<ALGO>& l)
+        : res{l.res[wave_id()], 0}, pend{l.pend[wave_id()], 0}, far{l.far[wave_id()], 0}, lds(l) {}
 
     template <class A>
-    __device__ __forceinline__ void push(const A& a, Slot* nxt, int to, uint32_t v) {
-        res.push(to == TO_RES, v, a.q_out, &nxt->n_res);
+    __device__ __forceinline__ void push(const A& a, uint32_t* q, uint32_t* q_count, int to, uint32_t v) {
+        res.push(to == TO_RES, v, q, q_count);
         pend.push(to == TO_PEND, v, a.pend_out, a.pend_count);
         if (ALGO == ALG_SSSP) far.push(to == TO_FAR, v, a.far_out, a.far_count);
     }
+    // The rest of the four waves, called by the whole workgroup.  One atomic a
+    // queue: atomics on one address take 9 ns each, so one a wave cost every
+    // step of a full grid up to 74 us a queue (R-MAT scale 22 SSSP, 27 steps:
+    // 6.5 -> 5.8 ms).
     template <class A>
-    __device__ __forceinline__ void flush(const A& a, Slot* nxt) {
-        res.flush(a.q_out, &nxt->n_res);
-        pend.flush(a.pend_out, a.pend_count);
-        if (ALGO == ALG_SSSP) far.flush(a.far_out, a.far_count);
+    __device__ __forceinline__ void flush(const A& a, uint32_t* q, uint32_t* q_count) {
+        const uint32_t w = wave_id();
+        if (lane_id() == 0) {
+            lds.n[0][w] = res.n;
+            lds.n[1][w] = pend.n;
+            lds.n[2][w] = far.n;
+        }
+        __syncthreads();
+        if (threadIdx.x < 3) {
+            uint32_t all = 0;
+            for (int i = 0; i < kWavesPerBlock; i++) all += lds.n[threadIdx.x][i];
+            uint32_t* count = threadIdx.x == 0 ? q_count : threadIdx.x == 1 ? a.pend_count : a.far_count;
+            if (all) lds.at[threadIdx.x] = atomicAdd(count, all);
+        }
+        __syncthreads();
+        auto copy = [&](int k, const uint32_t* buf, uint32_t n, uint32_t* to) {
+            uint32_t at = lds.at[k];
+            for (uint32_t i = 0; i < w; i++) at += lds.n[k][i];
+            for (uint32_t j = lane_id(); j < n; j += kWave) to[at + j] = buf[j];
+        };
+        copy(0, res.buf, res.n, q);
+        copy(1, pend.buf, pend.n, a.pend_out);
+        if (ALGO == ALG_SSSP) copy(2, far.buf, far.n, a.far_out);
     }
 };
 
-#define ASC_STAGE_DECL                                              \
-    __shared__ uint32_t s_stage[3][kWavesPerBlock][kStageCap];      \
-    Pushes<ALGO> pq{{s_stage[0][wave_id()], 0}, {s_stage[1][wave_id()], 0}, {s_stage[2][wave_id()], 0}}
+#define ASC_STAGE_DECL                        \
+    __shared__ PushLds<ALGO> s_stage;         \
+    Pushes<ALGO> pq(s_stage)
+
+// Vertices a workgroup takes per pass of expand_local_body: 256, halved down to
+// kPassMin while every workgroup still gets kPassShare passes or the frontier
+// is too small to give each one.  A frontier of a few ten thousand R-MAT
+// vertices has hundreds of edges each: 256 a pass left most CUs idle (directed
+// scale 22 BFS, 94 k vertices: 1009 us, 666 this way; 16 and 64 vertices, one
+// and four passes differ by 2 %).
+constexpr uint32_t kPassMin = 16, kPassShare = 2;
 
 // Expansion of the resident frontier (slot level % 4) by workgroup `bid` of
-// `nblk`: 256 frontier vertices at a time, their edges walked edge-balanced;
+// `nblk`: up to 256 frontier vertices at a time, their edges walked edge-balanced;
 // vertices with degree >= heavy_thr go to the heavy list instead.  Called by
 // k_expand_local and by persistent kernels (with their own block numbering).
 template <int ALGO, class OffT, class EdgeT>
@@ -167,12 +222,14 @@ __device__ __forceinline__ void expand_local_body(const TravArgs<OffT, EdgeT>& a
     const uint32_t n = cur->n_res;
     const uint32_t tid = threadIdx.x, lane = lane_id(), w = wave_id();
     unsigned long long my_edges = 0, my_verts = 0, m_claimed = 0;
+    uint32_t per = kBlock;   // vertices a pass
+    while (per > kPassMin && (uint64_t)per * nblk * kPassShare > n) per >>= 1;
 
-    for (uint32_t base = bid * kBlock; base < n; base += nblk * kBlock) {
+    for (uint32_t base = bid * per; base < n; base += nblk * per) {
         const uint32_t i = base + tid;
         uint32_t deg = 0, sv = 0;
         OffT beg = 0;
-        if (i < n) {
+        if (tid < per && i < n) {
             const uint32_t u = a.q_in[i];
             beg = a.off[u];
             uint64_t d = (uint64_t)(a.off[u + 1] - beg);
@@ -199,7 +256,7 @@ __device__ __forceinline__ void expand_local_body(const TravArgs<OffT, EdgeT>& a
         s_beg[tid] = beg;
         s_sv[tid] = sv;
         __syncthreads();
-        const uint32_t cnt = min(n - base, (uint32_t)kBlock);
+        const uint32_t cnt = min(n - base, per);
         for (uint32_t eb = w * kWave * kUnroll; eb < total; eb += kBlock * kUnroll) {
             uint32_t kk[kUnroll], vv[kUnroll], cc[kUnroll], pr[kUnroll];
             EdgeT ed[kUnroll];
@@ -228,14 +285,14 @@ __device__ __forceinline__ void expand_local_body(const TravArgs<OffT, EdgeT>& a
             int to[kUnroll];
             relax_commit_batch<ALGO>(a, vv, cc, pr, valid, level, to);
 #pragma unroll
-            for (int j = 0; j < kUnroll; j++) pq.push(a, nxt, to[j], vv[j]);
+            for (int j = 0; j < kUnroll; j++) pq.push(a, a.q_out, &nxt->n_res, to[j], vv[j]);
             if (ALGO == ALG_BFS && a.m_next) m_claimed += claimed_degrees(a, to, vv);
         }
         my_edges += total;
         my_verts += cnt;
         __syncthreads();
     }
-    pq.flush(a, nxt);
+    pq.flush(a, a.q_out, &nxt->n_res);
     if (ALGO == ALG_BFS && a.m_next) add_claimed(a.m_next, m_claimed);
     if (tid == 0 && my_verts) {
         atomicAdd(&a.stats->edges_local, my_edges);
@@ -333,13 +390,13 @@ __device__ __forceinline__ void expand_heavy_body(const TravArgs<OffT, EdgeT>& a
             int to[kUnroll];
             relax_commit_batch<ALGO>(a, vv, cc, pr, valid, level, to);
 #pragma unroll
-            for (int j = 0; j < kUnroll; j++) pq.push(a, nxt, to[j], vv[j]);
+            for (int j = 0; j < kUnroll; j++) pq.push(a, a.q_out, &nxt->n_res, to[j], vv[j]);
             if (ALGO == ALG_BFS && a.m_next) m_claimed += claimed_degrees(a, to, vv);
         }
         my_edges += tlen;
         __syncthreads();
     }
-    pq.flush(a, nxt);
+    pq.flush(a, a.q_out, &nxt->n_res);
     if (ALGO == ALG_BFS && a.m_next) add_claimed(a.m_next, m_claimed);
     if (tid == 0 && my_edges) atomicAdd(&a.stats->edges_heavy, my_edges);
 }

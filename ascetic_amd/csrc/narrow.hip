@@ -224,12 +224,11 @@ __global__ __launch_bounds__(kNwBlock) void k_narrow(TravArgs<OffT, EdgeT> a, Na
             // the atomics of the edges that lower something, and beside them
             // the offsets of the vertices they lower
             OffT b[U], e1[U];
-            uint32_t old[U], st[U];
+            uint32_t old[U];
 #pragma unroll
             for (int j = 0; j < U; j++) {
                 const uint32_t v = vv[j];
                 old[j] = BFS ? ~0u : 0u;
-                st[j] = a.fepoch;
                 b[j] = e1[j] = 0;
                 if (!ok[j]) continue;
                 if (BFS) {
@@ -237,11 +236,6 @@ __global__ __launch_bounds__(kNwBlock) void k_narrow(TravArgs<OffT, EdgeT> a, Na
                                      : atomicOr(a.visited + (v >> 5), 1u << (v & 31));
                 } else {
                     old[j] = atomicMin(a.val + v, cc[j]);
-                    // a far candidate enters the pile whether it lowers v after
-                    // all or not, once per vertex and run: an entry already
-                    // expanded at its value is dropped by the next split.  (One
-                    // above V lowers nothing: an unreached v would stay pending.)
-                    if (ALGO == ALG_SSSP && cc[j] >= theta && cc[j] <= na.V) st[j] = atomicMax(a.fstamp + v, a.fepoch);
                 }
                 b[j] = a.off[v];
                 e1[j] = a.off[v + 1];
@@ -255,11 +249,13 @@ __global__ __launch_bounds__(kNwBlock) void k_narrow(TravArgs<OffT, EdgeT> a, Na
                     push(level + 1, v, 0, b[j], (uint64_t)(e1[j] - b[j]));
                     continue;
                 }
-                if (ALGO == ALG_SSSP && st[j] < a.fepoch)
-                    nw_store(na.far[fcur] + atomicAdd(&s_nfar[fcur], 1u), v);
                 if (old[j] <= cc[j]) continue;
                 // (the 16-bit value filter is left as it is: an older entry is larger)
-                if (ALGO == ALG_SSSP && cc[j] >= theta) continue;
+                if (ALGO == ALG_SSSP && cc[j] >= theta) {
+                    // a vertex reached before is in the pile
+                    if (old[j] == a.unreached) nw_store(na.far[fcur] + atomicAdd(&s_nfar[fcur], 1u), v);
+                    continue;
+                }
                 if (e1[j] > b[j]) push(level + 1, v, cc[j], b[j], (uint64_t)(e1[j] - b[j]));
             }
         };

@@ -613,7 +613,7 @@ static int run_bfs_do(asc_graph* g, uint32_t src, uint32_t* out, asc_stats* st) 
             rc.node_sum += nf;
             a.q_in = t->q[level & 1];
             a.q_out = t->q[(level + 1) & 1];
-            const int lgrid = (int)std::max<uint64_t>(1, std::min<uint64_t>(grid, (nf + kBlock - 1) / kBlock));
+            const int lgrid = (int)std::max<uint64_t>(1, std::min<uint64_t>(grid, (nf + kPassMin - 1) / kPassMin));
             ASC_TRY(timed_launch(t, prof, KERN_LOCAL, s, [&] {
                 hipLaunchKernelGGL((k_expand_local<ALG_BFS, OffT, EdgeT>), dim3(lgrid), dim3(kBlock), 0, s, a, level);
             }));

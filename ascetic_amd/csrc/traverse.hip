@@ -166,13 +166,13 @@ __global__ __launch_bounds__(kBlock) void k_expand_part(TravArgs<OffT, EdgeT> a,
             int to[kUnroll];
             relax_commit_batch<ALGO>(a, vv, cc, pr, valid, level, to);
 #pragma unroll
-            for (int j = 0; j < kUnroll; j++) pq.push(a, nxt, to[j], vv[j]);
+            for (int j = 0; j < kUnroll; j++) pq.push(a, a.q_out, &nxt->n_res, to[j], vv[j]);
         }
         my_edges += tlen;
         my_verts += m;
         __syncthreads();
     }
-    pq.flush(a, nxt);
+    pq.flush(a, a.q_out, &nxt->n_res);
     if (tid == 0 && my_edges) {
         atomicAdd(SRC == PART_HOST ? &a.stats->edges_part_host : &a.stats->edges_part, my_edges);
         atomicAdd(SRC == PART_HOST ? &a.stats->verts_part_host : &a.stats->verts_part, my_verts);
@@ -373,7 +373,7 @@ __global__ __launch_bounds__(kBlock) void k_scan_apply(const uint32_t* x, uint32
 
 // Moves the far pile's entries whose value fell below theta into the current
 // frontier (resident) or the on-demand pile; the rest stays far.  A vertex
-// enters the far pile once per run (its far stamp stays set): a value that
+// enters the far pile once per run (when it is first reached): a value that
 // falls below theta is expanded in the band and can only fall further, and a
 // value that stays above is read again from the one entry at the next split,
 // so kept entries are copied without a stamp atomic.
@@ -384,30 +384,34 @@ __global__ __launch_bounds__(kBlock) void k_split_far(TravArgs<OffT, EdgeT> a, c
     ASC_STAGE_DECL;
     Slot* slot = a.slots + (level & 3);
     uint32_t lmin = 0xFFFFFFFFu;
-    for (uint32_t base = blockIdx.x * kBlock; base < n; base += gridDim.x * kBlock) {
-        const uint32_t i = base + threadIdx.x;
-        int to = TO_NONE;
-        uint32_t v = 0;
-        if (i < n) {
-            v = far_in[i];
-            const uint32_t d = a.val[v];
-            if (d >= a.theta) {
+    constexpr int U = 4;   // entries of a lane whose values are read together
+    for (uint64_t base = blockIdx.x * (uint64_t)kBlock; base < n; base += (uint64_t)gridDim.x * kBlock * U) {
+        uint32_t v[U], d[U];
+        bool in[U];
+#pragma unroll
+        for (int j = 0; j < U; j++) {
+            const uint64_t i = base + (uint64_t)j * gridDim.x * kBlock + threadIdx.x;
+            in[j] = i < n;
+            v[j] = far_in[in[j] ? i : 0];
+        }
+#pragma unroll
+        for (int j = 0; j < U; j++) d[j] = a.val[v[j]];
+#pragma unroll
+        for (int j = 0; j < U; j++) {
+            int to = TO_NONE;
+            if (in[j] && d[j] >= a.theta) {
                 // a vertex is expanded only below the band of its round and
                 // bands only rise, so done[v] < theta here: still pending
                 to = TO_FAR;
-                lmin = min(lmin, d);
-            } else if (a.done[v] != d) {
-                if (v < a.vs) to = atomicMax(a.stamp + v, level) < level ? TO_RES : TO_NONE;
-                else to = atomicMax(a.pstamp + v, a.pepoch) < a.pepoch ? TO_PEND : TO_NONE;
+                lmin = min(lmin, d[j]);
+            } else if (in[j] && a.done[v[j]] != d[j]) {
+                if (v[j] < a.vs) to = atomicMax(a.stamp + v[j], level) < level ? TO_RES : TO_NONE;
+                else to = atomicMax(a.pstamp + v[j], a.pepoch) < a.pepoch ? TO_PEND : TO_NONE;
             }
+            pq.push(a, q_level, &slot->n_res, to, v[j]);
         }
-        pq.res.push(to == TO_RES, v, q_level, &slot->n_res);
-        pq.pend.push(to == TO_PEND, v, a.pend_out, a.pend_count);
-        pq.far.push(to == TO_FAR, v, a.far_out, a.far_count);
     }
-    pq.res.flush(q_level, &slot->n_res);
-    pq.pend.flush(a.pend_out, a.pend_count);
-    pq.far.flush(a.far_out, a.far_count);
+    pq.flush(a, q_level, &slot->n_res);
 #pragma unroll
     for (int d = kWave / 2; d > 0; d >>= 1) lmin = min(lmin, (uint32_t)__shfl_xor(lmin, d, kWave));
     if (lane_id() == 0 && lmin != 0xFFFFFFFFu) atomicMin(&piles->min_far, lmin);
@@ -460,7 +464,7 @@ __global__ __launch_bounds__(kBlock) void k_run_init(RunInit a) {
     const uint64_t i0 = blockIdx.x * (uint64_t)kBlock + threadIdx.x, step = (uint64_t)gridDim.x * kBlock;
     if (a.val)
         for (uint64_t i = i0; i < a.V; i += step) a.val[i] = i == a.src ? 1u : a.unreached;
-    for (uint32_t* z : {a.stamp, a.pstamp, a.fstamp})
+    for (uint32_t* z : {a.stamp, a.pstamp})
         if (z)
             for (uint64_t i = i0; i < a.V; i += step) z[i] = 0;
     if (a.done)
@@ -469,6 +473,8 @@ __global__ __launch_bounds__(kBlock) void k_run_init(RunInit a) {
         for (uint64_t i = i0; i < (a.V + 31) / 32; i += step) a.visited[i] = i == a.src >> 5 ? 1u << (a.src & 31) : 0u;
     if (a.val16)
         for (uint64_t i = i0; i < (a.V + 1) / 2; i += step) a.val16[i] = 0xFFFFFFFFu;
+    if (a.seen8)
+        for (uint64_t i = i0; i < (a.V + 3) / 4; i += step) a.seen8[i] = 0;
     if (blockIdx.x != 0) return;
     uint32_t* st = (uint32_t*)a.stats;
     for (uint32_t i = threadIdx.x; i < sizeof(DevStats) / 4; i += kBlock) st[i] = 0;
@@ -583,6 +589,7 @@ void trav_free(TravState* t) {
         if (p) (void)hipFree(p);
     };
     f(t->val16);
+    f(t->seen8);
     for (int i = 0; i < 2; i++) f(t->pend[i]);
     for (int i = 0; i < kMaxPartBufs; i++) f(t->part[i]);
     f(t->od_list); f(t->od_prefix); f(t->scan_tmp); f(t->d_ch_v); f(t->d_ch_edges); f(t->d_ch_count); f(t->d_ch_dense);
@@ -721,7 +728,7 @@ int trav_ensure_relax(asc_graph* g) {
     const uint64_t V = g->h.V;
     t->mem_relax.parts.clear();
     t->mem_relax.bytes = 0;
-    for (uint32_t** p : {&t->stamp, &t->pstamp, &t->fstamp, &t->done, &t->far[0], &t->far[1]})
+    for (uint32_t** p : {&t->stamp, &t->pstamp, &t->done, &t->far[0], &t->far[1]})
         t->mem_relax.add(p, V);
     return t->mem_relax.alloc();
 }
@@ -773,9 +780,21 @@ static bool sssp_filter_pays(asc_graph* g) {
 
 // Bands of a narrow run, in wide bands: a small step costs its memory round
 // trips whatever its size, so wider bands trade re-expansions for fewer steps
-// (1201 x 1033 mesh, weights 1-255, in wide bands of 32: 39.6 ms at 2, 33.3 at
-// 4, 30.8 at 8, 30.4 at 16, 33.0 at 32).
-constexpr uint32_t kNarrowBands = 8;
+// (1201 x 1033 mesh, weights 1-255, narrow bands of 64: 39.6 ms, of 128 33.3,
+// of 256 30.8, of 512 30.4, of 1024 33.0; wide ones are 15).
+constexpr uint32_t kNarrowBands = 16;
+
+// A split reads the whole far pile, whatever it takes out of it.  Where a band
+// expanded fewer than kBandShare times as many vertices as the pile holds (the
+// tail of a run on skewed graphs), the next is kBandGrow times as wide: R-MAT
+// scale 22 needs 2 to 3 splits instead of 9 (3.9 -> 2.9 ms), scale 18 1.12 ->
+// 0.76, with no edge relaxed more; 1 and 2 instead of 4: 3.26 and 3.08 ms.
+constexpr uint64_t kBandShare = 4, kBandGrow = 4;
+
+// Smallest resident graph whose BFS steps probe bytes (TravArgs::seen8)
+// instead of the visited bits (directed R-MAT, bits / bytes: scale 17 309 / 321
+// us, scale 20 627 / 534, scale 22 1265 / 955, scale 24 3553 / 3071).
+constexpr uint64_t kSeenMinV = uint64_t(1) << 18;
 
 static uint32_t sssp_delta(asc_graph* g) {
     if (g->sssp_delta > 0) return (uint32_t)g->sssp_delta;
@@ -787,8 +806,12 @@ static uint32_t sssp_delta(asc_graph* g) {
     // re-expansions wide bands cause; measured: R-MAT scale 24, weights 1-64,
     // 6 to 30 times the mean weight equal, 2 times 5% slower; scale 28,
     // weights 1-255, 12 times 7% faster than 6); fully resident ones narrow
-    // bands (fewer re-expansions; a step costs only a launch and a sync)
-    const double f = g->static_vertices == g->h.V ? 0.25 : 12.0;
+    // bands (fewer re-expansions; a step costs only a launch and a sync, and
+    // bands grow once they cost more than they take: kBandShare).  0.25, 0.12
+    // and 0.06 of the mean: R-MAT scale 22, weights to 64, 2.88, 2.70, 2.61 ms;
+    // weights to 1000, 5.69, 5.25, 4.81; Erdos-Renyi V = 2^21, weights to 255,
+    // 5.04, 3.04, 3.49
+    const double f = g->static_vertices == g->h.V ? 0.12 : 12.0;
     return (uint32_t)std::min(std::max(1.0, f * g->mean_weight), 2147483648.0);
 }
 
@@ -1320,12 +1343,15 @@ static int run_traversal(asc_graph* g, uint32_t src, uint32_t* out, asc_stats* s
 
     // initial state
     if (use16 && !t->val16) ASC_HIP(hipMalloc(&t->val16, 4 * ((V + 1) / 2)));
+    const bool use8 = ALGO == ALG_BFS && vs == V && V >= kSeenMinV;
+    if (use8 && !t->seen8) ASC_HIP(hipMalloc(&t->seen8, 4 * ((V + 3) / 4)));
     RunInit ri{};
     ri.V = V;
     ri.slots = t->slots;
     ri.piles = t->piles;
     ri.stats = t->stats;
     ri.src = src;
+    if (use8) ri.seen8 = (uint32_t*)t->seen8;
     ri.unreached = (uint32_t)(V + 1);
     if (ALGO == ALG_CC) {
         ri.n_res0 = vs;
@@ -1342,7 +1368,6 @@ static int run_traversal(asc_graph* g, uint32_t src, uint32_t* out, asc_stats* s
     } else {
         ri.stamp = t->stamp;
         ri.pstamp = vs < V ? t->pstamp : nullptr;   // on-demand vertices only
-        ri.fstamp = ALGO == ALG_SSSP ? t->fstamp : nullptr;
         ri.done = t->done;
     }
     // the value filter serves fully resident graphs (narrow bands: few
@@ -1363,9 +1388,9 @@ static int run_traversal(asc_graph* g, uint32_t src, uint32_t* out, asc_stats* s
     a.edges = (const EdgeT*)g->d_edges;
     a.val = t->val;
     a.val16 = use16 ? t->val16 : nullptr;
+    a.seen8 = use8 ? t->seen8 : nullptr;
     a.stamp = t->stamp;
     a.pstamp = t->pstamp;
-    a.fstamp = t->fstamp;
     a.done = t->done;
     a.visited = t->visited;
     a.slots = t->slots;
@@ -1377,7 +1402,7 @@ static int run_traversal(asc_graph* g, uint32_t src, uint32_t* out, asc_stats* s
     a.heavy_thr = (uint32_t)effective_heavy_threshold(g);
     a.theta = (ALGO == ALG_SSSP && delta) ? 1 + delta : 0xFFFFFFFFu;
     a.pepoch = 1;
-    a.fepoch = 1;
+    a.unreached = (uint32_t)(V + 1);
     uint32_t pcur = 0, fcur = 0;
 
     uint32_t nr, npend, nfar = 0;
@@ -1397,6 +1422,7 @@ static int run_traversal(asc_graph* g, uint32_t src, uint32_t* out, asc_stats* s
     uint32_t level = 0;
     bool last_split_empty = false;
     const bool resident = vs == V;
+    uint64_t width = delta, band_nodes = 0;   // the next band's; vertices expanded before this one
     // edges of the frontier where known (the source, a small published one)
     uint64_t nedges = ALGO == ALG_CC ? g->h.E : g->h.off[src + 1] - g->h.off[src];
     for (;;) {
@@ -1448,7 +1474,10 @@ static int run_traversal(asc_graph* g, uint32_t src, uint32_t* out, asc_stats* s
         a.far_count = &t->piles->n_far[fcur];
         if (mode == M_SPLIT) {
             // advance the band; entries still beyond it move to the other far pile
-            const uint64_t th = (uint64_t)(last_split_empty ? std::max(a.theta, t->h[0].piles.min_far) : a.theta) + delta;
+            if (resident && rc.node_sum - band_nodes < kBandShare * (uint64_t)nfar)
+                width = std::min(width * kBandGrow, (uint64_t)delta << 8);
+            band_nodes = rc.node_sum;
+            const uint64_t th = (uint64_t)(last_split_empty ? std::max(a.theta, t->h[0].piles.min_far) : a.theta) + width;
             a.theta = (uint32_t)std::min<uint64_t>(th, 0xFFFFFFFFull);
             const uint32_t old = fcur;
             fcur ^= 1;
@@ -1477,7 +1506,7 @@ static int run_traversal(asc_graph* g, uint32_t src, uint32_t* out, asc_stats* s
                 ASC_HIP(hipEventRecord(e0, s));
             }
             // one workgroup per 256 frontier entries, at most `grid`
-            const int lgrid = (int)std::max<uint64_t>(1, std::min<uint64_t>(grid, ((uint64_t)nr + kBlock - 1) / kBlock));
+            const int lgrid = (int)std::max<uint64_t>(1, std::min<uint64_t>(grid, ((uint64_t)nr + kPassMin - 1) / kPassMin));
             ASC_TRY(timed_launch(t, prof, KERN_LOCAL, s, [&] {
                 hipLaunchKernelGGL((k_expand_local<ALGO, OffT, EdgeT>), dim3(lgrid), dim3(kBlock), 0, s, a, level);
             }));

@@ -96,11 +96,19 @@ struct TravArgs {
     // store can leave a larger one): never below val[v], so a candidate not
     // below it cannot lower val[v].  0xFFFF (not lowered yet, or a value
     // beyond 16 bits): the atomic is tried.  Half the bytes of val, so more
-    // of the probed vertices stay in cache.
+    // of the probed vertices stay in cache.  An XCD's L2 does not see the
+    // others' stores within a step: a lane whose atomic lowers nothing stores
+    // what it learned too, or every edge of that XCD to a hub tries again
+    // (R-MAT scale 22: 5.2 -> 3.9 ms a run).
     uint16_t* val16;
+    // BFS on a fully resident graph of kSeenMinV vertices and more (else
+    // null): 1 for a vertex some lane saw visited.  Atomics go past the L2 and
+    // drop the line from it, so a bitmap under claims is mostly read from
+    // memory; these bytes are plain stores, and an XCD that has not seen
+    // another's learns by one atomic.
+    uint8_t* seen8;
     uint32_t* stamp;                // SSSP/CC: level a resident vertex was last queued for
     uint32_t* pstamp;               // SSSP/CC: on-demand pile epoch a vertex was last added to
-    uint32_t* fstamp;               // SSSP: set (to fepoch, constant in a run) once a vertex enters the far pile
     uint32_t* done;                 // SSSP/CC: value a vertex was last expanded with
     uint32_t* visited;              // BFS bitmap
     const uint32_t* q_in;
@@ -120,7 +128,8 @@ struct TravArgs {
     uint32_t vs;                    // vertices [0, vs) are resident
     uint32_t heavy_thr;
     uint32_t theta;                 // SSSP near/far boundary (UINT_MAX: everything near)
-    uint32_t pepoch, fepoch;
+    uint32_t pepoch;
+    uint32_t unreached;             // SSSP: the value of a vertex not reached yet
 };
 
 template <class EdgeT>
@@ -160,7 +169,7 @@ struct LevelPub {
 
 // Arrays to set at the start of a run (null: not used by it).
 struct RunInit {
-    uint32_t *val, *stamp, *pstamp, *fstamp, *done, *visited, *val16;
+    uint32_t *val, *stamp, *pstamp, *done, *visited, *val16, *seen8;
     uint64_t V;
     Slot* slots;
     Piles* piles;
@@ -224,10 +233,10 @@ struct TravState {
     DevArena mem, mem_relax, mem_fast;
     uint64_t V = 0;
     uint32_t* val = nullptr;
+    uint8_t* seen8 = nullptr;
     uint16_t* val16 = nullptr;        // SSSP value filter (TravArgs::val16)
     uint32_t* stamp = nullptr;
     uint32_t* pstamp = nullptr;
-    uint32_t* fstamp = nullptr;
     uint32_t* done = nullptr;
     uint32_t* visited = nullptr;
     uint32_t* q[2] = {nullptr, nullptr};
