@@ -88,6 +88,48 @@ struct BatchArgs {
     uint32_t heavy_thr;
 };
 
+// Vertices a workgroup takes per pass of a local step (`most`, halved while the
+// frontier is too small to give every workgroup one): R-MAT frontiers of a few
+// thousand vertices have hundreds of edges each.
+__device__ __forceinline__ uint32_t pass_size(uint32_t n, uint32_t most) {
+    uint32_t per = most;
+    while (per > 16 && per * gridDim.x > n) per >>= 1;
+    return per;
+}
+
+// The rest of a workgroup's queue entries and the lanes that advanced: one
+// atomic each (same-address atomics take 9 ns: one a wave of a full grid 74 us),
+// the lanes' only where they are news to this XCD.  Called by the whole
+// workgroup.
+__device__ __forceinline__ void end_step(const WaveStage<kStageCap>& st, unsigned long long act, uint32_t* q,
+                                         Slot* nxt) {
+    __shared__ uint32_t s_n[kWavesPerBlock], s_at;
+    __shared__ unsigned long long s_act[kWavesPerBlock];
+    const uint32_t w = wave_id();
+#pragma unroll
+    for (int d = kWave / 2; d > 0; d >>= 1) act |= __shfl_xor(act, d, kWave);
+    if (lane_id() == 0) {
+        s_n[w] = st.n;
+        s_act[w] = act;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t all = 0;
+        unsigned long long any = 0;
+        for (int i = 0; i < kWavesPerBlock; i++) {
+            all += s_n[i];
+            any |= s_act[i];
+        }
+        if (all) s_at = atomicAdd(&nxt->n_res, all);
+        if (any & ~nxt->pad[0]) atomicOr(&nxt->pad[0], any);
+    }
+    __syncthreads();
+    if (!st.n) return;
+    uint32_t at = s_at;
+    for (uint32_t i = 0; i < w; i++) at += s_n[i];
+    for (uint32_t j = lane_id(); j < st.n; j += kWave) q[at + j] = st.buf[j];
+}
+
 // -- BFS lanes ------------------------------------------------------------------
 
 constexpr uint32_t kLev8Max = 0xFEu;   // largest level an 8-bit BFS lane holds (0xFF: unreached)
@@ -164,12 +206,13 @@ __global__ __launch_bounds__(kBlock) void k_msbfs_local(BatchArgs<OffT, EdgeT> a
     const uint32_t tid = threadIdx.x, lane = lane_id(), w = wave_id();
     WaveStage<kStageCap> st{s_stage[w], 0};
     unsigned long long act = 0;
-    for (uint32_t base = blockIdx.x * kBlock; base < n; base += gridDim.x * kBlock) {
+    const uint32_t per = pass_size(n, kBlock);
+    for (uint32_t base = blockIdx.x * per; base < n; base += gridDim.x * per) {
         const uint32_t i = base + tid;
         uint32_t deg = 0;
         OffT beg = 0;
         unsigned long long bits = 0;
-        if (i < n) {
+        if (tid < per && i < n) {
             const uint32_t u = a.q_in[i];
             bits = a.X[u] & td_mask;   // bottom-up lanes' bits were consumed already
             a.X[u] = 0;
@@ -193,7 +236,7 @@ __global__ __launch_bounds__(kBlock) void k_msbfs_local(BatchArgs<OffT, EdgeT> a
         s_beg[tid] = beg;
         s_bits[tid] = bits;
         __syncthreads();
-        const uint32_t cnt = min(n - base, (uint32_t)kBlock);
+        const uint32_t cnt = min(n - base, per);
         for (uint32_t eb = w * kWave * kMsUnroll; eb < total; eb += kBlock * kMsUnroll) {
             uint32_t v[kMsUnroll], valid = 0;
             unsigned long long bb[kMsUnroll];
@@ -216,10 +259,7 @@ __global__ __launch_bounds__(kBlock) void k_msbfs_local(BatchArgs<OffT, EdgeT> a
         }
         __syncthreads();
     }
-    st.flush(a.q_out, &nxt->n_res);
-#pragma unroll
-    for (int d = kWave / 2; d > 0; d >>= 1) act |= __shfl_xor(act, d, kWave);
-    if (lane == 0 && act) atomicOr(&nxt->pad[0], act);
+    end_step(st, act, a.q_out, nxt);
 }
 
 template <class OffT, class EdgeT>
@@ -280,10 +320,7 @@ __global__ __launch_bounds__(kBlock) void k_msbfs_heavy(BatchArgs<OffT, EdgeT> a
         }
         __syncthreads();
     }
-    st.flush(a.q_out, &nxt->n_res);
-#pragma unroll
-    for (int d = kWave / 2; d > 0; d >>= 1) act |= __shfl_xor(act, d, kWave);
-    if (lane == 0 && act) atomicOr(&nxt->pad[0], act);
+    end_step(st, act, a.q_out, nxt);
 }
 
 // Neighbour ids loaded before their frontier words are probed (8 and 16 ran
@@ -319,22 +356,19 @@ __global__ __launch_bounds__(kBlock) void k_msbfs_bottom_up(BatchArgs<OffT, Edge
                     for (int j = 0; j < kBuBatch; j++) nw |= a.X[u[j]] & need;
                 }
                 if (nw) {
-                    const unsigned long long old = atomicOr(a.seen + v, nw);
-                    nw &= ~old;
-                    if (nw) {
-                        act |= nw;
-                        msbfs_set_levels(a, (uint32_t)v, nw, step);
-                        push = atomicOr(a.Y + v, nw) == 0;
-                    }
+                    // v is this lane's alone until the kernel ends
+                    a.seen[v] |= nw;
+                    act |= nw;
+                    msbfs_set_levels(a, (uint32_t)v, nw, step);
+                    const unsigned long long y = a.Y[v];
+                    a.Y[v] = y | nw;
+                    push = y == 0;
                 }
             }
         }
         st.push(push, (uint32_t)v, a.q_out, &nxt->n_res);
     }
-    st.flush(a.q_out, &nxt->n_res);
-#pragma unroll
-    for (int d = kWave / 2; d > 0; d >>= 1) act |= __shfl_xor(act, d, kWave);
-    if (lane_id() == 0 && act) atomicOr(&nxt->pad[0], act);
+    end_step(st, act, a.q_out, nxt);
 }
 
 // Per lane q: vertices with bit q in Y (cnt[q]) and, for the top-down lanes
@@ -537,6 +571,11 @@ __device__ __forceinline__ bool mssp_relax(const BatchArgs<OffT, WEdge>& a, cons
     return atomicOr(a.Y + v, imp) == 0;
 }
 
+// Source rows of a workgroup's pass: 8 KB of LDS, so that eight workgroups fit
+// a CU (four with 256 rows; with smaller passes R-MAT scale 19, 19 lanes: 3.06
+// -> 1.66 ms of these steps a batch).
+constexpr uint32_t kRowTile = 64;
+
 template <class OffT>
 __global__ __launch_bounds__(kBlock) void k_mssp_local(BatchArgs<OffT, WEdge> a) {
     const uint32_t step = a.sp->step;
@@ -545,7 +584,7 @@ __global__ __launch_bounds__(kBlock) void k_mssp_local(BatchArgs<OffT, WEdge> a)
     __shared__ unsigned long long s_bits[kBlock];
     __shared__ uint32_t s_tmp[kWavesPerBlock];
     __shared__ uint32_t s_stage[kWavesPerBlock][kStageCap];
-    __shared__ uint4 s_rows[kBlock][kMaxLanes / 8];   // the tile's source rows (read by every edge of a vertex)
+    __shared__ uint4 s_rows[kRowTile][kMaxLanes / 8];   // the tile's source rows (read by every edge of a vertex)
     Slot* cur = a.slots + (step & 3);
     Slot* nxt = a.slots + ((step + 1) & 3);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -559,12 +598,13 @@ __global__ __launch_bounds__(kBlock) void k_mssp_local(BatchArgs<OffT, WEdge> a)
     const uint32_t row_u4 = a.stride / 8;
     WaveStage<kStageCap> st{s_stage[w], 0};
     unsigned long long act = 0;
-    for (uint32_t base = blockIdx.x * kBlock; base < n; base += gridDim.x * kBlock) {
+    const uint32_t per = pass_size(n, kRowTile);
+    for (uint32_t base = blockIdx.x * per; base < n; base += gridDim.x * per) {
         const uint32_t i = base + tid;
         uint32_t deg = 0, u = 0;
         OffT beg = 0;
         unsigned long long bits = 0;
-        if (i < n) {
+        if (tid < per && i < n) {
             u = a.q_in[i];
             bits = a.X[u];
             a.X[u] = 0;
@@ -592,7 +632,7 @@ __global__ __launch_bounds__(kBlock) void k_mssp_local(BatchArgs<OffT, WEdge> a)
         s_beg[tid] = beg;
         s_bits[tid] = bits;
         __syncthreads();
-        const uint32_t cnt = min(n - base, (uint32_t)kBlock);
+        const uint32_t cnt = min(n - base, per);
         for (uint32_t eb = w * kWave; eb < total; eb += kBlock) {
             const uint32_t e = eb + lane_id();
             bool push = false;
@@ -610,10 +650,7 @@ __global__ __launch_bounds__(kBlock) void k_mssp_local(BatchArgs<OffT, WEdge> a)
         }
         __syncthreads();
     }
-    st.flush(a.q_out, &nxt->n_res);
-#pragma unroll
-    for (int d = kWave / 2; d > 0; d >>= 1) act |= __shfl_xor(act, d, kWave);
-    if (lane_id() == 0 && act) atomicOr(&nxt->pad[0], act);
+    end_step(st, act, a.q_out, nxt);
 }
 
 template <class OffT>
@@ -673,10 +710,7 @@ __global__ __launch_bounds__(kBlock) void k_mssp_heavy(BatchArgs<OffT, WEdge> a)
         }
         __syncthreads();
     }
-    st.flush(a.q_out, &nxt->n_res);
-#pragma unroll
-    for (int d = kWave / 2; d > 0; d >>= 1) act |= __shfl_xor(act, d, kWave);
-    if (lane_id() == 0 && act) atomicOr(&nxt->pad[0], act);
+    end_step(st, act, a.q_out, nxt);
 }
 
 // -- admission ------------------------------------------------------------------

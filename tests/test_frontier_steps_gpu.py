@@ -50,3 +50,26 @@ def test_growing_bands(wmax, delta):
         for _ in range(2):
             assert np.array_equal(g.sssp(src)[0], O.dijkstra(csr, src))
     h.free()
+
+
+@pytest.mark.parametrize("n", [15, 2049, 32769, 140001])
+def test_served_star(gpu_ctx, n):
+    """Served lanes through frontiers of n vertices: passes of 16 to 256 (BFS)
+    and 64 (SSSP) vertices, from the hub and from three leaves."""
+    r = np.random.default_rng(n)
+    V = 2 * n + 1
+    a = np.concatenate([np.zeros(n, np.int64), np.arange(1, n + 1)])
+    b = np.concatenate([np.arange(1, n + 1), n + 1 + r.integers(0, n, n)])
+    w = r.integers(1, 100, 2 * n)
+    src, dst, wt = np.concatenate([a, b]), np.concatenate([b, a]), np.concatenate([w, w])
+    order = np.argsort(src, kind="stable")
+    off = np.concatenate([[0], np.cumsum(np.bincount(src, minlength=V))]).astype(np.uint64)
+    ew = np.stack([dst[order], wt[order]], 1).astype(np.uint32)
+    csr = O.CSR(off, ew[:, 0].copy(), ew[:, 1].copy())
+    sources = [0, 1, n, V - 1]
+    with gpu_ctx.from_arrays(off, ew) as g, A.Server(g, lanes=16) as srv:
+        outs = [(k, s, np.empty(V, np.uint32)) for s in sources for k in (A.Server.BFS, A.Server.SSSP)]
+        for t in [srv.submit(k, s, o) for k, s, o in outs]:
+            srv.wait(t)
+        for k, s, o in outs:
+            assert np.array_equal(o, O.bfs_queue(csr, s) if k == A.Server.BFS else O.dijkstra(csr, s)), (k, s)
