@@ -142,7 +142,8 @@ __global__ __launch_bounds__(kBlock) void k_expand_part(TravArgs<OffT, EdgeT> a,
                     const uint32_t x = ZC ? p.zc32[ix] : p.part32[ix];
                     if (p.pk_split) {
                         vv[j] = x;
-                        ww[j] = (uint32_t)(ZC ? p.zc_w8[ix] : p.part_w8[ix]) + p.pk_wmin;
+                        // (part buffers hold the weight bytes of SSSP runs alone)
+                        ww[j] = ALGO == ALG_SSSP ? (uint32_t)(ZC ? p.zc_w8[ix] : p.part_w8[ix]) + p.pk_wmin : 0u;
                     } else {
                         vv[j] = x & p.pk_mask;
                         ww[j] = (x >> p.pk_shift) + p.pk_wmin;
@@ -821,10 +822,10 @@ static uint32_t sssp_delta(asc_graph* g) {
 // src[k]: first record of the k-th listed vertex in the array gathered from
 // (the packed tail, indexed from static_edges on, or the host records).
 static void gather_part(asc_graph* g, const unsigned long long* src, const unsigned long long* prefix, uint64_t m,
-                        uint64_t lo, uint64_t hi, char* dst, char* dst_w) {
+                        uint64_t lo, uint64_t hi, char* dst, char* dst_w, bool weights) {
     if (g->packed) {
         gather_edges(*g->ctx->pool, (const char*)g->ptail.p, 4, src, prefix, m, lo, hi, dst);
-        if (g->pk_split)   // the weight bytes, at the same positions of their own array
+        if (g->pk_split && weights)   // the weight bytes, at the same positions of their own array
             gather_edges(*g->ctx->pool, (const char*)g->ptail_w.p, 1, src, prefix, m, lo, hi, dst_w);
     } else
         gather_edges(*g->ctx->pool, (const char*)g->h.edges.p, g->h.edge_bytes(), src, prefix, m, lo, hi, dst);
@@ -885,7 +886,8 @@ static int copy_to_part(asc_graph* g, TravState* t, int b, const char* src, cons
     }
     if (g->pk_split) {
         ASC_HIP(hipMemcpyAsync(t->part[b], src, 4 * cnt, hipMemcpyHostToDevice, s));
-        ASC_HIP(hipMemcpyAsync((char*)t->part[b] + 4 * t->part_edges, src_w, cnt, hipMemcpyHostToDevice, s));
+        if (t->stream_w)
+            ASC_HIP(hipMemcpyAsync((char*)t->part[b] + 4 * t->part_edges, src_w, cnt, hipMemcpyHostToDevice, s));
     } else {
         ASC_HIP(hipMemcpyAsync(t->part[b], src, cnt * g->stream_record_bytes(), hipMemcpyHostToDevice, s));
     }
@@ -921,7 +923,7 @@ static int copy_chunk_to_part(asc_graph* g, TravState* t, int b, uint64_t e0, ui
     char* dst = t->stage[sb].p;
     char* dst_w = dst + 4 * t->part_edges;
     const char* src = tail_rec(g, e0);
-    const char* src_w = tail_w8(g, e0);
+    const char* src_w = t->stream_w ? tail_w8(g, e0) : nullptr;
     const double t0 = now_ms();
     g->ctx->pool->parallel_for(n, [&](uint64_t lo, uint64_t hi) {
         std::memcpy(dst + lo * rb, src + lo * rb, (hi - lo) * rb);
@@ -996,7 +998,7 @@ static int stream_pile(asc_graph* g, TravArgs<OffT, EdgeT>& a, uint32_t& level, 
     const uint64_t nod = g->h.V - g->static_vertices;
     uint32_t* list_deg = t->od_list + nod;
     const bool pk = g->packed;
-    const size_t EB = g->stream_record_bytes();
+    const size_t EB = g->pk_split && !t->stream_w ? 4 : g->stream_record_bytes();   // bytes that cross the link
     const uint64_t S = g->static_edges;
     const int pile_grid = (int)std::max<uint32_t>(1, std::min<uint32_t>((npile + kBlock - 1) / kBlock, 4096));
     // the host gather's index of the first n list entries (the sparse
@@ -1287,7 +1289,7 @@ static int stream_pile(asc_graph* g, TravArgs<OffT, EdgeT>& a, uint32_t& level, 
             ASC_HIP(hipEventSynchronize(t->ev_stage[sb]));  // staging sb drained
             const double tg = now_ms();
             char* stage_w = t->stage[sb].p + 4 * PE;   // split form: weight bytes behind the ids
-            gather_part(g, t->h_src.p, t->h_prefix.p, n_sparse, lo, hi, t->stage[sb].p, stage_w);
+            gather_part(g, t->h_src.p, t->h_prefix.p, n_sparse, lo, hi, t->stage[sb].p, stage_w, t->stream_w);
             const double dt = now_ms() - tg;
             fill_round += dt;
             gather_round += dt;
@@ -1416,6 +1418,7 @@ static int run_traversal(asc_graph* g, uint32_t src, uint32_t* out, asc_stats* s
     RunCounters rc{};
     t->timed.clear();
     t->ev_next = 0;
+    t->stream_w = ALGO == ALG_SSSP;
     const double t0 = now_ms();
     rc.t_start = t0;
     if (g->static_vertices < V && t->part[0]) ASC_TRY(prefetch_chunks(g, t));

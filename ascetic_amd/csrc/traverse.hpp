@@ -234,6 +234,9 @@ struct TravState {
     uint64_t V = 0;
     uint32_t* val = nullptr;
     uint8_t* seen8 = nullptr;
+    // this run ships the split form's weight bytes (BFS and CC do without: 4
+    // of 5 bytes on the link; R-MAT scale 21, a third resident, 10.3 -> 9.0 ms)
+    bool stream_w = true;
     uint16_t* val16 = nullptr;        // SSSP value filter (TravArgs::val16)
     uint32_t* stamp = nullptr;
     uint32_t* pstamp = nullptr;

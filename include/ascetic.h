@@ -301,7 +301,8 @@ typedef struct {
     uint64_t edges_traversed;    /* edges relaxed (static + on-demand)        */
     uint64_t static_edges_traversed;
     uint64_t streamed_edges;     /* on-demand edges shipped over the link     */
-    uint64_t streamed_bytes;
+    uint64_t streamed_bytes;     /* their records' bytes (BFS and CC leave the
+                                    split form's weight byte behind)          */
     uint64_t dense_edges;        /* of streamed_edges: copied as whole chunks
                                     by DMA (asc_config.dense_threshold)       */
     uint64_t vertices_processed; /* frontier entries expanded                 */
