@@ -574,7 +574,10 @@ static int run_bfs_do(asc_graph* g, uint32_t src, uint32_t* out, asc_stats* st) 
     uint32_t level = 0;
     const double t0 = now_ms();
     while (nf > 0) {
-        if (bottom_up && nf < V / kBeta && nf < prev_nf) {
+        // (a frontier that the rule below would take bottom-up again stays: two
+        // conversions, 45 us at scale 20)
+        if (bottom_up && nf < V / kBeta && nf < prev_nf &&
+            (mf <= m_unexplored / kAlpha || (nf <= kNarrowCap && mf <= kNarrowEdges))) {
             // bitmap -> queue, slot ring restarted at this level
             hipLaunchKernelGGL(k_do_fill, dim3(1), dim3(kBlock), 0, s, (uint32_t*)t->slots, sizeof(Slot) * 4 / 4, 0u);
             hipLaunchKernelGGL(k_bitmap_to_queue, dim3(std::max<uint64_t>(1, std::min<uint64_t>((words + kBlock - 1) / kBlock, grid))),
