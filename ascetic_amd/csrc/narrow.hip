@@ -41,7 +41,7 @@ struct NarrowArgs {
     unsigned long long seq;
     uint32_t level, n_in;
     uint32_t n_far, fcur;
-    uint32_t theta, delta;
+    uint32_t theta, delta, most;    // band; the next band's width, doubled at every split up to `most`
     uint32_t edge_limit, V;
 };
 
@@ -65,7 +65,7 @@ __global__ __launch_bounds__(kNwBlock) void k_narrow(TravArgs<OffT, EdgeT> a, Na
     __shared__ uint32_t s_nfar[2], s_min;
     const uint32_t tid = threadIdx.x;
     const unsigned long long t_begin = wall_clock64();
-    uint32_t level = na.level, fcur = na.fcur, theta = na.theta;
+    uint32_t level = na.level, fcur = na.fcur, theta = na.theta, width = na.delta;
     unsigned long long nodes = 0, edges = 0;
     uint32_t steps = 0, splits = 0;
 
@@ -146,7 +146,8 @@ __global__ __launch_bounds__(kNwBlock) void k_narrow(TravArgs<OffT, EdgeT> a, Na
             if (lane_id() == 0 && lmin != 0xFFFFFFFFu) atomicMin(&s_min, lmin);
             __syncthreads();
             const uint32_t m = s_min;
-            theta = (uint32_t)min((unsigned long long)max(theta, m == 0xFFFFFFFFu ? 0u : m) + na.delta, 0xFFFFFFFFull);
+            theta = (uint32_t)min((unsigned long long)max(theta, m == 0xFFFFFFFFu ? 0u : m) + width, 0xFFFFFFFFull);
+            width = (uint32_t)min(2ull * width, (unsigned long long)na.most);
 #pragma unroll
             for (int j = 0; j < kNwFarPer; j++) {
                 const uint32_t i = j * kNwBlock + tid;
@@ -301,7 +302,7 @@ __global__ __launch_bounds__(kNwBlock) void k_narrow(TravArgs<OffT, EdgeT> a, Na
 
 template <int ALGO, class OffT, class EdgeT>
 int narrow_run(asc_graph* g, const TravArgs<OffT, EdgeT>& a, uint32_t n_in, uint32_t n_far, uint32_t delta,
-               NarrowState& io) {
+               uint32_t most, NarrowState& io) {
     TravState* t = g->trav;
     hipStream_t s = g->ctx->s_main;
     const bool prof = g->ctx->cfg.profile != 0;
@@ -319,6 +320,7 @@ int narrow_run(asc_graph* g, const TravArgs<OffT, EdgeT>& a, uint32_t n_in, uint
     na.fcur = io.fcur;
     na.theta = a.theta;
     na.delta = delta;
+    na.most = most;
     na.edge_limit = kNarrowEdges;
     na.V = (uint32_t)g->h.V;
     ASC_TRY(timed_launch(t, prof, KERN_LOCAL, s, [&] {
@@ -343,7 +345,7 @@ int narrow_run(asc_graph* g, const TravArgs<OffT, EdgeT>& a, uint32_t n_in, uint
 
 #define ASC_NARROW(ALGO, OffT, EdgeT)                                                                          \
     template int narrow_run<ALGO, OffT, EdgeT>(asc_graph*, const TravArgs<OffT, EdgeT>&, uint32_t, uint32_t, \
-                                               uint32_t, NarrowState&);
+                                               uint32_t, uint32_t, NarrowState&);
 #define ASC_NARROW_ALL(ALGO)           \
     ASC_NARROW(ALGO, uint32_t, uint32_t) \
     ASC_NARROW(ALGO, uint64_t, uint32_t) \

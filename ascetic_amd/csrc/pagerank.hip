@@ -1668,8 +1668,10 @@ static int pr_blocked_build(asc_graph* g, PrState* p, bool by_name) {
     const uint32_t* src = (const uint32_t*)g->d_edges;
     // rows left to the pull, in order
     std::vector<uint32_t> heavy(p->rows_front);
-    if (p->rows_front)
-        ASC_HIP(hipMemcpy(heavy.data(), p->rows_heavy, 4 * heavy.size(), hipMemcpyDeviceToHost));
+    if (p->rows_front) {
+        ASC_HIP(hipMemcpyAsync(heavy.data(), p->rows_heavy, 4 * heavy.size(), hipMemcpyDeviceToHost, s));
+        ASC_HIP(hipStreamSynchronize(s));
+    }
     std::sort(heavy.begin(), heavy.end());
     const uint64_t* ho = g->h.off.p;
     std::vector<PbBin> bins;

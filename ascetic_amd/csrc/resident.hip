@@ -589,7 +589,7 @@ static int run_bfs_do(asc_graph* g, uint32_t src, uint32_t* out, asc_stats* st) 
             // small top-down levels run back to back in one workgroup
             NarrowState io;
             io.level = level;
-            ASC_TRY((narrow_run<ALG_BFS, OffT, EdgeT>(g, a, (uint32_t)nf, 0, 0, io)));
+            ASC_TRY((narrow_run<ALG_BFS, OffT, EdgeT>(g, a, (uint32_t)nf, 0, 0, 0, io)));
             const uint64_t reached = io.expanded + io.edges - mf;   // edges of the vertices claimed
             m_unexplored = m_unexplored > reached ? m_unexplored - reached : 0;
             level = io.level;

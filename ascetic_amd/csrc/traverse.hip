@@ -783,6 +783,8 @@ static bool sssp_filter_pays(asc_graph* g) {
 // trips whatever its size, so wider bands trade re-expansions for fewer steps
 // (1201 x 1033 mesh, weights 1-255, narrow bands of 64: 39.6 ms, of 128 33.3,
 // of 256 30.8, of 512 30.4, of 1024 33.0; wide ones are 15).
+// They start at one and double with every split, for the same reason as
+// kBandBulk.
 constexpr uint32_t kNarrowBands = 16;
 
 // A split reads the whole far pile, whatever it takes out of it.  Where a band
@@ -791,11 +793,19 @@ constexpr uint32_t kNarrowBands = 16;
 // scale 22 needs 2 to 3 splits instead of 9 (3.9 -> 2.9 ms), scale 18 1.12 ->
 // 0.76, with no edge relaxed more; 1 and 2 instead of 4: 3.26 and 3.08 ms.
 constexpr uint64_t kBandShare = 4, kBandGrow = 4;
+// Bands grow only once a V / kBandBulk-th of all vertices was expanded: a run
+// from a vertex far from the hubs has small bands before its bulk too, and
+// bands as wide as the bulk's distances relax its edges several times (R-MAT
+// scale 26 from random vertices: 70 ms without this and with the narrow bands
+// below at their full width from the start).
+constexpr uint64_t kBandBulk = 8;
 
 // Smallest resident graph whose BFS steps probe bytes (TravArgs::seen8)
 // instead of the visited bits (directed R-MAT, bits / bytes: scale 17 309 / 321
 // us, scale 20 627 / 534, scale 22 1265 / 955, scale 24 3553 / 3071).
-constexpr uint64_t kSeenMinV = uint64_t(1) << 18;
+// Beyond 2^25 the bytes leave the MALL to memory (symmetric scale 26 top-down
+// 18.3 / 25.8 ms; scale 24 5.38 / 5.44, directed V = 2^25 4202 / 3762 us).
+constexpr uint64_t kSeenMinV = uint64_t(1) << 18, kSeenMaxV = uint64_t(1) << 25;
 
 static uint32_t sssp_delta(asc_graph* g) {
     if (g->sssp_delta > 0) return (uint32_t)g->sssp_delta;
@@ -1345,7 +1355,7 @@ static int run_traversal(asc_graph* g, uint32_t src, uint32_t* out, asc_stats* s
 
     // initial state
     if (use16 && !t->val16) ASC_HIP(hipMalloc(&t->val16, 4 * ((V + 1) / 2)));
-    const bool use8 = ALGO == ALG_BFS && vs == V && V >= kSeenMinV;
+    const bool use8 = ALGO == ALG_BFS && vs == V && V >= kSeenMinV && V <= kSeenMaxV;
     if (use8 && !t->seen8) ASC_HIP(hipMalloc(&t->seen8, 4 * ((V + 3) / 4)));
     RunInit ri{};
     ri.V = V;
@@ -1425,6 +1435,8 @@ static int run_traversal(asc_graph* g, uint32_t src, uint32_t* out, asc_stats* s
     uint32_t level = 0;
     bool last_split_empty = false;
     const bool resident = vs == V;
+    const uint64_t narrow_most = std::min<uint64_t>((uint64_t)kNarrowBands * delta, 0x7FFFFFFFu);
+    uint64_t narrow_width = std::min<uint64_t>(delta, narrow_most);
     uint64_t width = delta, band_nodes = 0;   // the next band's; vertices expanded before this one
     // edges of the frontier where known (the source, a small published one)
     uint64_t nedges = ALGO == ALG_CC ? g->h.E : g->h.off[src + 1] - g->h.off[src];
@@ -1435,7 +1447,9 @@ static int run_traversal(asc_graph* g, uint32_t src, uint32_t* out, asc_stats* s
             NarrowState io;
             io.level = level;
             io.fcur = fcur;
-            ASC_TRY((narrow_run<ALGO, OffT, EdgeT>(g, a, nr, nfar, (uint32_t)std::min<uint64_t>((uint64_t)kNarrowBands * delta, 0x7FFFFFFFu), io)));
+            ASC_TRY((narrow_run<ALGO, OffT, EdgeT>(
+                g, a, nr, nfar, (uint32_t)std::min(narrow_width, narrow_most), (uint32_t)narrow_most, io)));
+            narrow_width = std::min(narrow_width << std::min(io.splits, 31u), narrow_most);
             level = io.level;
             nr = io.n;
             nedges = io.edges;
@@ -1477,7 +1491,7 @@ static int run_traversal(asc_graph* g, uint32_t src, uint32_t* out, asc_stats* s
         a.far_count = &t->piles->n_far[fcur];
         if (mode == M_SPLIT) {
             // advance the band; entries still beyond it move to the other far pile
-            if (resident && rc.node_sum - band_nodes < kBandShare * (uint64_t)nfar)
+            if (resident && rc.node_sum >= V / kBandBulk && rc.node_sum - band_nodes < kBandShare * (uint64_t)nfar)
                 width = std::min(width * kBandGrow, (uint64_t)delta << 8);
             band_nodes = rc.node_sum;
             const uint64_t th = (uint64_t)(last_split_empty ? std::max(a.theta, t->h[0].piles.min_far) : a.theta) + width;

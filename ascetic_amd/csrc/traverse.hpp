@@ -101,7 +101,7 @@ struct TravArgs {
     // what it learned too, or every edge of that XCD to a hub tries again
     // (R-MAT scale 22: 5.2 -> 3.9 ms a run).
     uint16_t* val16;
-    // BFS on a fully resident graph of kSeenMinV vertices and more (else
+    // BFS on a fully resident graph of kSeenMinV to kSeenMaxV vertices (else
     // null): 1 for a vertex some lane saw visited.  Atomics go past the L2 and
     // drop the line from it, so a bitmap under claims is mostly read from
     // memory; these bytes are plain stores, and an XCD that has not seen
@@ -343,7 +343,7 @@ int timed_launch(TravState* t, bool prof, int kind, hipStream_t s, F&& launch) {
 // starts at a.theta and advances by `delta`.
 template <int ALGO, class OffT, class EdgeT>
 int narrow_run(asc_graph* g, const TravArgs<OffT, EdgeT>& a, uint32_t n_in, uint32_t n_far, uint32_t delta,
-               NarrowState& io);
+               uint32_t most, NarrowState& io);
 
 // Shared end of a traversal run: kernel statistics from the recorded events
 // and DevStats, the values copied to `out` (value convention applied), and
