@@ -136,7 +136,8 @@ typedef struct {
     int pr_group;                /* lanes per vertex in the PageRank pull
                                     (4,8,16,32,64); 0 = blocks of rows, or
                                     the tuned value                           */
-    int sssp_delta;              /* SSSP bucket width (near-far); 0 = tuned,
+    int sssp_delta;              /* SSSP bucket width (near-far; bands of a
+                                    resident graph may grow); 0 = tuned,
                                     <0 = plain frontier Bellman-Ford          */
     int verbose;                 /* print per-phase timings like the reference */
     int profile;                 /* 1: time every relax kernel with HIP events
