@@ -28,7 +28,8 @@ __device__ __forceinline__ uint32_t candidate(uint32_t sv, uint32_t w) {
 // relax_commit_batch decides from it and performs the atomics.
 template <int ALGO, class OffT, class EdgeT>
 __device__ __forceinline__ uint32_t relax_probe(const TravArgs<OffT, EdgeT>& a, uint32_t v) {
-    if (ALGO == ALG_BFS) return a.seen8 ? 0u - (uint32_t)a.seen8[v] : a.visited[v >> 5];
+    if (ALGO == ALG_BFS)   // a byte either way: a branch would part the loads of a batch
+        return (a.seen8 ? a.seen8 : (const uint8_t*)a.visited)[v >> (a.seen8 ? 0 : 3)];
     if (ALGO == ALG_SSSP && a.val16) {
         // 0xFFFF: nothing known (not lowered yet, or a value beyond 16 bits),
         // so the atomic is tried
@@ -63,7 +64,7 @@ __device__ __forceinline__ void relax_commit_batch(const TravArgs<OffT, EdgeT>& 
 #pragma unroll
     for (int j = 0; j < kUnroll; j++) {
         to[j] = TO_NONE;
-        if (ALGO == ALG_BFS) try_[j] = ((valid >> j) & 1u) && !(probe[j] & (1u << (v[j] & 31)));
+        if (ALGO == ALG_BFS) try_[j] = ((valid >> j) & 1u) && !(probe[j] & (a.seen8 ? 1u : 1u << (v[j] & 7)));
         else try_[j] = ((valid >> j) & 1u) && cand[j] < probe[j];
         if (!try_[j]) continue;
         if (ALGO == ALG_BFS) old[j] = atomicOr(a.visited + (v[j] >> 5), 1u << (v[j] & 31));

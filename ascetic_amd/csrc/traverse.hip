@@ -804,7 +804,7 @@ constexpr uint64_t kBandBulk = 8;
 // instead of the visited bits (directed R-MAT, bits / bytes: scale 17 309 / 321
 // us, scale 20 627 / 534, scale 22 1265 / 955, scale 24 3553 / 3071).
 // Beyond 2^25 the bytes leave the MALL to memory (symmetric scale 26 top-down
-// 18.3 / 25.8 ms; scale 24 5.38 / 5.44, directed V = 2^25 4202 / 3762 us).
+// 18.3 / 25.8 ms; scale 24 5.36 / 5.09, directed V = 2^25 4202 / 3762 us).
 constexpr uint64_t kSeenMinV = uint64_t(1) << 18, kSeenMaxV = uint64_t(1) << 25;
 
 static uint32_t sssp_delta(asc_graph* g) {
