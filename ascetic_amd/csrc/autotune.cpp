@@ -151,7 +151,7 @@ int asc_autotune(asc_graph* g, double budget_ms, asc_tuning* out) {
             sweep(&g->sssp_delta, {-1, std::max(1, mw / 2), mw, 4 * mw});
         }
     } else if (g->static_vertices == g->h.V && g->h.V >= (uint64_t(1) << 20)) {
-        // the tiled pull (the default here): source segment size
+        // the tiled pull (taken where the blocked layout does not fit): source segment size
         if (g->pr_tile_src_bits <= 0) g->pr_tile_src_bits = 15;
         sweep(&g->pr_tile_src_bits, {13, 14, 16, 17, 18});
     } else {

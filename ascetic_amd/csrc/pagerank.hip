@@ -3,12 +3,13 @@
 // Normalised mode: r0 = 1/V; r' = (1-d)/V + d*(sum_{u->v} r[u]/outdeg[u] +
 // dangling/V) for a fixed number of iterations.  Ranks and the gathered
 // contributions c[u] = r[u]/outdeg[u] are FP32 (4 bytes per random gather);
-// each vertex's in-edge sum, the residual sum |r'-r| and the dangling mass
-// are accumulated in FP64.  The pull is coalesced: G lanes of a wave share a
-// vertex and read its in-edge ids contiguously; vertices with in-degree >=
-// the heavy threshold are summed by a whole workgroup instead.  The residual
-// and dangling sums are produced inside the same kernel, so iterations run
-// back-to-back without a host synchronisation.
+// each vertex's in-edge sum (64-bit fixed point in the blocked schedule, FP32
+// in the tiled one), the residual sum |r'-r| and the dangling mass are
+// accumulated in FP64.  Large resident graphs take the propagation-blocked
+// schedule, smaller ones row blocks, streamed rows the same sums without a
+// plan; a set pr_group keeps the pull in which G lanes share a vertex.  The
+// residual and dangling sums are produced inside the same kernels, so
+// iterations run back-to-back without a host synchronisation.
 //
 // Reference mode (gpu_kernels.cuh:533-594, CalculateOpt.cu:547-721): FP64,
 // 0.15 + 0.85*sum over active vertices, threshold 0.001, loop while any

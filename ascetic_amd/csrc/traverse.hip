@@ -9,7 +9,7 @@
 // overload adjacency of every active vertex every iteration.  Here the relax
 // kernels append improved vertices to device queues through per-wave LDS
 // staging, so a step costs O(frontier edges) and one host sync:
-//   k_expand_local  one workgroup per 256 frontier vertices; degrees below the
+//   k_expand_local  16 to 256 frontier vertices a workgroup; degrees below the
 //                   heavy threshold are expanded edge-balanced inside the
 //                   workgroup (LDS prefix scan + per-lane binary search), so
 //                   consecutive lanes read consecutive edges of a vertex;
@@ -1522,7 +1522,7 @@ static int run_traversal(asc_graph* g, uint32_t src, uint32_t* out, asc_stats* s
                 if (!e0) return ASC_ERR_DEVICE;
                 ASC_HIP(hipEventRecord(e0, s));
             }
-            // one workgroup per 256 frontier entries, at most `grid`
+            // one workgroup per kPassMin frontier entries, at most `grid`
             const int lgrid = (int)std::max<uint64_t>(1, std::min<uint64_t>(grid, ((uint64_t)nr + kPassMin - 1) / kPassMin));
             ASC_TRY(timed_launch(t, prof, KERN_LOCAL, s, [&] {
                 hipLaunchKernelGGL((k_expand_local<ALGO, OffT, EdgeT>), dim3(lgrid), dim3(kBlock), 0, s, a, level);
