@@ -12,27 +12,11 @@
 
 #include "device_common.hpp"
 #include "internal.hpp"
+#include "out_ring.hpp"
 
 namespace asc {
 
-constexpr uint32_t kOutPiece = 1u << 15;   // 32-bit words per piece (128 KiB: 2.3 us of the link, ~16 us of a thread)
-// Pieces per launch and workgroups per piece: a launch takes ~10 us beside its
-// bytes' time on the link, and more workgroups only add system fences (16 MB
-// result: 8 pieces of 16 workgroups 520 us, of 4 450; 16 of 16 480, of 8 430,
-// of 4 400, of 2 410; 32 of 4 400).
-constexpr int kOutGroup = 16;
-// pieces in flight: two groups, one on the link while the other is copied
-// (page-locking its 4 MiB takes ~290 us once, where 2 MiB take ~35)
-constexpr int kOutRing = 2 * kOutGroup;
-constexpr int kOutBlocks = 4;
-constexpr uint64_t kOutAlone = 2;          // up to this many pieces the calling thread copies alone
-constexpr int kOutHelpers = 7;             // threads that help it with more
-
-// Written by the device, a cache line each.
-struct OutPub {
-    unsigned long long seq;
-    unsigned long long pad[15];
-};
+constexpr int kOutBlocks = 4;              // workgroups per piece, at most (kOutGroup)
 
 struct OutStage {
     HostBuf<uint32_t> buf;          // kOutRing pieces (fewer for a small result)
