@@ -10,6 +10,7 @@
 #include <condition_variable>
 #include <cstdint>
 #include <cstring>
+#include <exception>
 #include <memory>
 #include <mutex>
 #include <thread>
@@ -87,8 +88,13 @@ struct OutJob {
 
 class OutHelpers {
 public:
+    // As many as the system grants, up to n: a thread that cannot be had must
+    // not end a query (or the process), the calling thread copies alone.
     explicit OutHelpers(int n) {
-        for (int i = 0; i < n; i++) threads_.emplace_back([this] { loop(); });
+        try {
+            for (int i = 0; i < n; i++) threads_.emplace_back([this] { loop(); });
+        } catch (const std::exception&) {
+        }
     }
     ~OutHelpers() {
         {

@@ -1,5 +1,8 @@
 // Plays the device to the ring loop (out_ring.hpp) on the CPU.
+#include <sys/resource.h>
+
 #include <cstdio>
+#include <cstring>
 
 #include "out_ring.hpp"
 
@@ -116,9 +119,33 @@ int with_helpers(OutHelpers& helpers) {
     return 0;
 }
 
+// No room for another thread's stack (8 MiB by default).
+int no_threads() {
+    Ring r(3 * kOutPiece);
+    std::thread([] {}).join();   // the runtime's own first allocations
+    unsigned long pages = 0;
+    FILE* f = fopen("/proc/self/statm", "r");
+    CHECK(f && fscanf(f, "%lu", &pages) == 1);
+    fclose(f);
+    // glibc keeps the stack of a thread that ended, so one more may start
+    const rlimit lim{pages * 4096 + (2u << 20), RLIM_INFINITY};
+    CHECK(setrlimit(RLIMIT_AS, &lim) == 0);
+    OutHelpers helpers(4);
+    helpers.post(r.job);
+    const int rc = out_collect(*r.job, [&](uint64_t g) { return r.deliver_group(g); }, [] { return (int)ASC_OK; });
+    helpers.drop(r.job);
+    CHECK(rc == ASC_OK && r.right());
+    return 0;
+}
+
 }  // namespace
 
-int main() {
+int main(int argc, char** argv) {
+    if (argc > 1 && !strcmp(argv[1], "no-threads")) {
+        const int bad = no_threads();
+        if (!bad) printf("ok\n");
+        return bad;
+    }
     OutHelpers helpers(3);
     const int bad = slow_helper() + late_device() + with_helpers(helpers) + failed_launch(helpers);
     if (!bad) printf("ok\n");

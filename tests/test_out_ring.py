@@ -1,7 +1,8 @@
 """The loop that collects results (out_ring.hpp), with a device played by the
 test: a helper that stops inside a copy while every queued piece has arrived
 is waited for, a late device too, a device that ends without delivering and a
-launch that fails are errors."""
+launch that fails are errors; where the system grants no more threads, the
+calling one copies alone."""
 import os
 import shutil
 import subprocess
@@ -20,6 +21,7 @@ def check(tmp_path_factory):
 
 
 @pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
-def test_ring_loop(check):
-    r = subprocess.run([check], capture_output=True, text=True, timeout=60)
+@pytest.mark.parametrize("args", [[], ["no-threads"]])
+def test_ring_loop(check, args):
+    r = subprocess.run([check, *args], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0 and r.stdout == "ok\n", r.stdout + r.stderr
