@@ -519,7 +519,7 @@ __global__ void k_init_cc(uint32_t* val, uint32_t* pstamp, uint32_t* q, uint32_t
 // (BFS, SSSP: `off` given) the reached vertices and their degrees added up.
 template <class OffT>
 __global__ __launch_bounds__(kBlock) void k_finish_values(const uint32_t* val, const OffT* off, uint32_t unreached,
-                                                          int zero_based, unsigned long long* reach, OutGroup g) {
+                                                          int zero_based, DevStats* stats, OutGroup g) {
     __shared__ unsigned long long s_r[kWavesPerBlock], s_d[kWavesPerBlock];
     const OutSlot s = out_slot(g);
     unsigned long long r = 0, d = 0;
@@ -559,24 +559,19 @@ __global__ __launch_bounds__(kBlock) void k_finish_values(const uint32_t* val, c
                 d += s_d[i];
             }
             if (r) {
-                atomicAdd(reach, r);
-                atomicAdd(reach + 1, d);
+                atomicAdd(&stats->reached, r);
+                atomicAdd(&stats->degree_sum, d);
             }
         }
     }
     out_done(s);
 }
 
-// Behind the last values: the statistics of the run, and the counts above
-// (cleared for the next run).  One lane.
-__global__ void k_finish_stats(const DevStats* stats, unsigned long long* reach, FinishPub* pub,
-                               unsigned long long seq) {
+// Behind the last values: the statistics of the run, the counts above among
+// them.  One lane.
+__global__ void k_finish_stats(const DevStats* stats, FinishPub* pub, unsigned long long seq) {
     if (threadIdx.x != 0) return;
     host_store_words(&pub->stats, *stats);
-    host_store(&pub->reached, reach[0]);
-    host_store(&pub->degree_sum, reach[1]);
-    reach[0] = 0;
-    reach[1] = 0;
     host_publish(&pub->seq, seq);
 }
 
@@ -679,9 +674,7 @@ int trav_ensure(asc_graph* g) {
     t->mem.add(&t->slots, 4);
     t->mem.add(&t->piles, 1);
     t->mem.add(&t->stats, 1);
-    t->mem.add(&t->d_reach, 2);
     ASC_TRY(t->mem.alloc());
-    ASC_HIP(hipMemsetAsync(t->d_reach, 0, 16, g->ctx->s_main));
     ASC_TRY(t->h.alloc(1, true));
     std::memset((void*)t->h.p, 0, sizeof(HostPubs));
     ASC_HIP(hipHostGetDevicePointer((void**)&t->d_h, t->h.p, 0));
@@ -1600,8 +1593,7 @@ int finish_traversal(asc_graph* g, int algo, int path, uint32_t* out, asc_stats*
     const bool zero_based = count && ctx->cfg.value_convention == ASC_VALUES_ZERO_BASED;
     const unsigned long long want = ++t->finish_seq;
     auto send_stats = [&]() -> int {
-        hipLaunchKernelGGL(k_finish_stats, dim3(1), dim3(kWave), 0, ctx->s_main, t->stats, t->d_reach, &t->d_h->finish,
-                           want);
+        hipLaunchKernelGGL(k_finish_stats, dim3(1), dim3(kWave), 0, ctx->s_main, t->stats, &t->d_h->finish, want);
         ASC_HIP(hipGetLastError());
         return ASC_OK;
     };
@@ -1610,11 +1602,11 @@ int finish_traversal(asc_graph* g, int algo, int path, uint32_t* out, asc_stats*
             if (g->off_bytes == 4)
                 hipLaunchKernelGGL((k_finish_values<uint32_t>), dim3(blocks), dim3(kBlock), 0, ctx->s_main, t->val,
                                    count ? (const uint32_t*)g->d_off : nullptr, (uint32_t)(V + 1), zero_based ? 1 : 0,
-                                   t->d_reach, og);
+                                   t->stats, og);
             else
                 hipLaunchKernelGGL((k_finish_values<uint64_t>), dim3(blocks), dim3(kBlock), 0, ctx->s_main, t->val,
                                    count ? (const uint64_t*)g->d_off : nullptr, (uint32_t)(V + 1), zero_based ? 1 : 0,
-                                   t->d_reach, og);
+                                   t->stats, og);
             ASC_HIP(hipGetLastError());
             return (uint64_t)(og.piece + kOutGroup) * kOutPiece >= V ? send_stats() : ASC_OK;
         }));
@@ -1660,8 +1652,8 @@ int finish_traversal(asc_graph* g, int algo, int path, uint32_t* out, asc_stats*
     }
     if (out && st) {
         // reached vertices and their degree sum (Graph500 TEPS numerator)
-        st->reached = count ? t->h[0].finish.reached : V;
-        st->reached_degree_sum = count ? t->h[0].finish.degree_sum : g->h.E;
+        st->reached = count ? ds.reached : V;
+        st->reached_degree_sum = count ? ds.degree_sum : g->h.E;
         // BFS is level-synchronous: each reached vertex is active in
         // exactly one iteration, so the reference's nodeSum (actives summed
         // over iterations, CalculateOpt.cu:183-190) is the reached count,

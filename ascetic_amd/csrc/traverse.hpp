@@ -45,6 +45,7 @@ struct Piles {
     uint32_t pad[2];
 };
 
+// Cleared at the start of a run (also what one that failed left behind).
 struct DevStats {
     unsigned long long edges_local;   // k_expand_local
     unsigned long long verts_local;
@@ -60,12 +61,13 @@ struct DevStats {
     // a level's first kernel notes when it began, its publish adds the time
     // since (fully resident runs; streamed ones are timed by events)
     unsigned long long t_begin, ticks;
+    // reached vertices and their degrees, counted while the values are sent
+    unsigned long long reached, degree_sum;
 };
 
 // What the end of a run hands to the host beside the values (seq last).
 struct FinishPub {
     DevStats stats;
-    unsigned long long reached, degree_sum;
     unsigned long long seq;
 };
 
@@ -267,7 +269,6 @@ struct TravState {
     HostBuf<HostPubs> h;
     HostPubs* d_h = nullptr;
     unsigned long long lvl_seq = 0, narrow_seq = 0, pub_seq = 0, finish_seq = 0;
-    unsigned long long* d_reach = nullptr;   // reached vertices and their degrees while values are sent
     OutStage out;
     // the host gather's index of a round's sparse segment: first record of
     // each listed vertex in the gathered array (written by the device through
