@@ -100,7 +100,7 @@ class GraphInfo(C.Structure):
 class KernelStats(C.Structure):
     _fields_ = [
         ("launches", C.c_uint32),
-        ("pad", C.c_uint32),
+        ("record_bytes", C.c_uint32),
         ("ms", C.c_double),
         ("edges", C.c_uint64),
         ("vertices", C.c_uint64),
@@ -144,6 +144,8 @@ class Stats(C.Structure):
         d["path"] = PATH_NAMES[self.path] if 0 <= self.path < len(PATH_NAMES) else self.path
         d["kernels"] = {KERNEL_NAMES[i]: {n: getattr(self.kern[i], n) for n in ("launches", "ms", "edges", "vertices")}
                         for i in range(len(KERNEL_NAMES))}
+        # what crossed the link (streamed_bytes counts whole records of the on-demand store)
+        d["link_bytes"] = self.streamed_edges * self.kern[KERNEL_NAMES.index("expand_part")].record_bytes
         return d
 
 

@@ -281,6 +281,8 @@ struct asc_graph {
     uint32_t pk_shift = 32, pk_wmin = 0;
     // bytes per streamed on-demand edge
     size_t stream_record_bytes() const { return packed ? (pk_split ? 5 : 4) : h.edge_bytes(); }
+    // the same on the link, where a run without weights leaves the split form's weight bytes out
+    size_t link_record_bytes(bool weights) const { return packed && pk_split && !weights ? 4 : stream_record_bytes(); }
     // the on-demand records sit in page-locked memory (DMA and zero-copy
     // reads straight from them); pageable packed tails go through staging
     bool tail_pinned() const {

@@ -2003,6 +2003,7 @@ static int pr_normalised(asc_graph* g, const asc_pr_opts* o, float* rank_out, do
         st->host_cores = hardware_threads();
         st->streamed_edges = p->streamed_edges * (uint64_t)iters;
         st->streamed_bytes = 4 * st->streamed_edges;
+        st->kern[KERN_PART].record_bytes = p->chunks.empty() ? 0 : 4;
         st->parts = (uint32_t)(p->chunks.size() * (size_t)iters);
         st->kern[3].launches = (uint32_t)iters;
         st->kern[3].ms = kms;

@@ -97,13 +97,14 @@ int write_raw(const std::string& path, const void* p, size_t bytes) {
 void print_stats_json(const char* algo, const asc_graph_info& gi, const asc_stats& st, double gteps) {
     printf("{\"algo\": \"%s\", \"V\": %llu, \"E\": %llu, \"static_edges\": %llu, \"ondemand_edges\": %llu, "
            "\"iterations\": %u, \"node_sum\": %llu, \"edges_traversed\": %llu, \"streamed_bytes\": %llu, "
-           "\"parts\": %u, \"reached\": %llu, \"total_ms\": %.3f, \"static_ms\": %.3f, \"overload_ms\": %.3f, "
-           "\"fill_ms\": %.3f, \"gteps\": %.4f, \"host_cores\": %d}\n",
+           "\"link_bytes\": %llu, \"parts\": %u, \"reached\": %llu, \"total_ms\": %.3f, \"static_ms\": %.3f, "
+           "\"overload_ms\": %.3f, \"fill_ms\": %.3f, \"gteps\": %.4f, \"host_cores\": %d}\n",
            algo, (unsigned long long)gi.num_vertices, (unsigned long long)gi.num_edges,
            (unsigned long long)gi.static_edges, (unsigned long long)gi.ondemand_edges, st.iterations,
            (unsigned long long)st.node_sum, (unsigned long long)st.edges_traversed,
-           (unsigned long long)st.streamed_bytes, st.parts, (unsigned long long)st.reached, st.total_ms,
-           st.static_ms, st.overload_ms, st.fill_ms, gteps, st.host_cores);
+           (unsigned long long)st.streamed_bytes,
+           (unsigned long long)(st.streamed_edges * st.kern[2].record_bytes), st.parts,
+           (unsigned long long)st.reached, st.total_ms, st.static_ms, st.overload_ms, st.fill_ms, gteps, st.host_cores);
 }
 
 int run_gen(const Args& a) {

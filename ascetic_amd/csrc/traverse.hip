@@ -1001,7 +1001,7 @@ static int stream_pile(asc_graph* g, TravArgs<OffT, EdgeT>& a, uint32_t& level, 
     const uint64_t nod = g->h.V - g->static_vertices;
     uint32_t* list_deg = t->od_list + nod;
     const bool pk = g->packed;
-    const size_t EB = g->pk_split && !t->stream_w ? 4 : g->stream_record_bytes();   // bytes that cross the link
+    const size_t EB = g->link_record_bytes(t->stream_w);   // bytes that cross the link
     const uint64_t S = g->static_edges;
     const int pile_grid = (int)std::max<uint32_t>(1, std::min<uint32_t>((npile + kBlock - 1) / kBlock, 4096));
     // the host gather's index of the first n list entries (the sparse
@@ -1625,6 +1625,8 @@ int finish_traversal(asc_graph* g, int algo, int path, uint32_t* out, asc_stats*
     kern[KERN_PART_HOST].vertices = ds.verts_part_host;
     kern[KERN_BU].edges = ds.edges_bu;
     kern[KERN_BU].vertices = ds.verts_bu;
+    kern[KERN_PART].record_bytes = kern[KERN_PART_HOST].record_bytes =
+        g->static_vertices < V ? (uint32_t)g->link_record_bytes(t->stream_w) : 0;
     kern[KERN_UF].edges = ds.edges_uf;
     kern[KERN_UF].vertices = path == PATH_UNION_FIND ? V : 0;
 
@@ -1665,7 +1667,8 @@ int finish_traversal(asc_graph* g, int algo, int path, uint32_t* out, asc_stats*
                "overloadProcess time is %.3f ms\nfillProcess time is %.3f ms\nnodeSum : %llu\n"
                "move overload size : %llu\n",
                st->total_ms, st->pre_ms, st->static_ms, st->overload_ms, st->fill_ms,
-               (unsigned long long)st->node_sum, (unsigned long long)st->streamed_bytes);
+               (unsigned long long)st->node_sum,
+               (unsigned long long)(st->streamed_edges * st->kern[KERN_PART].record_bytes));
     }
     return ASC_OK;
 }

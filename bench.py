@@ -692,9 +692,7 @@ def c4_shape_section(A, _abi, O, args, cpu_threads):
             ctx.synchronize()
             step_s = (time.perf_counter() - t0) / n_runs
             num = st["reached_degree_sum"] / 2
-            sb = float(np.mean([r["streamed_bytes"] for r in runs]))
-            if algo == "bfs" and sb == 5 * float(np.mean([r["streamed_edges"] for r in runs])):
-                sb *= 0.8   # the split form's weight bytes stay on the host
+            sb = float(np.mean([r["link_bytes"] for r in runs]))
             sec = {"gteps": round(num / step_s / 1e9, 4), "ms_per_run": round(step_s * 1e3, 3), "runs": n_runs,
                    "iterations": st["iterations"], "reached": st["reached"],
                    "stream_record_bytes": round(sb / max(1.0, float(np.mean([r["streamed_edges"] for r in runs])))),
@@ -766,9 +764,7 @@ def c4_full_section(A, _abi, O, args, shape):
             ctx.synchronize()
             step_s = (time.perf_counter() - t0) / args.c4_full_runs
             num = st["reached_degree_sum"] / 2
-            sb = float(np.mean([r["streamed_bytes"] for r in runs]))
-            if algo == "bfs" and sb == 5 * float(np.mean([r["streamed_edges"] for r in runs])):
-                sb *= 0.8   # the split form's weight bytes stay on the host
+            sb = float(np.mean([r["link_bytes"] for r in runs]))
             out[algo] = {"gteps": round(num / step_s / 1e9, 4), "ms_per_run": round(step_s * 1e3, 1),
                          "runs": args.c4_full_runs, "iterations": st["iterations"], "reached": st["reached"],
                          "stream_record_bytes": round(sb / max(1.0, float(np.mean([r["streamed_edges"]

@@ -283,7 +283,10 @@ int asc_graph_replan(asc_graph* g, uint64_t edge_budget_bytes, double advise_rat
 /* ---- per-run statistics (phase names follow CalculateOpt.cu:30-36) ------ */
 typedef struct {
     uint32_t launches;
-    uint32_t pad;
+    uint32_t record_bytes;       /* [2], [7]: bytes a streamed record took on
+                                    the link in this run (BFS and CC leave the
+                                    split form's weight byte on the host);
+                                    else 0                                    */
     double ms;                   /* summed launch durations (HIP events)      */
     uint64_t edges;              /* edge records relaxed                      */
     uint64_t vertices;           /* frontier / list entries expanded          */
@@ -302,8 +305,9 @@ typedef struct {
     uint64_t edges_traversed;    /* edges relaxed (static + on-demand)        */
     uint64_t static_edges_traversed;
     uint64_t streamed_edges;     /* on-demand edges shipped over the link     */
-    uint64_t streamed_bytes;     /* their records' bytes (BFS and CC leave the
-                                    split form's weight byte behind)          */
+    uint64_t streamed_bytes;     /* their bytes as the on-demand store holds
+                                    them; the link carried streamed_edges *
+                                    kern[2].record_bytes                      */
     uint64_t dense_edges;        /* of streamed_edges: copied as whole chunks
                                     by DMA (asc_config.dense_threshold)       */
     uint64_t vertices_processed; /* frontier entries expanded                 */
