@@ -1641,25 +1641,35 @@ static int pr_check_outdeg(const asc_graph* g, PrState* p) {
 // 0.86 / 0.79).
 constexpr uint64_t kPbMinV = uint64_t(1) << 17, kPbMinE = uint64_t(1) << 23;
 
+// Shape of the propagation-blocked layout: 2^14 sources a slice and 2^13
+// destinations a bin: 64 KB of LDS each, two workgroups a CU (V = 2^23, 2^28
+// edges: 14.7 ms for 20 iterations, also with 2^15 sources, 15.0 with 2^14
+// destinations; R-MAT scale 20: 2.20, 2.26, 2.57).  Larger ones where runs
+// would be shorter than 64 edges; AUTO leaves graphs with less than 16 a run
+// to the tiled pull, also where the layout was built by name.
+struct PbShape {
+    uint32_t bits = 14, dbits = 13;
+    uint64_t most;                // edges of a bin
+    bool long_runs;               // 16 edges a run and more
+    PbShape(uint64_t V, uint64_t E, uint32_t cus) {
+        most = std::max<uint64_t>(1u << 16, E / (8 * (uint64_t)cus));
+        auto runs = [&] { return ((V >> bits) + 1) * (std::max(V >> dbits, E / most) + 1); };
+        if (E / 64 < runs()) bits = 15;
+        if (E / 64 < runs()) dbits = 14;
+        long_runs = E / 16 >= runs();
+    }
+};
+
 // Builds the propagation-blocked layout once (every edge resident, at most
 // kPbMaxSlices slices, fewer than 2^31 octs, its arrays within free device
 // memory); pb_state = -1 when it cannot be built.
 template <class OffT>
-static int pr_blocked_build(asc_graph* g, PrState* p, bool by_name) {
+static int pr_blocked_build(asc_graph* g, PrState* p, const PbShape& shape) {
     if (p->pb_state != 0) return ASC_OK;
     const uint64_t V = g->h.V, E = g->h.E;
     const uint32_t cus = (uint32_t)g->ctx->num_cus;
-    const uint64_t most = std::max<uint64_t>(1u << 16, E / (8 * (uint64_t)cus));   // edges of a bin
-    // 2^14 sources a slice and 2^13 destinations a bin: 64 KB of LDS each, two
-    // workgroups a CU (V = 2^23, 2^28 edges: 14.7 ms for 20 iterations, also
-    // with 2^15 sources, 15.0 with 2^14 destinations; R-MAT scale 20: 2.20,
-    // 2.26, 2.57).  Larger ones where runs would be shorter than 64 edges;
-    // AUTO leaves graphs with less than 16 a run to the tiled pull.
-    uint32_t bits = 14, dbits = 13;
-    auto runs_of = [&] { return ((V >> bits) + 1) * (std::max(V >> dbits, E / most) + 1); };
-    if (E / 64 < runs_of()) bits = 15;
-    if (E / 64 < runs_of()) dbits = 14;
-    if (!by_name && E / 16 < runs_of()) return ASC_OK;
+    const uint64_t most = shape.most;
+    const uint32_t bits = shape.bits, dbits = shape.dbits;
     p->pb_state = -1;
     const uint64_t ns = (V + (1ull << bits) - 1) >> bits;
     if (g->static_vertices != V || E == 0 || E >= 0xFFFFFFFFull || V > (uint64_t(1) << 28) || ns > kPbMaxSlices)
@@ -1867,8 +1877,11 @@ static int pr_normalised(asc_graph* g, const asc_pr_opts* o, float* rank_out, do
     const int G = g->pr_group > 0 ? g->pr_group : 0;
     const bool by_name = o->method == ASC_PR_BLOCKED;
     const bool big = o->method == ASC_PR_AUTO && g->static_vertices == V && V >= (uint64_t(1) << 20);
-    const bool blocks = by_name || big || (o->method == ASC_PR_AUTO && !G && V >= kPbMinV && g->h.E >= kPbMinE);
-    if (blocks) ASC_TRY(pr_blocked_build<OffT>(g, p, by_name));
+    const PbShape shape(V, g->h.E, (uint32_t)ctx->num_cus);
+    const bool blocks =
+        by_name || (shape.long_runs &&
+                    (big || (o->method == ASC_PR_AUTO && !G && V >= kPbMinV && g->h.E >= kPbMinE)));
+    if (blocks) ASC_TRY(pr_blocked_build<OffT>(g, p, shape));
     const bool blocked = blocks && p->pb_state == 1;
     if (o->method == ASC_PR_BLOCKED && !blocked) {
         set_last_error("propagation-blocked PageRank needs every edge resident, E < 2^32 and room for its slots");
