@@ -5,12 +5,14 @@
 // Coordinate descent, one parameter at a time in that order, each candidate
 // timed as the minimum of two runs of the workload: BFS (and SSSP for
 // weighted graphs) from the maximum-degree vertex and three seeded random
-// vertices with out-edges, or three normalised PageRank iterations for BFS
-// CSC graphs.  The serving width is timed as the drain time of a burst of
-// 2 x width BFS queries.  The sweep stops early when `budget_ms` is spent,
-// keeping the best values found.  Results live on the graph (they are read at
-// launch time, nothing is re-uploaded) and can be saved in a tuning table
-// keyed by a fingerprint of the graph.
+// vertices with out-edges, or three normalised PageRank iterations for CSC
+// graphs, whose schedule in the warm-up run says what there is to sweep (the
+// tiles' segment size, the lanes per vertex, or nothing).  The serving width
+// is timed as the drain time of a burst of 2 x width BFS queries.  The sweep
+// stops early when `budget_ms` is spent, keeping the best values found.
+// Results live on the graph (they are read at launch time, nothing is
+// re-uploaded) and can be saved in a tuning table keyed by a fingerprint of
+// the graph.
 #include <algorithm>
 #include <cmath>
 #include <fstream>
@@ -150,10 +152,13 @@ int asc_autotune(asc_graph* g, double budget_ms, asc_tuning* out) {
             const int mw = std::max(1, (int)std::lround(g->mean_weight > 0 ? g->mean_weight : 32.0));
             sweep(&g->sssp_delta, {-1, std::max(1, mw / 2), mw, 4 * mw});
         }
-    } else if (g->static_vertices == g->h.V && g->h.V >= (uint64_t(1) << 20)) {
-        // the tiled pull (taken where the blocked layout does not fit): source segment size
+    } else if (g->pr_schedule == ASC_PR_TILED) {
+        // source segment size
         if (g->pr_tile_src_bits <= 0) g->pr_tile_src_bits = 15;
         sweep(&g->pr_tile_src_bits, {13, 14, 16, 17, 18});
+    } else if (g->pr_schedule == ASC_PR_BLOCKED && g->h.V >= (uint64_t(1) << 20)) {
+        // nothing to set: the blocked schedule has no such parameter, and from
+        // this V on a pr_group does not replace it
     } else {
         sweep(&g->pr_group, {4, 8, 16, 32, 64});
     }

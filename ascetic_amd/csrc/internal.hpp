@@ -297,6 +297,7 @@ struct asc_graph {
     bool host_edges_released = false;   // h.edges freed after packing (asc_config.release_host_edges)
     uint64_t fp = 0;                // graph fingerprint (cached before a release)
     int pr_tile_src_bits = 0;       // PageRank tile shape (0 = default)
+    int pr_schedule = -1;           // asc_pr_method the last normalised run took
     int pr_tile_dst_bits = 0;
     int blocks_per_cu = 0;          // workgroups per CU of traversal launches (0 = 8)
     uint32_t max_degree = 0, max_degree_vertex = 0;

@@ -1908,6 +1908,7 @@ static int pr_normalised(asc_graph* g, const asc_pr_opts* o, float* rank_out, do
         set_last_error("source-segmented PageRank needs every edge resident, V <= 2^31 and room for its tiles");
         return ASC_ERR_UNSUPPORTED;
     }
+    g->pr_schedule = tiled ? ASC_PR_TILED : blocked ? ASC_PR_BLOCKED : ASC_PR_PULL;
     if (!tiled && !blocked && !G) ASC_TRY(pr_rows_build<OffT>(g, p));
     const double t0 = now_ms();
     ASC_HIP(hipEventRecord(p->ev[0], s));

@@ -32,3 +32,15 @@ def test_auto_does_not_remember_a_named_schedule(gpu_ctx):
     assert np.array_equal(first, tiled)            # (one iteration from equal ranks: every sum is the same each time)
     assert not np.array_equal(named, tiled)        # exact sums against sums rounded to FP32
     assert np.array_equal(again, first)
+
+
+@pytest.mark.parametrize("n,schedule", [(10000, "tiled"), (100000, "blocked")])
+def test_tuner_sweeps_what_the_schedule_reads(gpu_ctx, n, schedule):
+    off, src, od = pairs(n, 2)
+    with gpu_ctx.from_arrays(off, src, out_degree=od) as g:
+        t = g.autotune(budget_ms=10000)
+    assert t["pr_group"] == 0 and t["score_ms"] <= t["untuned_ms"]
+    if schedule == "tiled":
+        assert t["pr_tile_src_bits"] in (13, 14, 15, 16, 17, 18)
+    else:
+        assert t["pr_tile_src_bits"] == 0 and t["score_ms"] == t["untuned_ms"]
