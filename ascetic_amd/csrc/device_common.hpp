@@ -40,12 +40,16 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
-// Publishing to mapped host memory that the host polls.  The words before the
-// sequence number are written through to the host (system-scope stores) and
-// the number itself is a releasing store.  Plain stores followed by
-// __threadfence_system() are not enough: the host then saw a new number beside
-// a cache line that still held old words in 30 of 7.4 M publishes (none in
-// 2.5 M this way), and a run that reads an old frontier size ends early.
+// Publishing to mapped host memory that the host polls: the sequence number is
+// an atomic store with release at system scope, which orders what its lane
+// stored before it, and what other lanes stored that this lane has
+// synchronized with (output.hpp: out_done); the host's polling load acquires.
+// A number stored plainly is ordered by nothing, a __threadfence_system()
+// ahead of it included (a fence orders through an atomic access behind it):
+// with plain stores on both sides of the fence the host saw a new number beside
+// old words in 30 of 7.4 M publishes (none in 2.5 M this way), and a run that
+// reads an old frontier size ends early.  The few words of a publish are
+// system-scope stores too, so none waits in the L2 for the release.
 template <class T>
 __device__ __forceinline__ void host_store(T* p, T v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);

@@ -70,16 +70,19 @@ __device__ __forceinline__ OutSlot out_slot(const OutGroup& g) {
 }
 
 // Ends a piece: once every workgroup of it has called this (all lanes, after
-// their stores to s.dst), the piece is published.  The stores are plain ones,
-// ordered by each lane's system fence before its workgroup is counted and by
-// the releasing store of the sequence number (1.1 M pieces of 128 and 512 KiB
-// checked: none seen early); storing every word through to the host instead
-// carries 0.1 GB/s.
+// their stores to s.dst), the piece is published.  The stores are plain ones
+// (storing every word through to the host carries 0.1 GB/s); what orders them
+// is the chain lane -> its workgroup's lane 0 by the barrier -> the lane 0 that
+// counts last by the acquiring and releasing count -> the host by that lane's
+// releasing store of the sequence number and the host's acquiring load.  Each
+// lane's fence sends its stores on their way to the host before the count, from
+// whichever XCD's L2 they are in (1.1 M pieces of 128 and 512 KiB checked: none
+// seen early).
 __device__ __forceinline__ void out_done(const OutSlot& s) {
     __threadfence_system();
     __syncthreads();
-    if (threadIdx.x != 0 || atomicAdd(s.arrived, 1u) != s.blocks - 1) return;
-    __threadfence_system();
+    if (threadIdx.x != 0) return;
+    if (__hip_atomic_fetch_add(s.arrived, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) != s.blocks - 1) return;
     *s.arrived = 0;
     host_publish(&s.pub->seq, s.seq);
 }
