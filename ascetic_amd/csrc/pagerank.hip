@@ -851,11 +851,16 @@ __global__ __launch_bounds__(kPbBlock) void k_pb_scatter(const float* __restrict
 // the largest contribution c below 2^e and fewer than 2^12 edges a row, units
 // of 2^(e - 51) cannot overflow, a contribution of 2^-27 of the largest still
 // keeps its 24 bits, and sums are exact in these units whatever their order.
-// Every rank is at least its base, so a contribution of kPbSpread bases at
-// most keeps an edge's rounding below 2^-32 of the rank.  Beyond that (a
-// vertex with a large share of all rank and few out-edges, or out-degrees too
-// small for the edges, whose ranks grow to infinity) sums are FP64.
-constexpr double kPbSpread = 1 << 20;
+// A smaller one is off by half a unit at most, 2^-51 c, and the 4095 of a row
+// may all be off the same way (a clique's are equal).  Every rank is at least
+// its base, so with c at most kPbSpread bases a row stays within 2^-26 of the
+// rank, a quarter of what rounding it to FP32 may change (2^20 instead of 2^13
+// bases: ranks of a 4095-clique beside a hub of 2^18 leaves two units off
+// those of FP64 sums).  R-MAT and Erdos-Renyi graphs reach 2^3 to 2^5 bases.
+// Beyond kPbSpread (a vertex with a large share of all rank and few out-edges,
+// or out-degrees too small for the edges, whose ranks grow to infinity) sums
+// are FP64.
+constexpr double kPbSpread = 1 << 13;
 __device__ __forceinline__ uint32_t pb_most(const double* slot) {
     const uint32_t l = lane_id();
     uint32_t m = l < (uint32_t)kPrLines ? *(const uint32_t*)(slot + kAccMax + l * kAccLine) : 0u;
