@@ -211,7 +211,7 @@ static int finish_graph(asc_ctx* ctx, asc_graph* g, asc_graph** out) {
     g->ctx = ctx;
     g->edge_budget_bytes = ctx->cfg.edge_budget_bytes;
     g->advise_rate = ctx->cfg.advise_rate;
-    if (g->h.E >= (uint64_t(1) << 32)) g->off_bytes = 8;
+    g->off_bytes = device_offset_bytes(g->h.E, g->off_bytes);
     g->heavy_threshold = ctx->cfg.heavy_threshold;
     g->pr_group = ctx->cfg.pr_group;
     g->sssp_delta = ctx->cfg.sssp_delta;

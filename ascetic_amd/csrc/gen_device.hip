@@ -455,7 +455,7 @@ int graph_generate(asc_ctx* ctx, const asc_gen_params* p, asc_graph** out) {
     gen.release();
     const double t_deg = now_ms();
     g->h.E = E;
-    g->off_bytes = (E >= (uint64_t(1) << 32) || p->offset_bytes == 8) ? 8 : 4;
+    g->off_bytes = device_offset_bytes(E, p->offset_bytes);
     g->edge_budget_bytes = ctx->cfg.edge_budget_bytes;
     g->advise_rate = ctx->cfg.advise_rate;
     g->heavy_threshold = ctx->cfg.heavy_threshold;

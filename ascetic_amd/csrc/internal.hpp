@@ -130,6 +130,13 @@ struct DevTmp {
     }
 };
 
+// Width of the edge offsets on the device: 4 bytes only while a kernel that
+// walks edges in 32 bits can step past the last one without wrapping (the
+// longest stride is the 2048 edges of a workgroup's pass).
+inline int device_offset_bytes(uint64_t E, int wanted) {
+    return wanted == 8 || E > (uint64_t(1) << 32) - (uint64_t(1) << 16) ? 8 : 4;
+}
+
 // Several device arrays in one allocation (one of a megabyte or more takes
 // ~270 us): add() each, then alloc() once; freed with the arena.
 struct DevArena {
