@@ -592,6 +592,7 @@ static int run_bfs_do(asc_graph* g, uint32_t src, uint32_t* out, asc_stats* st) 
             ASC_TRY((narrow_run<ALG_BFS, OffT, EdgeT>(g, a, (uint32_t)nf, 0, 0, 0, io)));
             const uint64_t reached = io.expanded + io.edges - mf;   // edges of the vertices claimed
             m_unexplored = m_unexplored > reached ? m_unexplored - reached : 0;
+            rc.node_sum += io.nodes;
             level = io.level;
             prev_nf = nf;
             nf = io.n;
@@ -605,6 +606,7 @@ static int run_bfs_do(asc_graph* g, uint32_t src, uint32_t* out, asc_stats* st) 
                                dim3(kBlock), 0, s, t->q[level & 1], t->slots + (level & 3), t->bm[cur]);
             bottom_up = true;
         }
+        rc.node_sum += nf;
         if (bottom_up) {
             ASC_TRY(timed_launch(t, prof, KERN_BU, s, [&] {
                 hipLaunchKernelGGL((k_bfs_bottom_up<OffT, EdgeT>), dim3(bu_grid), dim3(kBlock), 0, s, a.off, a.edges,
@@ -613,7 +615,6 @@ static int run_bfs_do(asc_graph* g, uint32_t src, uint32_t* out, asc_stats* st) 
             }));
             cur ^= 1;
         } else {
-            rc.node_sum += nf;
             a.q_in = t->q[level & 1];
             a.q_out = t->q[(level + 1) & 1];
             const int lgrid = (int)std::max<uint64_t>(1, std::min<uint64_t>(grid, (nf + kPassMin - 1) / kPassMin));
