@@ -454,11 +454,6 @@ __global__ __launch_bounds__(kBlock) void k_trav_publish(const Slot* slot, const
     if (timed) stats->ticks += wall_clock64() - stats->t_begin;
 }
 
-__global__ void k_fill_u32(uint32_t* p, uint64_t n, uint32_t v) {
-    for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
-        p[i] = v;
-}
-
 // Start of a run in one launch: every array at its initial value, the step-0
 // frontier of BFS / SSSP the source alone (GraphMeta.cuh:432-446).
 __global__ __launch_bounds__(kBlock) void k_run_init(RunInit a) {
