@@ -20,14 +20,18 @@ OutStage::~OutStage() {
     if (arrived) (void)hipFree(arrived);
 }
 
-int OutStage::ensure(uint64_t result_words) {
+int OutStage::ensure(uint64_t result_words, hipStream_t s) {
     const uint64_t want = std::min<uint64_t>(result_words, (uint64_t)kOutPiece * kOutRing);
     if (!arrived) {
         ASC_TRY(pub.alloc(kOutRing, true));
         for (int i = 0; i < kOutRing; i++) pub[i].seq = 0;
         ASC_HIP(hipHostGetDevicePointer((void**)&d_pub, pub.p, 0));
-        ASC_HIP(hipMalloc(&arrived, 4 * kOutRing * 32));
-        ASC_HIP(hipMemset(arrived, 0, 4 * kOutRing * 32));
+        // cleared on the stream of the kernels that count in it: it does not
+        // wait for the null stream, and hipMemset need not wait for the device
+        DevTmp<uint32_t> count;
+        ASC_HIP(hipMalloc(&count.p, 4 * kOutRing * 32));
+        ASC_HIP(hipMemsetAsync(count.p, 0, 4 * kOutRing * 32, s));
+        std::swap(arrived, count.p);
     }
     if (words < want) {
         words = 0;
@@ -46,7 +50,7 @@ int out_send(OutStage& o, uint32_t* const* dst, uint32_t parts, uint64_t words, 
     job->per_part = (words + kOutPiece - 1) / kOutPiece;
     job->pieces = job->per_part * parts;
     if (job->pieces >= 0xFFFFFFFFull) return ASC_ERR_RANGE;
-    ASC_TRY(o.ensure(job->pieces == 1 ? words : job->pieces * kOutPiece));
+    ASC_TRY(o.ensure(job->pieces == 1 ? words : job->pieces * kOutPiece, s));
     job->pub = o.pub.p;
     job->buf = o.buf.p;
     job->dst = dst;

@@ -27,7 +27,7 @@ struct OutStage {
     uint64_t words = 0;             // capacity
     unsigned long long seq = 0;     // pieces sent so far
     ~OutStage();
-    int ensure(uint64_t result_words);
+    int ensure(uint64_t result_words, hipStream_t s);   // s: the stream of every send
 };
 
 // A group of consecutive pieces, for the kernel that writes them: `blocks`
