@@ -1641,9 +1641,12 @@ static int pr_check_outdeg(const asc_graph* g, PrState* p) {
 // Below, the row blocks' gathers come out of the L2s and two launches an
 // iteration on few workgroups cost more (ms of 20 iterations, blocked / row
 // blocks: R-MAT scale 18, 7.6e6 edges 0.91 / 0.80, Erdos-Renyi V = 2^18, 8.4e6
-// edges 0.66 / 1.07, V = 2^17, 1.7e7 edges 0.85 / 1.82); from V = 2^20 on the
-// lines hold however few the edges (V = 2^20, 4.2e6 edges: 0.53 / 0.96, R-MAT
-// 0.86 / 0.79).
+// edges 0.66 / 1.07, V = 2^17, 1.7e7 edges 0.85 / 1.82).  Between the first two
+// points lies the line on edges, but they differ in skew more than in edges:
+// on a skewed graph just above it the row blocks may still be the faster, on
+// an even one just below it the blocked schedule, by what the points show.
+// From V = 2^20 on the blocked schedule is taken however few the edges (V =
+// 2^20, 4.2e6 edges: Erdos-Renyi 0.53 / 0.96, R-MAT 0.86 / 0.79).
 constexpr uint64_t kPbMinV = uint64_t(1) << 17, kPbMinE = uint64_t(1) << 23;
 
 // Shape of the propagation-blocked layout: 2^14 sources a slice and 2^13
@@ -1905,7 +1908,10 @@ static int pr_normalised(asc_graph* g, const asc_pr_opts* o, float* rank_out, do
     const uint32_t db_auto = (V >> 15) >= 4 * (uint64_t)ctx->num_cus ? 15u : 14u;
     const uint32_t db = o->tile_dst_bits > 0 ? (uint32_t)o->tile_dst_bits
                         : g->pr_tile_dst_bits > 0 ? (uint32_t)g->pr_tile_dst_bits : db_auto;
-    // AUTO: the tiled pull where the blocked layout cannot be built
+    // AUTO: the tiled pull where the blocked layout cannot be built or its
+    // runs would be short, as on every large graph before there was that
+    // layout.  On R-MAT graphs the row blocks are faster than the tiles (the
+    // table above kPbBlock); no graph of that kind was measured this sparse.
     const bool want_tiled = o->method == ASC_PR_TILED || (big && !blocked);
     if (want_tiled) ASC_TRY(pr_tiled_build<OffT>(g, p, sb, db));
     const bool tiled = want_tiled && p->tl_state == 1;

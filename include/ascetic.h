@@ -365,8 +365,10 @@ typedef struct {
     double threshold;            /* reference mode: 0.001                     */
     int max_iterations;          /* reference mode safety cap (0 = 10000)     */
     int method;                  /* normalised mode: asc_pr_method            */
-    /* ASC_PR_TILED tile shape (0 = tuned): sources per segment 2^src_bits,
-     * destinations per block 2^dst_bits (<= 14), src_bits + dst_bits <= 32 */
+    /* Tile shape where the tiled schedule runs, by name or chosen by
+     * ASC_PR_AUTO (0 = tuned): sources per segment 2^src_bits, destinations
+     * per block 2^dst_bits (<= 15), src_bits + dst_bits <= 32; the other
+     * schedules have no tiles and ignore it */
     int tile_src_bits;
     int tile_dst_bits;
 } asc_pr_opts;
@@ -376,7 +378,8 @@ typedef enum {
     ASC_PR_AUTO = 0,     /* ASC_PR_BLOCKED when every edge is resident and
                             V >= 2^20, or V >= 2^17 with 2^23 edges and no
                             pr_group set; ASC_PR_TILED where V >= 2^20 and
-                            the blocked layout does not fit; else the pull  */
+                            the blocked layout does not fit or would have
+                            fewer than 16 edges a run; else the pull        */
     ASC_PR_PULL = 1,     /* pull over the in-CSR                             */
     ASC_PR_BLOCKED = 2,  /* propagation-blocked (scatter by slices of sources,
                             LDS sums per bin of destinations); needs every
